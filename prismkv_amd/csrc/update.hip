@@ -25,10 +25,11 @@
 //
 // Launches of one update (all G groups at once; the update runs every
 // `interval` tokens, its cost is amortised):
-//   encode   LDS-tiled fp32 GEMM, 64 tokens x 64 buckets per workgroup,
-//            writes a = relu(...) [G][N][F] and a histogram of the positive
-//            values' top 11 bits (4 replicas of each global bin, so the
-//            flushes of ~750 workgroups do not queue on one address);
+//   wsplit   W as pairs of f16 in the encode's operand order;
+//   encode   the GEMM on the f16 matrix cores, 256 tokens x 64 buckets per
+//            workgroup and step, writes a = relu(...) [G][N][F] and a
+//            histogram of the positive values' top 11 bits (4 replicas of
+//            each global bin, so the flushes do not queue on one address);
 //   digit    one workgroup per group picks the histogram bin holding the
 //            budget-th largest value (3 levels: bits 30..20, 19..9, 8..0);
 //   refine   re-reads a, histograms the values inside the chosen prefix;
@@ -55,7 +56,6 @@ namespace prismkv {
 namespace {
 
 constexpr int kUT = 256;
-constexpr int kTT = 64;        // tokens per encode tile
 constexpr int kFT = 64;        // buckets per encode tile
 constexpr int kFTiles = (kF + kFT - 1) / kFT;  // 47
 constexpr int kBins = 2048;
@@ -75,7 +75,7 @@ constexpr int kBuildCenter = 1;      // prismkv_build flag: compute the center (
 enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kListed, kListLen, kCtl = 16 };
 enum { kModeTopK = 0, kModeAllPositive = 1 };
 
-// Key loads of the two key element types: 2, 4 or 8 consecutive dims as the
+// Key loads of the two key element types: 2 or 8 consecutive dims as the
 // raw loaded bits (kept packed while in flight) and their fp32 values.
 template <typename KT>
 struct KeyLoad;
@@ -83,14 +83,9 @@ struct KeyLoad;
 template <>
 struct KeyLoad<uint16_t> {  // bf16
   typedef uint32_t Raw2;
-  typedef uint2 Raw4;
   static __device__ __forceinline__ Raw2 load2(const uint16_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
   static __device__ __forceinline__ float lo(Raw2 r) { return bf16_lo(r); }
   static __device__ __forceinline__ float hi(Raw2 r) { return bf16_hi(r); }
-  static __device__ __forceinline__ Raw4 load4(const uint16_t* p) { return *reinterpret_cast<const uint2*>(p); }
-  static __device__ __forceinline__ float4 f4(Raw4 r) {
-    return make_float4(bf16_lo(r.x), bf16_hi(r.x), bf16_lo(r.y), bf16_hi(r.y));
-  }
   static __device__ __forceinline__ void load8(const uint16_t* p, float (&x)[8]) {
     const uint4 v = *reinterpret_cast<const uint4*>(p);
     x[0] = bf16_lo(v.x); x[1] = bf16_hi(v.x); x[2] = bf16_lo(v.y); x[3] = bf16_hi(v.y);
@@ -101,12 +96,9 @@ struct KeyLoad<uint16_t> {  // bf16
 template <>
 struct KeyLoad<float> {
   typedef float2 Raw2;
-  typedef float4 Raw4;
   static __device__ __forceinline__ Raw2 load2(const float* p) { return *reinterpret_cast<const float2*>(p); }
   static __device__ __forceinline__ float lo(Raw2 r) { return r.x; }
   static __device__ __forceinline__ float hi(Raw2 r) { return r.y; }
-  static __device__ __forceinline__ Raw4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-  static __device__ __forceinline__ float4 f4(Raw4 r) { return r; }
   static __device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
     const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
     x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
@@ -126,6 +118,8 @@ struct UpdateArgs {
   int* counts;     // [G][kFP]
   float* moments;  // [G][kChunks][256][32]
   float* act;      // [G][N][F]
+  _Float16* wsplit;  // [G][kFTiles][kWTile] W split for the encode
+  float* wscale;     // [G][kFTiles * 64] the buckets' inverse scales
   unsigned* hist;  // [G][kLevels][kRep][kBins]
   unsigned* ctl;   // [G][kCtl]
   unsigned* tcount;  // [G][tie_blocks] ties per contiguous range of a
@@ -142,142 +136,269 @@ __device__ __forceinline__ unsigned* hist_of(const UpdateArgs& a, int g, int lev
 }
 
 // ---------------------------------------------------------------------------
-// encode: grid (ceil(N / 128), P, G) x 512.  Workgroup (y, part) takes the
-// tokens [128 y, 128 y + 128), wave w the 16 rows 128 y + 16 w + i, and the
-// bucket tiles part, part + P, ... (64 buckets each).  The wave's
-// x = (k - center) / scale is computed once, into registers, and each bucket
-// tile's W streams through LDS, double-buffered: the next tile's W is
-// requested into registers while the current tile is multiplied, then
-// stored to the other buffer.  Products run on fp32 MFMA
-// (v_mfma_f32_16x16x4f32: lane l feeds A[i = l % 16][k = l / 16],
-// B[k][j = l % 16] and holds D[4 (l / 16) + r][l % 16]).  A is W (bucket
-// rows) and B is x (token columns), so D is [bucket][token] and lane (i, q)
-// ends with buckets 4 q .. 4 q + 3 of token i, stored as one 16-byte store.
-// Lane (i, q) = (l % 16, l / 16) supplies the dims 16 kb + 4 q + t of dim
-// block kb to step t: its W values are one 16-byte LDS read per 16-bucket
-// column and block, its x values those of token row i at its 32 dims.  A and
-// B always pair the same dim, so the steps only reorder the sum over the 128
-// dims (the same order for every token and bucket).  P is the smallest count that gives the launch
-// kEncMinWgs workgroups (two per CU), so the x of a token is computed P times
-// in all rather than once per bucket tile.
+// The encode's products run on the f16 matrix cores as a split: an fp32 value
+// v times a power of two is hi + lo, hi = f16(v), lo = f16(v - hi), and
+//   x . w = x_hi . w_hi + x_hi . w_lo + x_lo . w_hi
+// in fp32 accumulators (three f16 MFMAs of 32 dims instead of eight fp32 ones
+// of 4).  hi + lo is within 2^-22 of v at most and 2^-24.8 rms, x_lo . w_lo
+// (left out) 2^-24.7 rms of its product, so the split costs less than the
+// roundings of a 128-step fp32 chain: against 64 bits the activations are
+// within 1.4e-7 (2-norm over a block) where the fp32 MFMA chain had 2.1e-7.
+// The power of two, per key row and per bucket, brings the largest magnitude
+// to [2^14, 2^15), so nothing overflows f16 and what underflows is below 2^-39
+// of that largest one.  A row or bucket that is not finite, or whose largest
+// magnitude lies outside 2^+-60 (the scales' products would leave fp32), is
+// not split: its values are computed by plain fp32 chains (exact_value).
+//
+// wsplit: grid (kFTiles, G) x 256 writes W in the order the encode reads it:
+// tile ft (64 buckets) is 32 fragments of 1 KB, [kb (4)][hi, lo][j (4)], lane
+// (i, q) of a fragment holding bucket 64 ft + 16 j + i, dims 32 kb + 8 q .. + 7
+// (an MFMA A operand).  Splitting W here and not in each encode workgroup
+// takes it off the encode's VALU, which its epilogue already fills; it reads
+// and writes 12.3 MB for 8 groups (5 us).
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kET = 512;                          // encode workgroup
-constexpr int kRowTile = 16;                      // tokens per wave
-constexpr int kEncTokens = kET / 64 * kRowTile;   // tokens per workgroup (128)
-constexpr int kEncMinWgs = 512;                   // workgroups the bucket-tile parts aim for
-constexpr int kWLoads = kFT * kD / 4 / kET;       // float4 of a W tile per thread (4)
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+constexpr int kScaleExp = 14;   // scaled rows have their largest magnitude in [2^14, 2^15)
+constexpr int kMaxScale = 60;   // |exponent| of a row's or bucket's largest magnitude, at most
+constexpr int kWTile = kFT * kD * 2;  // f16 values of a split W tile
+constexpr int kKB = kD / 32;          // MFMA dim blocks
 
-// K chunk kb (4 dims 16 kb + 4 q ..) of token row t0 + i for lane (i, q).
+// The power of two that scales a row of largest magnitude m, and its inverse;
+// inverse 0 marks a row that is not split.
+__device__ __forceinline__ float2 row_scale(float m) {
+  if (m == 0.f) return make_float2(1.f, 1.f);
+  const int e = (int)(__float_as_uint(m) >> 23) - 127;  // 128 for infinities and NaN, -127 for subnormals
+  if (!(e >= -kMaxScale && e <= kMaxScale)) return make_float2(0.f, 0.f);
+  const int k = kScaleExp - e;
+  return make_float2(__uint_as_float((unsigned)(127 + k) << 23), __uint_as_float((unsigned)(127 - k) << 23));
+}
+
+__device__ __forceinline__ void split8(const float (&x)[8], float scale, half8& hi, half8& lo) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = x[j] * scale;
+    hi[j] = (_Float16)v;
+    lo[j] = (_Float16)(v - (float)hi[j]);
+  }
+}
+
+// The larger magnitude as bits: NaN and infinities order above every number.
+__device__ __forceinline__ unsigned mag_max(unsigned m, float x) { return max(m, __float_as_uint(x) & 0x7fffffffu); }
+
+__global__ __launch_bounds__(kUT) void wsplit_kernel(UpdateArgs a) {
+  const int ft = blockIdx.x, g = blockIdx.y, j = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int f = ft * kFT + 16 * j + (lane & 15);
+  float w[kKB][8];
+  unsigned m = 0u;
+#pragma unroll
+  for (int kb = 0; kb < kKB; ++kb) {
+    float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+    if (f < kF) {
+      const float4* row = reinterpret_cast<const float4*>(a.W + ((size_t)g * kF + f) * kD + 32 * kb + 8 * (lane >> 4));
+      u = row[0];
+      v = row[1];
+    }
+    w[kb][0] = u.x; w[kb][1] = u.y; w[kb][2] = u.z; w[kb][3] = u.w;
+    w[kb][4] = v.x; w[kb][5] = v.y; w[kb][6] = v.z; w[kb][7] = v.w;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) m = mag_max(m, w[kb][t]);
+  }
+  m = max(m, (unsigned)__shfl_xor((int)m, 16));
+  m = max(m, (unsigned)__shfl_xor((int)m, 32));
+  const float2 sc = row_scale(__uint_as_float(m));
+  _Float16* tile = a.wsplit + ((size_t)g * kFTiles + ft) * kWTile;
+#pragma unroll
+  for (int kb = 0; kb < kKB; ++kb) {
+    half8 hi, lo;
+    split8(w[kb], sc.x, hi, lo);
+    *reinterpret_cast<half8*>(tile + ((kb * 2 + 0) * 4 + j) * 512 + lane * 8) = hi;
+    *reinterpret_cast<half8*>(tile + ((kb * 2 + 1) * 4 + j) * 512 + lane * 8) = lo;
+  }
+  if (lane < 16) a.wscale[((size_t)g * kFTiles + ft) * kFT + 16 * j + lane] = sc.y;
+}
+
+// ---------------------------------------------------------------------------
+// encode: grid (ceil(N / 256), P, G) x 512.  Workgroup (y, part) takes the
+// tokens [256 y, 256 y + 256), wave w the 32 rows 256 y + 32 w + 16 tb + i, and
+// the bucket tiles part, part + P, ... (64 buckets each).  The wave's
+// x = (k - center) / scale is computed in fp32 and split once, into registers
+// (64 of them), and each bucket tile's split W streams through LDS,
+// double-buffered: the next tile is requested into registers while the current
+// one is multiplied.  Products run on v_mfma_f32_16x16x32_f16 (lane (i, q) =
+// (l % 16, l / 16) feeds A[i][8 q + t] and B[8 q + t][i], t = 0..7, and holds
+// D[4 q + r][i]): A is W (bucket rows) and B is x (token columns), so lane
+// (i, q) ends with buckets 4 q .. 4 q + 3 of token i, stored as one 16-byte
+// store.  32 tokens per wave, because a wave reads the whole 32 KB tile from
+// LDS whatever its tokens: at 16 the 8 waves' reads took as long as their
+// products.  P is chosen on the host (encode_parts).  8 groups, MI355X, with
+// the fp32 MFMA kernel's time before: 1024 tokens 46.6 us (78), 4096 148 us
+// (262), 65536 3.02 ms (4.10); what is left is the histogram's LDS atomics and
+// the 12 KB per token of activations, not the products.
+// ---------------------------------------------------------------------------
+constexpr int kET = 512;                          // encode workgroup
+constexpr int kTB = 2;                            // 16-token blocks per wave
+constexpr int kRowTile = 16 * kTB;                // tokens per wave
+constexpr int kEncTokens = kET / 64 * kRowTile;   // tokens per workgroup (256)
+constexpr int kWLoads = kWTile * 2 / 16 / kET;    // 16-byte loads of a W tile per thread (4)
+
+// relu(x . w + b) of key row `tok` of the block and bucket f by one fp32 chain:
+// rows and buckets that the split does not serve.
 template <typename KT>
-__device__ __forceinline__ typename KeyLoad<KT>::Raw4 key_chunk(const UpdateArgs& a, int g, int t0, int kb) {
-  const int li = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
-  const int row = min(t0 + li, a.N - 1);  // rows past the block repeat the last one (masked at the store)
-  const KT* k = static_cast<const KT*>(a.k);
-  return KeyLoad<KT>::load4(k + (size_t)g * a.ks + (size_t)(a.H + row) * kD + 16 * kb + 4 * lq);
+__device__ float exact_value(const UpdateArgs& a, int g, int tok, int f) {
+  const KT* k = static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)(a.H + tok) * kD;
+  const float* w = a.W + ((size_t)g * kF + f) * kD;
+  const float* c = a.center + (size_t)g * kD;
+  const float sc = a.scale[g];
+  float s = 0.f;
+#pragma unroll 1
+  for (int d = 0; d < kD; ++d) s = fmaf((to_f32(k[d]) - c[d]) / sc, w[d], s);
+  return s + a.b[(size_t)g * kF + f];
 }
 
 template <typename KT>
 __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   const int y = blockIdx.x, part = blockIdx.y, parts = gridDim.y, g = blockIdx.z, tid = threadIdx.x;
   const int w = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
-  __shared__ __align__(16) float ws[2][kFT][kD + 4];  // [buffer][bucket][dim], padded against bank conflicts
-  __shared__ __align__(16) float cs[kD];              // center
+  __shared__ __align__(16) u32x4 ws[2][kET * kWLoads];  // [buffer][a split W tile]
   __shared__ unsigned hist[kBins];
   const int t0 = y * kEncTokens + w * kRowTile;  // the wave's first token
-  typename KeyLoad<KT>::Raw4 kr[kD / 16];
+  const bool live = t0 < a.N;                    // uniform per wave: a wave without tokens only moves W
+  const u32x4* wg = reinterpret_cast<const u32x4*>(a.wsplit + (size_t)g * kFTiles * kWTile);
+  auto load_w = [&](int ft, u32x4 (&r)[kWLoads]) {
 #pragma unroll
-  for (int kb = 0; kb < kD / 16; ++kb) kr[kb] = key_chunk<KT>(a, g, t0, kb);
-  const float* wg = a.W + (size_t)g * kF * kD;
-  // thread tid moves float4 tid + kET u of a 64 x 128 W tile (bucket i / 32, dims 4 (i % 32) ..)
-  auto load_w = [&](int ft, float4 (&r)[kWLoads]) {
-#pragma unroll
-    for (int u = 0; u < kWLoads; ++u) {
-      const int i = tid + kET * u, f = ft * kFT + i / (kD / 4);
-      r[u] = f < kF ? *reinterpret_cast<const float4*>(wg + (size_t)f * kD + 4 * (i % (kD / 4)))
-                    : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    for (int u = 0; u < kWLoads; ++u) r[u] = wg[(size_t)ft * (kET * kWLoads) + tid + kET * u];
   };
-  auto store_w = [&](int buf, const float4 (&r)[kWLoads]) {
+  auto store_w = [&](int buf, const u32x4 (&r)[kWLoads]) {
 #pragma unroll
-    for (int u = 0; u < kWLoads; ++u) {
-      const int i = tid + kET * u;
-      *reinterpret_cast<float4*>(&ws[buf][i / (kD / 4)][4 * (i % (kD / 4))]) = r[u];
-    }
+    for (int u = 0; u < kWLoads; ++u) ws[buf][tid + kET * u] = r[u];
   };
-  float4 wr[kWLoads];
+  u32x4 wr[kWLoads];
   load_w(part, wr);
   for (int i = tid; i < kBins; i += kET) hist[i] = 0;
-  if (tid < kD) cs[tid] = a.center[(size_t)g * kD + tid];
-  __syncthreads();
-  // x = (k - center) / key_scale in fp32 (core.py:98) for this lane's row and 32 dims
-  const float sc = a.scale[g];
-  float4 xs[kD / 16];
+  // x = (k - center) / key_scale in fp32 (core.py:98): lane (i, q) holds dims
+  // 32 kb + 8 q .. + 7 of tokens t0 + i and t0 + 16 + i
+  half8 xh[kTB][kKB], xl[kTB][kKB];
+  float xinv[kTB];
+  bool bad_x = false;
+  if (live) {
+    const float sc = a.scale[g];
+    const float* cg = a.center + (size_t)g * kD + 8 * lq;
+    const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + 8 * lq;
 #pragma unroll
-  for (int kb = 0; kb < kD / 16; ++kb) {
-    const float4 r = KeyLoad<KT>::f4(kr[kb]);
-    const float4 c = *reinterpret_cast<const float4*>(&cs[16 * kb + 4 * lq]);
-    xs[kb] = make_float4((r.x - c.x) / sc, (r.y - c.y) / sc, (r.z - c.z) / sc, (r.w - c.w) / sc);
+    for (int tb = 0; tb < kTB; ++tb) {
+      const int row = a.H + min(t0 + 16 * tb + li, a.N - 1);  // rows past the block repeat the last one (masked below)
+      float x[kKB][8];
+      unsigned m = 0u;
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb) KeyLoad<KT>::load8(kg + (size_t)row * kD + 32 * kb, x[kb]);
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          x[kb][t] = (x[kb][t] - cg[32 * kb + t]) / sc;
+          m = mag_max(m, x[kb][t]);
+        }
+      m = max(m, (unsigned)__shfl_xor((int)m, 16));
+      m = max(m, (unsigned)__shfl_xor((int)m, 32));
+      const float2 s2 = row_scale(__uint_as_float(m));
+      xinv[tb] = s2.y;
+      bad_x |= s2.y == 0.f;
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb) split8(x[kb], s2.x, xh[tb][kb], xl[tb][kb]);
+    }
   }
+  const bool bad_rows = __any(bad_x);
   store_w(0, wr);
   __syncthreads();
   const float* bg = a.b + (size_t)g * kF;
+  const float* sg = a.wscale + (size_t)g * kFTiles * kFT;
   float* ag = a.act + (size_t)g * a.N * kF;
+  auto take = [&](float v) {  // histogram of a positive value
+    if (v > 0.f) atomicAdd(&hist[__float_as_uint(v) >> 20], 1u);
+  };
   int buf = 0;
   for (int ft = part; ft < kFTiles; ft += parts) {  // uniform
     const bool more = ft + parts < kFTiles;
     if (more) load_w(ft + parts, wr);  // in flight while this tile is multiplied
-    const int f0 = ft * kFT;
-    // the output is bucket-major (lane (i, q): buckets f0 + 16 j + 4 q .. + 3
-    // of token t0 + i), so each lane's 4 values of a j go out as one 16-byte
-    // store; kF is a multiple of 4, so those 4 buckets are live together
-    float4 bias[kFT / 16];
+    if (live) {
+      const int f0 = ft * kFT;
+      // lane (i, q): buckets f0 + 16 j + 4 q .. + 3; kF is a multiple of 4, so
+      // those 4 buckets are live together
+      float4 bias[kFT / 16], winv[kFT / 16];
+      bool bad_w = false;
 #pragma unroll
-    for (int j = 0; j < kFT / 16; ++j) {
-      const int f = f0 + 16 * j + 4 * lq;
-      bias[j] = f < kF ? *reinterpret_cast<const float4*>(bg + f) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    f32x4 acc[kFT / 16];
-#pragma unroll
-    for (int j = 0; j < kFT / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < kD / 16; ++kb) {
-      const float4 xa = xs[kb];
-      float4 bv[kFT / 16];
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j)
-        bv[j] = *reinterpret_cast<const float4*>(&ws[buf][16 * j + li][16 * kb + 4 * lq]);
-      // the four accumulators interleaved: no MFMA waits on the one before it.
-      // A = W (bucket rows), B = x (token columns): D[bucket][token], the
-      // same products in the same order as x W^T, transposed
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j].x, xa.x, acc[j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j].y, xa.y, acc[j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j].z, xa.z, acc[j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[j].w, xa.w, acc[j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // bias, relu, histogram of the positive values, store: lane (i, q) holds
-    // buckets f0 + 16 j + 4 q + r of token t0 + i
-    const int tok = t0 + li;
-#pragma unroll
-    for (int j = 0; j < kFT / 16; ++j) {
-      const int f = f0 + 16 * j + 4 * lq;
-      const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = acc[j][r] + b4[r];
-        v[r] = x > 0.f ? x : 0.f;  // relu; non-positive values are never selected
+      for (int j = 0; j < kFT / 16; ++j) {
+        const int f = f0 + 16 * j + 4 * lq;
+        bias[j] = f < kF ? *reinterpret_cast<const float4*>(bg + f) : make_float4(0.f, 0.f, 0.f, 0.f);
+        winv[j] = *reinterpret_cast<const float4*>(sg + f);
+        bad_w |= winv[j].x == 0.f || winv[j].y == 0.f || winv[j].z == 0.f || winv[j].w == 0.f;
       }
-      if (tok < a.N && f < kF) {
-        *reinterpret_cast<float4*>(&ag[(size_t)tok * kF + f]) = make_float4(v[0], v[1], v[2], v[3]);
+      f32x4 acc[kTB][kFT / 16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (v[r] > 0.f) atomicAdd(&hist[__float_as_uint(v[r]) >> 20], 1u);
+      for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+        for (int j = 0; j < kFT / 16; ++j) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const half8* wt = reinterpret_cast<const half8*>(ws[buf]) + lane;
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb) {
+        half8 wh[kFT / 16], wl[kFT / 16];
+#pragma unroll
+        for (int j = 0; j < kFT / 16; ++j) {
+          wh[j] = wt[((kb * 2 + 0) * 4 + j) * 64];
+          wl[j] = wt[((kb * 2 + 1) * 4 + j) * 64];
+        }
+        // eight accumulators interleaved: no MFMA waits on the one before it
+#pragma unroll
+        for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+          for (int j = 0; j < kFT / 16; ++j)
+            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
+#pragma unroll
+        for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+          for (int j = 0; j < kFT / 16; ++j)
+            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xl[tb][kb], acc[tb][j], 0, 0, 0);
+#pragma unroll
+        for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+          for (int j = 0; j < kFT / 16; ++j)
+            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
+      }
+      // bias, relu, histogram of the positive values, store
+      if (!bad_rows && !__any(bad_w)) {
+#pragma unroll
+        for (int tb = 0; tb < kTB; ++tb) {
+          const int tok = t0 + 16 * tb + li;
+#pragma unroll
+          for (int j = 0; j < kFT / 16; ++j) {
+            const int f = f0 + 16 * j + 4 * lq;
+            const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
+            const float s4[4] = {winv[j].x, winv[j].y, winv[j].z, winv[j].w};
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              // the scales are powers of two: one rounding, that of the sum with the bias
+              const float s = fmaf(acc[tb][j][r] * xinv[tb], s4[r], b4[r]);
+              v[r] = s > 0.f ? s : 0.f;  // relu; non-positive values are never selected
+            }
+            if (tok < a.N && f < kF) {
+              *reinterpret_cast<float4*>(&ag[(size_t)tok * kF + f]) = make_float4(v[0], v[1], v[2], v[3]);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) take(v[r]);
+            }
+          }
+        }
+      } else {
+#pragma unroll 1
+        for (int e = 0; e < kTB * kFT / 4; ++e) {
+          const int tok = t0 + 16 * (e >> 4) + li, f = f0 + 16 * ((e >> 2) & 3) + 4 * lq + (e & 3);
+          if (tok < a.N && f < kF) {
+            const float s = exact_value<KT>(a, g, tok, f), v = s > 0.f ? s : 0.f;
+            ag[(size_t)tok * kF + f] = v;
+            take(v);
+          }
+        }
       }
     }
     if (more) {  // the other buffer was last read before the previous barrier
@@ -1105,7 +1226,7 @@ using namespace prismkv;
 // therefore serves every smaller block: no call finds another call's
 // activations or list where it expects zeroed histograms.
 struct UpdateLayout {
-  size_t hist, ctl, tcount, part, act, list, total;
+  size_t hist, ctl, tcount, part, wsplit, wscale, act, list, total;
   unsigned list_cap;
   UpdateLayout(int groups, int N) {
     size_t o = 0;
@@ -1114,6 +1235,8 @@ struct UpdateLayout {
     ctl = take((size_t)groups * kCtl * sizeof(unsigned));
     tcount = take((size_t)groups * kMaxTieBlocks * 2 * sizeof(unsigned));
     part = take((size_t)groups * kCenterParts * kD * sizeof(double));
+    wsplit = take((size_t)groups * kFTiles * kWTile * sizeof(_Float16));
+    wscale = take((size_t)groups * kFTiles * kFT * sizeof(float));
     act = take((size_t)groups * N * kF * sizeof(float));
     // the compact list: room for 16 candidates per key (twice the 8 H
     // budget of an index build) plus the chunk tails, at least 2^19
@@ -1139,6 +1262,8 @@ static UpdateArgs make_args(uint64_t k, uint64_t W, uint64_t b, uint64_t center,
   a.counts = reinterpret_cast<int*>(counts);
   a.moments = reinterpret_cast<float*>(moments);
   a.act = reinterpret_cast<float*>(w + L.act);
+  a.wsplit = reinterpret_cast<_Float16*>(w + L.wsplit);
+  a.wscale = reinterpret_cast<float*>(w + L.wscale);
   a.hist = reinterpret_cast<unsigned*>(w + L.hist);
   a.ctl = reinterpret_cast<unsigned*>(w + L.ctl);
   a.tcount = reinterpret_cast<unsigned*>(w + L.tcount);
@@ -1157,13 +1282,31 @@ static UpdateArgs make_args(uint64_t k, uint64_t W, uint64_t b, uint64_t center,
   return a;
 }
 
+// Bucket-tile parts of an encode over `rows` (token tiles x groups) workgroups
+// per part: one workgroup runs per CU, so a launch takes ceil(rows P / 256)
+// rounds of ceil(47 / P) tiles each plus about two tiles' time to load and
+// split its keys; the P of the least total.
+static int encode_parts(int rows) {
+  int best = 1;
+  long long least = -1;
+  for (int p = 1; p <= kFTiles; ++p) {
+    const long long cost = ((long long)rows * p + 255) / 256 * ((kFTiles + p - 1) / p + 2);
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = p;
+    }
+  }
+  return best;
+}
+
 // encode .. ties: the exact batch-wide positive Top-k of the N keys' activations
 // and their bitmap bits.
 template <typename KT>
 static void launch_selection(const UpdateArgs& a, int groups, hipStream_t s) {
   const int token_tiles = (a.N + kEncTokens - 1) / kEncTokens;
-  const int parts = std::max(1, std::min(kFTiles, (kEncMinWgs + token_tiles * groups - 1) / (token_tiles * groups)));
-  hipLaunchKernelGGL(encode_kernel<KT>, dim3(token_tiles, parts, groups), dim3(kET), 0, s, a);
+  hipLaunchKernelGGL(wsplit_kernel, dim3(kFTiles, groups), dim3(kUT), 0, s, a);
+  hipLaunchKernelGGL(encode_kernel<KT>, dim3(token_tiles, encode_parts(token_tiles * groups), groups), dim3(kET), 0, s,
+                     a);
   hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, 0);
   for (int level = 1; level < kLevels; ++level) {
     hipLaunchKernelGGL(refine_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a, level);

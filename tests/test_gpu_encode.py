@@ -1,0 +1,105 @@
+"""The encode of the index update and build (relu((k - center) / scale W^T + b),
+src/prismkv/core.py:47-48,98) where its f16 split or its tiles can go wrong:
+blocks around a workgroup's 256 tokens and a wave's 32, rows and buckets of
+extreme magnitudes (scaled per row and per bucket), and rows and buckets that
+are not split (all zero, beyond 2^60, infinite or NaN)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import expect
+
+pytestmark = pytest.mark.gpu
+
+F, G, D, H = 3000, 8, 128, 40
+
+
+def run_append(k, W, b, center, scale, block, key_mean=8):
+    from prismkv_amd import Native8B
+    zeros = torch.zeros(G, F, dtype=torch.int64, device="cuda")
+    op = Native8B.from_tables(H, zeros, torch.zeros(G, F, D, device="cuda"), torch.zeros(G, F, D, device="cuda"),
+                              torch.zeros(G, 1, dtype=torch.int32, device="cuda"),
+                              torch.zeros(G, F + 1, dtype=torch.int32, device="cuda"), center=center,
+                              capacity=H + block)
+    op.set_encoder_tables(W, b, scale, key_mean)
+    op.append(k, block)
+    torch.cuda.synchronize()
+    return op, op.update_activations(block)
+
+
+def inputs(block, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    k = torch.randn(G, H + block, D, generator=gen, device="cuda").to(torch.bfloat16)
+    W = torch.randn(G, F, D, generator=gen, device="cuda") / D ** 0.5
+    b = 0.05 * torch.randn(G, F, generator=gen, device="cuda")
+    center = 0.1 * torch.randn(G, D, generator=gen, device="cuda")
+    scale = torch.linspace(0.7, 2.0, G, device="cuda")
+    return k, W, b, center, scale
+
+
+def check(k, W, b, center, scale, act, rows=slice(None), buckets=slice(None)):
+    for g in range(G):
+        # x in fp32 with the device's operations, the sums in 64 bits
+        x = ((k[g, H:].float() - center[g]) / scale[g])[rows].cpu().numpy()
+        w, bg = W[g][buckets].cpu().numpy(), b[g][buckets].cpu().numpy()
+        want = np.maximum(x.astype(np.float64) @ w.astype(np.float64).T + bg, 0.0)
+        # the bound of any fp32 summation order of the 128 products (expect.encode_error_bound)
+        bound = (D + 2) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T) + \
+            2.0 ** -24 * np.abs(bg)
+        got = act[g][rows][:, buckets].cpu().numpy().astype(np.float64)
+        assert (np.abs(got - want) <= bound + 1e-45).all(), (g, float(np.abs(got - want).max()))
+
+
+@pytest.mark.parametrize("block", [1, 15, 31, 33, 255, 256, 257, 513, 4096])
+def test_encode_tile_edges(block):
+    k, W, b, center, scale = inputs(block, 400 + block)
+    op, act = run_append(k, W, b, center, scale, block)
+    check(k, W, b, center, scale, act)
+    assert int(op.n.sum()) == G * 8 * block  # the budget, exactly
+
+
+def test_encode_is_closer_to_64_bits_than_an_fp32_chain():
+    # the split's products and sums are off by less than 128 fp32 roundings: 1.4e-7
+    # measured, 2.1e-7 for fp32 MFMA chains; the bound lies between the two
+    k, W, b, center, scale = inputs(1024, 5)
+    _, act = run_append(k, W, b, center, scale, 1024)
+    x = (k[:, H:].float() - center[:, None]) / scale[:, None, None]
+    want = torch.stack([torch.relu(x[g].double() @ W[g].double().T + b[g].double()) for g in range(G)])
+    assert float((act.double() - want).norm() / want.norm()) < 1.8e-7
+
+
+@pytest.mark.parametrize("exponent", [-100, -59, -30, 30, 55])
+def test_encode_row_and_bucket_scales(exponent):
+    # keys and buckets spread over 2^exponent: per-row and per-bucket powers of two (and,
+    # beyond 2^60, the plain fp32 chains) keep the relative precision of each
+    k, W, b, center, scale = inputs(300, 71)
+    center.zero_()
+    k[:, H::3] = (k[:, H::3].float() * 2.0 ** exponent).to(torch.bfloat16)
+    W[:, ::5] *= 2.0 ** (-exponent)
+    b[:, ::5] = 0.0
+    b[:, 1::5] = 0.0
+    _, act = run_append(k, W, b, center, scale, 300)
+    check(k, W, b, center, scale, act)
+
+
+def test_encode_rows_and_buckets_that_are_not_split():
+    k, W, b, center, scale = inputs(290, 72)
+    center.zero_()
+    k[:, H + 7] = 0                      # a zero row: relu(b)
+    k[2, H + 40, 5] = float("inf")       # its activations: +inf or 0 with the sign of W's column
+    k[3, H + 41] = float("nan")          # all NaN sums: relu keeps none
+    W[4, 17] = 0                         # a dead bucket
+    W[5, 2999, 3] = float("inf")
+    W[6, 64] = W[6, 64] * 2.0 ** 80      # beyond the split's range
+    b[6, 64] = 0
+    _, act = run_append(k, W, b, center, scale, 290)
+    assert torch.equal(act[:5, 7], torch.relu(b[:5]))
+    want = torch.where(W[2, :, 5] > 0, float("inf"), 0.0)
+    assert torch.equal(act[2, 40], want)
+    assert not bool(act[3, 41].any())
+    assert torch.equal(act[4, :, 17], torch.relu(b[4, 17]).expand(290))
+    x = (k[5, H:].float() / scale[5])[:, 3]
+    rows = torch.arange(290, device="cuda") != 7
+    assert torch.equal(act[5, rows, 2999], torch.where(x[rows] > 0, float("inf"), 0.0))
+    rest = [r for r in range(290) if r not in (7, 40, 41)]
+    check(k, W, b, center, scale, act, rows=rest, buckets=[f for f in range(F) if f != 2999])
