@@ -269,8 +269,9 @@ uint64_t prismkv_mapped_pointer(uint64_t host);
  *     table) <- Chan merge of the old moments with the block's population
  *     moments, in fp32 and the operation order of core.py:190-199.
  * `work` is prismkv_update_work_bytes(groups, N) bytes, zero-filled once
- * before first use and left zeroed; a workspace sized for the largest block
- * serves every smaller one.  N <= 4096; K rows, W and b 16-byte aligned;
+ * before first use (the bytes from prismkv_update_act_offset on need not be)
+ * and left so; a workspace sized for the largest block serves every smaller
+ * one.  N <= 4096; K rows, W and b 16-byte aligned;
  * returns -1 on bad sizes.  The block's dense activations [G][N][3000] f32
  * stay in the workspace from byte prismkv_update_act_offset(groups) on until
  * the next call (the same offset, for `batch` groups, in prismkv_build's).
@@ -293,7 +294,10 @@ int prismkv_update(uint64_t k, uint64_t W, uint64_t b, uint64_t center, uint64_t
  * population mean and variance of the ORIGINAL keys (core.py:76-89), written
  * directly.  Groups are processed `batch` at a time; `work` is
  * prismkv_build_work_bytes(batch, H) bytes (H x 3000 fp32 activations per
- * group of a batch), zero-filled once before first use and left zeroed.
+ * group of a batch), zero-filled once before first use as prismkv_update's.
+ * With flags & 4 the activations need not be left in the workspace: the
+ * tables are the same, and the activations are not written (they still are
+ * where a group's candidates do not fit their list).
  * H <= 2^20, row_words a multiple of 4 and >= (H+31)/32, bits, W, b and K
  * rows 16-byte aligned; -1 on bad sizes, -2 on unknown flags. */
 size_t prismkv_build_work_bytes(int batch, int H);

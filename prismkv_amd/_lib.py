@@ -112,6 +112,17 @@ def nbytes(t) -> int:
     return t.numel() * t.element_size()
 
 
+def selection_work(nbytes_: int, head: int, device):
+    """A workspace of prismkv_build / prismkv_update: its first `head` bytes
+    (prismkv_update_act_offset) zeroed, the activations and candidate lists
+    behind them not (12 KB per key and group that the kernels write before
+    they read them)."""
+    import torch
+    work = torch.empty(max(nbytes_, 1), dtype=torch.uint8, device=device)
+    work[:head].zero_()
+    return work
+
+
 def load(path=None) -> Library:
     key = str(Path(path or DEFAULT_LIBRARY).resolve())
     lib = _loaded.get(key)

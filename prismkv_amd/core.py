@@ -67,10 +67,10 @@ def _work(name, nbytes, device):
     return buf
 
 
-def _fresh_work(nbytes, device):
-    """A new zero-filled workspace of its own for one build or update, whose
-    activations stay readable in it (index.native keeps no workspace)."""
-    return torch.zeros(max(nbytes, 1), dtype=torch.uint8, device=device)
+def _fresh_work(lib, nbytes, device):
+    """A new workspace of its own for one build or update (index.native keeps
+    no workspace)."""
+    return _lib.selection_work(nbytes, lib.query("prismkv_update_act_offset", 1), device)
 
 
 @dataclass
@@ -243,10 +243,10 @@ def build_index(keys, sae, key_scale, *, center=None):
     scale = torch.tensor([float(key_scale)], dtype=torch.float32, device=device)
     c = torch.zeros(1, DIM, device=device) if center is None else \
         torch.as_tensor(center).to(device=device, dtype=torch.float32).reshape(1, DIM).clone()
-    work = _fresh_work(lib.query("prismkv_build_work_bytes", 1, n), device)
+    work = _fresh_work(lib, lib.query("prismkv_build_work_bytes", 1, n), device)
     lib.call("prismkv_build" + suffix, keys.data_ptr(), W.data_ptr(), b.data_ptr(), c.data_ptr(), scale.data_ptr(),
              t.bits.data_ptr(), t.n.data_ptr(), t.moments.data_ptr(), work.data_ptr(), 1, 1, n, int(sae.key_mean),
-             1 if center is None else 0, keys.stride(0) * n, t.row_words, _lib.nbytes(work), stream=_stream())
+             4 | (1 if center is None else 0), keys.stride(0) * n, t.row_words, _lib.nbytes(work), stream=_stream())
     mean, var = untile_moments(t.moments)
     out = FeatureIndex(n, c[0] if center is None else torch.as_tensor(center).to(device), t.n[0, :FEATURES].long(),
                        mean[0].contiguous(), var[0].contiguous(), _lists_from_bits(t.bits, 0, n))
@@ -274,7 +274,7 @@ def append_index(index, new_keys, sae, key_scale):
     W, b = _encoder(sae, device)
     scale = torch.tensor([float(key_scale)], dtype=torch.float32, device=device)
     c = torch.as_tensor(index.center).to(device=device, dtype=torch.float32).reshape(1, DIM).contiguous()
-    work = _fresh_work(lib.query("prismkv_update_work_bytes", 1, N), device)
+    work = _fresh_work(lib, lib.query("prismkv_update_work_bytes", 1, N), device)
     # the kernels read K rows [H, H + N) of the buffer: address the block as those rows
     row_bytes = DIM * new_keys.element_size()
     base = new_keys.data_ptr() - H * row_bytes

@@ -25,29 +25,33 @@
 //
 // Launches of one update (all G groups at once; the update runs every
 // `interval` tokens, its cost is amortised):
-//   wsplit   W as pairs of f16 in the encode's operand order;
+//   sample   W as pairs of f16 in the encode's operand order, and a histogram
+//            (13 bits) of the positive activations of a few hundred tokens;
 //   encode   the GEMM on the f16 matrix cores, 256 tokens x 64 buckets per
-//            workgroup and step, writes a = relu(...) [G][N][F] and a
-//            histogram of the positive values' top 11 bits (4 replicas of
-//            each global bin, so the flushes do not queue on one address);
-//   digit    one workgroup per group picks the histogram bin holding the
-//            budget-th largest value (3 levels: bits 30..20, 19..9, 8..0);
-//   refine   re-reads a, histograms the values inside the chosen prefix;
-//   emit     sets bitmap bits for a > tau (or all positives when fewer
-//            than the budget are positive) and for a == tau when every tie
-//            fits the budget;
-//   ties     only when ties overflow the budget: per contiguous range of a,
-//            count the ties, then take the first `need` in flat order;
+//            workgroup and step, a = relu(...): the values at or above a floor
+//            read off the sample (about twice the budget of them) go to the
+//            group's candidate list as (flat index, value), and, where the
+//            caller reads them, all of them to [G][N][F];
+//   select   one workgroup per group finds tau, the budget-th largest value,
+//            in the list and, when ties at tau overflow the budget, the flat
+//            index of the last one taken;
+//   emit     sets the members' bitmap bits;
 //   moments  per 32-bucket tile: new members from the bitmap, two-pass
 //            moments of their keys, merge, counts += new.
+// The sample decides only how long the list is.  Where it misjudged (fewer
+// candidates than the budget, or more than the list holds) the same kernels
+// read the dense activations instead, and the result is the same.
 // Keys are the model's bf16 K cache or fp32 rows (the `_f32` entry points):
 // the kernels that read keys take the element type as a template argument
 // and widen every key to fp32 at the load, so both compute the same fp32 /
 // double arithmetic on the values they are given.
 // The build runs the same selection over all H keys of a group (in batches
 // of groups, so the activations of one batch fit the workspace) after a
-// center pass and a bitmap clear, and computes every bucket's moments from
-// scratch (build_moments: one workgroup per bucket, any member count).
+// center pass and a bitmap clear, with select's work spread over many
+// workgroups for long histories (histogram / digit / refine, three levels),
+// and computes every bucket's moments from scratch (build_moments: one
+// workgroup per bucket, any member count).  Unless the caller keeps them, a
+// build never writes its activations (12 KB per key) at all.
 #include <algorithm>
 
 #include "common.h"
@@ -66,13 +70,16 @@ constexpr int kMaxTieBlocks = 4096;  // contiguous ranges of a per group for the
 constexpr int kTieMinLen = 65536;    // values per range at least (multiple of 4 * kUT)
 constexpr int kTieGrid = 256;        // workgroups per group of the tie kernels
 constexpr int kCenterParts = 64;     // row ranges of the center sum
-constexpr int kListChunk = 256;      // list entries a wave reserves at once once its workgroup's buffer is full
-constexpr unsigned kListSlack = (unsigned)kRefineBlocks * (kUT / 64) * kListChunk;  // unfilled chunk tails, at most
+constexpr unsigned kListSlack = 1u << 18;  // list entries beyond kListPerKey per key
+constexpr int kListPerKey = 48;
+constexpr int kSampleShift = 18, kSampleBins = 1 << (31 - kSampleShift);  // 13-bit digits of positive floats: 3.1% each
+constexpr int kSelectMax = 4096;  // keys up to which one workgroup per group selects
 constexpr int kMaxBuild = 1 << 20;   // keys per group of a build (N * F < 2^32 flat indices)
 constexpr int kBuildCenter = 1;      // prismkv_build flag: compute the center (else it is an input)
+constexpr int kBuildNoAct = 4;       // prismkv_build flag: the activations need not be left in the workspace
 
 // ctl words per group
-enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kListed, kListLen, kCtl = 16 };
+enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kFloor, kListLen, kCut, kTieLen, kCtl = 16 };
 enum { kModeTopK = 0, kModeAllPositive = 1 };
 
 // Key loads of the two key element types: 2 or 8 consecutive dims as the
@@ -83,26 +90,40 @@ struct KeyLoad;
 template <>
 struct KeyLoad<uint16_t> {  // bf16
   typedef uint32_t Raw2;
-  static __device__ __forceinline__ Raw2 load2(const uint16_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
+  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, 0, 0);
+  }
   static __device__ __forceinline__ float lo(Raw2 r) { return bf16_lo(r); }
   static __device__ __forceinline__ float hi(Raw2 r) { return bf16_hi(r); }
+  typedef u32x4 Raw8;
+  static __device__ __forceinline__ Raw8 raw8(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
+  static __device__ __forceinline__ float at(const Raw8& r, int j) { return j & 1 ? bf16_hi(r[j >> 1]) : bf16_lo(r[j >> 1]); }
   static __device__ __forceinline__ void load8(const uint16_t* p, float (&x)[8]) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    x[0] = bf16_lo(v.x); x[1] = bf16_hi(v.x); x[2] = bf16_lo(v.y); x[3] = bf16_hi(v.y);
-    x[4] = bf16_lo(v.z); x[5] = bf16_hi(v.z); x[6] = bf16_lo(v.w); x[7] = bf16_hi(v.w);
+    const Raw8 v = raw8(p);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = at(v, j);
   }
 };
 
 template <>
 struct KeyLoad<float> {
-  typedef float2 Raw2;
-  static __device__ __forceinline__ Raw2 load2(const float* p) { return *reinterpret_cast<const float2*>(p); }
-  static __device__ __forceinline__ float lo(Raw2 r) { return r.x; }
-  static __device__ __forceinline__ float hi(Raw2 r) { return r.y; }
+  typedef unsigned Raw2 __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+  }
+  static __device__ __forceinline__ float lo(Raw2 r) { return __uint_as_float(r[0]); }
+  static __device__ __forceinline__ float hi(Raw2 r) { return __uint_as_float(r[1]); }
+  struct Raw8 {
+    u32x4 a, b;
+  };
+  static __device__ __forceinline__ Raw8 raw8(const float* p) {
+    return Raw8{reinterpret_cast<const u32x4*>(p)[0], reinterpret_cast<const u32x4*>(p)[1]};
+  }
+  static __device__ __forceinline__ float at(const Raw8& r, int j) { return __uint_as_float(j < 4 ? r.a[j & 3] : r.b[j & 3]); }
   static __device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
-    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+    const Raw8 v = raw8(p);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = at(v, j);
   }
 };
 
@@ -119,17 +140,35 @@ struct UpdateArgs {
   float* moments;  // [G][kChunks][256][32]
   float* act;      // [G][N][F]
   _Float16* wsplit;  // [G][kFTiles][kWTile] W split for the encode
-  float* wscale;     // [G][kFTiles * 64] the buckets' inverse scales
   unsigned* hist;  // [G][kLevels][kRep][kBins]
   unsigned* ctl;   // [G][kCtl]
   unsigned* tcount;  // [G][tie_blocks] ties per contiguous range of a
-  uint2* list;       // [G][list_cap] (flat index, value bits) of the values at or above tau's first digit
-  unsigned list_cap;  // entries per group (0 bits: an unfilled chunk entry)
+  unsigned* sample;  // [G][kSampleBins] histogram of the sample tokens' positive values
+  uint2* list;       // [G][list_cap] candidates: (flat index, value bits) of the values at or above the floor
+  unsigned* ties;    // [G][list_cap] flat indices of the values equal to tau, when they overflow the budget
+  unsigned list_cap;  // entries per group
+  unsigned target;    // sample values at or above the floor, at least
+  int listed;         // whether the call collects candidates
   int H, N;          // first key row / bitmap column, keys indexed
   long long budget;  // N * key_mean
   int tie_blocks;
   long long tie_len;  // values per range, a multiple of 4 * kUT
 };
+
+__device__ __forceinline__ unsigned budget_of(const UpdateArgs& a) {
+  const long long n = (long long)a.N * kF;
+  return (unsigned)(a.budget < n ? a.budget : n);
+}
+
+// Whether the group's candidate list holds every value the selection can take
+// (after the collecting encode): it did not overflow, and it has the budget's
+// number of values or every positive one.
+__device__ __forceinline__ bool list_ok(const UpdateArgs& a, int g) {
+  if (!a.listed) return false;
+  const unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  const unsigned len = ctl[kListLen];
+  return len <= a.list_cap && (len >= budget_of(a) || ctl[kFloor] <= 1u);
+}
 
 __device__ __forceinline__ unsigned* hist_of(const UpdateArgs& a, int g, int level) {
   return a.hist + ((size_t)g * kLevels + level) * kRep * kBins;
@@ -150,18 +189,19 @@ __device__ __forceinline__ unsigned* hist_of(const UpdateArgs& a, int g, int lev
 // magnitude lies outside 2^+-60 (the scales' products would leave fp32), is
 // not split: its values are computed by plain fp32 chains (exact_value).
 //
-// wsplit: grid (kFTiles, G) x 256 writes W in the order the encode reads it:
-// tile ft (64 buckets) is 32 fragments of 1 KB, [kb (4)][hi, lo][j (4)], lane
-// (i, q) of a fragment holding bucket 64 ft + 16 j + i, dims 32 kb + 8 q .. + 7
-// (an MFMA A operand).  Splitting W here and not in each encode workgroup
-// takes it off the encode's VALU, which its epilogue already fills; it reads
-// and writes 12.3 MB for 8 groups (5 us).
+// The split W of tile ft (64 buckets) is 32 fragments of 1 KB,
+// [kb (4)][hi, lo][j (4)], lane (i, q) = (l % 16, l / 16) of a fragment holding
+// bucket 64 ft + 16 j + i, dims 32 kb + 8 q .. + 7 (an MFMA A operand), then
+// the buckets' biases and inverse scales, so that the encode's loop has no
+// other load that would wait behind the stores of the tile before.  It is
+// made once per call, by the sample kernel, and not in each encode workgroup:
+// that takes it off the encode's VALU, which its epilogue already fills.
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int kScaleExp = 14;   // scaled rows have their largest magnitude in [2^14, 2^15)
 constexpr int kMaxScale = 60;   // |exponent| of a row's or bucket's largest magnitude, at most
-constexpr int kWTile = kFT * kD * 2;  // f16 values of a split W tile
+constexpr int kWTile = kFT * kD * 2 + kFT * 4;  // f16 words of a split W tile: the fragments, 64 biases, 64 inverse scales (fp32)
 constexpr int kKB = kD / 32;          // MFMA dim blocks
 
 // The power of two that scales a row of largest magnitude m, and its inverse;
@@ -183,64 +223,118 @@ __device__ __forceinline__ void split8(const float (&x)[8], float scale, half8& 
   }
 }
 
-// The larger magnitude as bits: NaN and infinities order above every number.
-__device__ __forceinline__ unsigned mag_max(unsigned m, float x) { return max(m, __float_as_uint(x) & 0x7fffffffu); }
-
-__global__ __launch_bounds__(kUT) void wsplit_kernel(UpdateArgs a) {
-  const int ft = blockIdx.x, g = blockIdx.y, j = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int f = ft * kFT + 16 * j + (lane & 15);
-  float w[kKB][8];
-  unsigned m = 0u;
-#pragma unroll
-  for (int kb = 0; kb < kKB; ++kb) {
-    float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
-    if (f < kF) {
-      const float4* row = reinterpret_cast<const float4*>(a.W + ((size_t)g * kF + f) * kD + 32 * kb + 8 * (lane >> 4));
-      u = row[0];
-      v = row[1];
-    }
-    w[kb][0] = u.x; w[kb][1] = u.y; w[kb][2] = u.z; w[kb][3] = u.w;
-    w[kb][4] = v.x; w[kb][5] = v.y; w[kb][6] = v.z; w[kb][7] = v.w;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) m = mag_max(m, w[kb][t]);
-  }
-  m = max(m, (unsigned)__shfl_xor((int)m, 16));
-  m = max(m, (unsigned)__shfl_xor((int)m, 32));
-  const float2 sc = row_scale(__uint_as_float(m));
-  _Float16* tile = a.wsplit + ((size_t)g * kFTiles + ft) * kWTile;
-#pragma unroll
-  for (int kb = 0; kb < kKB; ++kb) {
-    half8 hi, lo;
-    split8(w[kb], sc.x, hi, lo);
-    *reinterpret_cast<half8*>(tile + ((kb * 2 + 0) * 4 + j) * 512 + lane * 8) = hi;
-    *reinterpret_cast<half8*>(tile + ((kb * 2 + 1) * 4 + j) * 512 + lane * 8) = lo;
-  }
-  if (lane < 16) a.wscale[((size_t)g * kFTiles + ft) * kFT + 16 * j + lane] = sc.y;
-}
-
-// ---------------------------------------------------------------------------
-// encode: grid (ceil(N / 256), P, G) x 512.  Workgroup (y, part) takes the
-// tokens [256 y, 256 y + 256), wave w the 32 rows 256 y + 32 w + 16 tb + i, and
-// the bucket tiles part, part + P, ... (64 buckets each).  The wave's
-// x = (k - center) / scale is computed in fp32 and split once, into registers
-// (64 of them), and each bucket tile's split W streams through LDS,
-// double-buffered: the next tile is requested into registers while the current
-// one is multiplied.  Products run on v_mfma_f32_16x16x32_f16 (lane (i, q) =
-// (l % 16, l / 16) feeds A[i][8 q + t] and B[8 q + t][i], t = 0..7, and holds
-// D[4 q + r][i]): A is W (bucket rows) and B is x (token columns), so lane
-// (i, q) ends with buckets 4 q .. 4 q + 3 of token i, stored as one 16-byte
-// store.  32 tokens per wave, because a wave reads the whole 32 KB tile from
-// LDS whatever its tokens: at 16 the 8 waves' reads took as long as their
-// products.  P is chosen on the host (encode_parts).  8 groups, MI355X, with
-// the fp32 MFMA kernel's time before: 1024 tokens 46.6 us (78), 4096 148 us
-// (262), 65536 3.02 ms (4.10); what is left is the histogram's LDS atomics and
-// the 12 KB per token of activations, not the products.
-// ---------------------------------------------------------------------------
 constexpr int kET = 512;                          // encode workgroup
 constexpr int kTB = 2;                            // 16-token blocks per wave
 constexpr int kRowTile = 16 * kTB;                // tokens per wave
 constexpr int kEncTokens = kET / 64 * kRowTile;   // tokens per workgroup (256)
-constexpr int kWLoads = kWTile * 2 / 16 / kET;    // 16-byte loads of a W tile per thread (4)
+constexpr int kWLoads = kFT * kD * 4 / 16 / kET;  // 16-byte loads of a W tile per thread (4),
+constexpr int kWTail = kFT * 8 / 16;              // and of its biases and scales, by the first threads (32)
+constexpr int kWRows = kWTile * 2 / 16;           // 16-byte words of a tile
+constexpr int kJ = kFT / 16;                      // 16-bucket columns of a tile (4)
+
+// The wave's key rows and its center, as loaded: lane (i, q) takes dims
+// 32 kb + 8 q .. + 7 of its own tokens.  All of it is requested before any is
+// used, so the split below waits for one memory round trip.
+template <typename KT>
+struct RowsRaw {
+  typename KeyLoad<KT>::Raw8 k[kTB][kKB];
+  f32x4 c[kKB][2];
+  float scale;
+  __device__ __forceinline__ void load(const UpdateArgs& a, int g, const int (&tok)[kTB]) {
+    const int lq = (threadIdx.x >> 4) & 3;
+    const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + 8 * lq;
+    const float* cg = a.center + (size_t)g * kD + 8 * lq;
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+      for (int kb = 0; kb < kKB; ++kb)
+        k[tb][kb] = KeyLoad<KT>::raw8(kg + (size_t)(a.H + tok[tb]) * kD + 32 * kb);
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb) {
+      c[kb][0] = *reinterpret_cast<const f32x4*>(cg + 32 * kb);
+      c[kb][1] = *reinterpret_cast<const f32x4*>(cg + 32 * kb + 4);
+    }
+    scale = a.scale[g];
+  }
+};
+
+// d / s in fp32, rounded to nearest, for many d: r = 1 / s (rounded), one
+// product, its remainder and one correction, which round as the division does
+// while nothing leaves the normal range (8e8 random pairs, none differs); an
+// infinite or NaN d gives NaN, a row that the split does not serve.
+__device__ __forceinline__ float divide_by(float d, float s, float r) {
+  const float q = d * r;
+  return fmaf(fmaf(-q, s, d), r, q);
+}
+
+// The split x = (k - center) / key_scale (fp32, core.py:98) of the wave's
+// tokens.  xinv: the inverse of each row's scale; returns whether a row of the
+// wave is not split.
+template <typename KT>
+__device__ __forceinline__ bool split_rows(const RowsRaw<KT>& raw, half8 (&xh)[kTB][kKB], half8 (&xl)[kTB][kKB],
+                                           float (&xinv)[kTB]) {
+  const float s = raw.scale, rs = 1.0f / s;
+  // (the scale's own range bounds what divide_by may meet)
+  bool bad = !(fabsf(s) >= 0x1p-60f && fabsf(s) <= 0x1p60f);
+#pragma unroll
+  for (int tb = 0; tb < kTB; ++tb) {
+    float x[kKB][8], m = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb)
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const float d = KeyLoad<KT>::at(raw.k[tb][kb], t) - raw.c[kb][t >> 2][t & 3];
+        m = fmaxf(m, fabsf(d));  // NaN is passed over: its sums are NaN either way
+        x[kb][t] = divide_by(d, s, rs);
+      }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    const float2 s2 = row_scale(fabsf(divide_by(m, s, rs)));  // the largest |x|; NaN for an infinite m
+    xinv[tb] = s2.y;
+    bad |= s2.y == 0.f;
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb) split8(x[kb], s2.x, xh[tb][kb], xl[tb][kb]);
+  }
+  return __any(bad);
+}
+
+// acc[tb][j] = the products of the wave's 32 tokens with a split W tile in LDS:
+// v_mfma_f32_16x16x32_f16, lane (i, q) feeding A[i][8 q + t] and B[8 q + t][i],
+// t = 0..7, and holding D[4 q + r][i].  A is W (bucket rows), B is x (token
+// columns), so lane (i, q) ends with buckets 16 j + 4 q + r of token i.
+__device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)[kTB][kKB], const half8 (&xl)[kTB][kKB],
+                                              f32x4 (&acc)[kTB][kJ]) {
+  const half8* wt = reinterpret_cast<const half8*>(ws) + (threadIdx.x & 63);
+#pragma unroll
+  for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kb = 0; kb < kKB; ++kb) {
+    half8 wh[kJ], wl[kJ];
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+      wh[j] = wt[((kb * 2 + 0) * kJ + j) * 64];
+      wl[j] = wt[((kb * 2 + 1) * kJ + j) * 64];
+    }
+    // eight accumulators interleaved: no MFMA waits on the one before it
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+        acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+        acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xl[tb][kb], acc[tb][j], 0, 0, 0);
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+        acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
+  }
+}
 
 // relu(x . w + b) of key row `tok` of the block and bucket f by one fp32 chain:
 // rows and buckets that the split does not serve.
@@ -256,150 +350,333 @@ __device__ float exact_value(const UpdateArgs& a, int g, int tok, int f) {
   return s + a.b[(size_t)g * kF + f];
 }
 
+// The values of one bucket tile for the wave's tokens, after the products:
+// four(tb, j, v) gets lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3,
+// in rolled form one(tb, j, r, v) where a row or bucket is not split.  `tok` is
+// the lane's two tokens; sg the tile's biases, then its inverse bucket scales.
+template <typename KT, typename Four, typename One>
+__device__ __forceinline__ void tile_values(const UpdateArgs& a, int g, int f0, const int (&tok)[kTB],
+                                            const float (&xinv)[kTB], bool bad_rows, const float* sg,
+                                            const f32x4 (&acc)[kTB][kJ], Four four, One one) {
+  const int lq = (threadIdx.x >> 4) & 3;
+  float4 bias[kJ], winv[kJ];
+  bool bad_w = false;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const int o = 16 * j + 4 * lq;
+    bias[j] = *reinterpret_cast<const float4*>(sg + o);
+    winv[j] = *reinterpret_cast<const float4*>(sg + kFT + o);
+    bad_w |= winv[j].x == 0.f || winv[j].y == 0.f || winv[j].z == 0.f || winv[j].w == 0.f;
+  }
+  if (!bad_rows && !__any(bad_w)) {
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
+        const float s4[4] = {winv[j].x, winv[j].y, winv[j].z, winv[j].w};
+        float v[4];
+        // the scales are powers of two: one rounding, that of the sum with the bias
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fmaf(acc[tb][j][r] * xinv[tb], s4[r], b4[r]);
+        four(tb, j, v);
+      }
+  } else {
+#pragma unroll 1
+    for (int e = 0; e < kTB * kJ * 4; ++e) {
+      const int tb = e >> 4, j = (e >> 2) & 3, f = f0 + 16 * j + 4 * lq + (e & 3);
+      one(tb, j, e & 3, f < kF ? exact_value<KT>(a, g, tb ? tok[1] : tok[0], f) : 0.f);
+    }
+  }
+}
+
+// Token of sample row r of S (a.N tokens): one of each N / S consecutive ones,
+// at a place that r decides, so that no period of the text meets the sample's.
+__device__ __forceinline__ int sample_token(int r, int S, int N) {
+  if (S == N) return r;
+  const unsigned step = (unsigned)N / (unsigned)S;
+  return (int)((long long)r * N / S) + (int)((((unsigned)r * 0x9E3779B9u) >> 8) % step);
+}
+
+// Where the histogram keeps a bin: 37 words from its neighbour's, so that the
+// bins of an octave, which every workgroup adds to, lie in lines of their own
+// (the atomics of a line are serial); and the inverse of 37 mod 8192.
+constexpr unsigned kPlace = 37u, kPlaceInverse = 7085u;
+static_assert((kPlace * kPlaceInverse) % kSampleBins == 1u, "inverse places");
+__device__ __forceinline__ unsigned sample_place(unsigned bin) { return bin * kPlace % kSampleBins; }
+
+// ---------------------------------------------------------------------------
+// sample: grid (max(ceil(S / 256), 1), kFTiles, G) x 512.  Splits bucket tile
+// ft of W (the first token tile's workgroups write it for the encode), and adds
+// to the group's histogram, for each of S sample tokens and each 16 buckets of
+// the tile (a lane's), the largest activation if it is positive.  Around tau a
+// token's 16 buckets hold 0.04 values, so that counts all but 4% of them; a
+// token that outweighs the others (a hundred times the memberships) counts
+// for 188 at most, and the floor stays one that serves the others.  S = 0 only
+// splits.
+// ---------------------------------------------------------------------------
 template <typename KT>
+__global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
+  const int y = blockIdx.x, ft = blockIdx.y, g = blockIdx.z, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  __shared__ __align__(16) u32x4 ws[kWRows];
+  __shared__ unsigned hist[kSampleBins];
+  const int r0 = y * kEncTokens + w * kRowTile;  // the wave's first sample row
+  const bool live = r0 < S;                      // uniform per wave
+  int tok[kTB];
+  RowsRaw<KT> raw;
+  if (live) {
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb) tok[tb] = sample_token(min(r0 + 16 * tb + (lane & 15), S - 1), S, a.N);
+    raw.load(a, g, tok);
+  }
+  if (w < kJ) {  // wave j splits the tile's column j
+    const int f = ft * kFT + 16 * w + (lane & 15);
+    float x[kKB][8], m = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb) {
+      float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+      if (f < kF) {
+        const float4* row = reinterpret_cast<const float4*>(a.W + ((size_t)g * kF + f) * kD + 32 * kb + 8 * (lane >> 4));
+        u = row[0];
+        v = row[1];
+      }
+      x[kb][0] = u.x; x[kb][1] = u.y; x[kb][2] = u.z; x[kb][3] = u.w;
+      x[kb][4] = v.x; x[kb][5] = v.y; x[kb][6] = v.z; x[kb][7] = v.w;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) m = fmaxf(m, fabsf(x[kb][t]));
+    }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    const float2 sc = row_scale(m);
+    half8* lds = reinterpret_cast<half8*>(ws) + lane;
+    half8* out = reinterpret_cast<half8*>(a.wsplit + ((size_t)g * kFTiles + ft) * kWTile) + lane;
+#pragma unroll
+    for (int kb = 0; kb < kKB; ++kb) {
+      half8 hi, lo;
+      split8(x[kb], sc.x, hi, lo);
+      lds[((kb * 2 + 0) * kJ + w) * 64] = hi;
+      lds[((kb * 2 + 1) * kJ + w) * 64] = lo;
+      if (y == 0) {
+        out[((kb * 2 + 0) * kJ + w) * 64] = hi;
+        out[((kb * 2 + 1) * kJ + w) * 64] = lo;
+      }
+    }
+    if (lane < 16) {
+      float* tail = reinterpret_cast<float*>(ws + kET * kWLoads) + 16 * w + lane;
+      tail[0] = f < kF ? a.b[(size_t)g * kF + f] : 0.f;
+      tail[kFT] = sc.y;
+      if (y == 0) {
+        float* t = reinterpret_cast<float*>(a.wsplit + ((size_t)g * kFTiles + ft) * kWTile + kFT * kD * 2) + 16 * w + lane;
+        t[0] = tail[0];
+        t[kFT] = tail[kFT];
+      }
+    }
+  }
+  if (y == 0 && ft == 0 && tid == 0) a.ctl[(size_t)g * kCtl + kListLen] = 0u;
+  if (S == 0) return;  // uniform
+  for (int i = tid; i < kSampleBins; i += kET) hist[i] = 0u;
+  half8 xh[kTB][kKB], xl[kTB][kKB];
+  float xinv[kTB];
+  bool bad_rows = false;
+  if (live) bad_rows = split_rows<KT>(raw, xh, xl, xinv);
+  __syncthreads();
+  if (live) {
+    f32x4 acc[kTB][kJ];
+    tile_products(ws, xh, xl, acc);
+    float most[kTB] = {0.f, 0.f};
+    tile_values<KT>(a, g, ft * kFT, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws + kET * kWLoads), acc,
+                    [&](int tb, int j, const float (&v)[4]) {
+      most[tb] = fmaxf(most[tb], fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+    }, [&](int tb, int j, int r, float v) {
+      if (tb) most[1] = fmaxf(most[1], v); else most[0] = fmaxf(most[0], v);
+    });
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb)
+      if (r0 + 16 * tb + (lane & 15) < S && most[tb] > 0.f)
+        atomicAdd(&hist[__float_as_uint(most[tb]) >> kSampleShift], 1u);
+  }
+  __syncthreads();
+  unsigned* sh = a.sample + (size_t)g * kSampleBins;
+  for (int i = tid; i < kSampleBins; i += kET)
+    if (hist[i]) atomicAdd(&sh[sample_place(i)], hist[i]);
+}
+
+// ---------------------------------------------------------------------------
+// encode: grid (ceil(N / 256), P, G) x 512.  Workgroup (y, part) takes the
+// tokens [256 y, 256 y + 256), wave w the 32 rows 256 y + 32 w + 16 tb + i, and
+// the bucket tiles part, part + P, ... (64 buckets each).  The wave's x is
+// computed and split once, into registers (64 of them), and each bucket tile's
+// split W streams through LDS, double-buffered: the next tile is requested into
+// registers while the current one is multiplied.  32 tokens per wave, because
+// a wave reads the whole 32 KB tile from LDS whatever its tokens: at 16 the 8
+// waves' reads took as long as their products.  P is chosen on the host
+// (encode_parts).
+//
+// kCollect: the values at or above the group's floor, the lower edge of the
+// sample histogram's bin that holds the target-th largest value, go to the
+// candidate list: each wave gathers its own in LDS (places from a ballot, no
+// atomics) and moves them to a range of the list that it reserves with one
+// atomic; the workgroup's rest goes out together at the end.  An LDS histogram
+// of every positive value instead, 1024 per wave and tile on some thirty bins,
+// took longer than the products (64K keys, 8 groups: 3.0 ms and a 1.3 ms pass
+// over the stored activations; now 1.33 ms and no pass).  The products alone
+// take 0.90 ms of it (1.3 PFLOP/s; a large f16 library product reaches 1.2),
+// the epilogue's multiply-add, compare and branch per value the rest.
+// kStore: every activation is written, one 16-byte store per lane and column.
+// Without kCollect the kernel is the dense path of a call that collects no
+// candidates, or whose list turned out unusable (else it returns at once).
+// ---------------------------------------------------------------------------
+constexpr int kWaveBuf = 512;  // candidates a wave gathers; a column of 4 values adds at most 256
+
+template <typename KT, bool kStore, bool kCollect>
 __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   const int y = blockIdx.x, part = blockIdx.y, parts = gridDim.y, g = blockIdx.z, tid = threadIdx.x;
   const int w = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
-  __shared__ __align__(16) u32x4 ws[2][kET * kWLoads];  // [buffer][a split W tile]
-  __shared__ unsigned hist[kBins];
+  __shared__ __align__(16) u32x4 ws[2][kWRows];  // [buffer][a split W tile]
+  __shared__ uint2 cand[kCollect ? kET / 64 : 1][kCollect ? kWaveBuf : 1];
+  __shared__ unsigned wsum[kET / 64], floor_s, base_s;
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  if constexpr (!kCollect)
+    if (list_ok(a, g)) return;  // uniform
   const int t0 = y * kEncTokens + w * kRowTile;  // the wave's first token
   const bool live = t0 < a.N;                    // uniform per wave: a wave without tokens only moves W
   const u32x4* wg = reinterpret_cast<const u32x4*>(a.wsplit + (size_t)g * kFTiles * kWTile);
-  auto load_w = [&](int ft, u32x4 (&r)[kWLoads]) {
+  auto load_w = [&](int ft, u32x4 (&r)[kWLoads + 1]) {
 #pragma unroll
-    for (int u = 0; u < kWLoads; ++u) r[u] = wg[(size_t)ft * (kET * kWLoads) + tid + kET * u];
+    for (int u = 0; u < kWLoads; ++u) r[u] = wg[(size_t)ft * kWRows + tid + kET * u];
+    r[kWLoads] = wg[(size_t)ft * kWRows + kET * kWLoads + (tid & (kWTail - 1))];
   };
-  auto store_w = [&](int buf, const u32x4 (&r)[kWLoads]) {
+  auto store_w = [&](int buf, const u32x4 (&r)[kWLoads + 1]) {
 #pragma unroll
     for (int u = 0; u < kWLoads; ++u) ws[buf][tid + kET * u] = r[u];
+    if (tid < kWTail) ws[buf][kET * kWLoads + tid] = r[kWLoads];
   };
-  u32x4 wr[kWLoads];
-  load_w(part, wr);
-  for (int i = tid; i < kBins; i += kET) hist[i] = 0;
-  // x = (k - center) / key_scale in fp32 (core.py:98): lane (i, q) holds dims
-  // 32 kb + 8 q .. + 7 of tokens t0 + i and t0 + 16 + i
+  // the part's bucket tiles: consecutive ones, whose stores meet in the lines of a token's row
+  const int first = part * kFTiles / parts, last = (part + 1) * kFTiles / parts;
+  u32x4 wr[kWLoads + 1];
+  load_w(first, wr);
   half8 xh[kTB][kKB], xl[kTB][kKB];
   float xinv[kTB];
-  bool bad_x = false;
+  int tok[kTB];
+  bool bad_rows = false;
   if (live) {
-    const float sc = a.scale[g];
-    const float* cg = a.center + (size_t)g * kD + 8 * lq;
-    const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + 8 * lq;
+    RowsRaw<KT> raw;
 #pragma unroll
-    for (int tb = 0; tb < kTB; ++tb) {
-      const int row = a.H + min(t0 + 16 * tb + li, a.N - 1);  // rows past the block repeat the last one (masked below)
-      float x[kKB][8];
-      unsigned m = 0u;
-#pragma unroll
-      for (int kb = 0; kb < kKB; ++kb) KeyLoad<KT>::load8(kg + (size_t)row * kD + 32 * kb, x[kb]);
-#pragma unroll
-      for (int kb = 0; kb < kKB; ++kb)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          x[kb][t] = (x[kb][t] - cg[32 * kb + t]) / sc;
-          m = mag_max(m, x[kb][t]);
-        }
-      m = max(m, (unsigned)__shfl_xor((int)m, 16));
-      m = max(m, (unsigned)__shfl_xor((int)m, 32));
-      const float2 s2 = row_scale(__uint_as_float(m));
-      xinv[tb] = s2.y;
-      bad_x |= s2.y == 0.f;
-#pragma unroll
-      for (int kb = 0; kb < kKB; ++kb) split8(x[kb], s2.x, xh[tb][kb], xl[tb][kb]);
-    }
+    for (int tb = 0; tb < kTB; ++tb)
+      tok[tb] = min(t0 + 16 * tb + li, a.N - 1);  // rows past the block repeat the last one (masked below)
+    raw.load(a, g, tok);
+    bad_rows = split_rows<KT>(raw, xh, xl, xinv);
   }
-  const bool bad_rows = __any(bad_x);
   store_w(0, wr);
-  __syncthreads();
-  const float* bg = a.b + (size_t)g * kF;
-  const float* sg = a.wscale + (size_t)g * kFTiles * kFT;
-  float* ag = a.act + (size_t)g * a.N * kF;
-  auto take = [&](float v) {  // histogram of a positive value
-    if (v > 0.f) atomicAdd(&hist[__float_as_uint(v) >> 20], 1u);
+  float least[kTB];  // the lane's floor per token: NaN (nothing is collected) for rows past the block
+  if constexpr (kCollect) {
+    // every workgroup reads the same histogram and puts its bins in order, in
+    // the buffer of the second W tile; then thread t has the 16 bins below 8192 - 16 t
+    constexpr int kPer = kSampleBins / kET;
+    const uint4* sh = reinterpret_cast<const uint4*>(a.sample + (size_t)g * kSampleBins);
+    unsigned* ordered = reinterpret_cast<unsigned*>(ws[1]);
+    uint4 h[kPer / 4];
+#pragma unroll
+    for (int u = 0; u < kPer / 4; ++u) h[u] = sh[tid + kET * u];
+#pragma unroll
+    for (int u = 0; u < kPer / 4; ++u) {
+      const unsigned at = 4u * (unsigned)(tid + kET * u);
+      ordered[at * kPlaceInverse % kSampleBins] = h[u].x;
+      ordered[(at + 1u) * kPlaceInverse % kSampleBins] = h[u].y;
+      ordered[(at + 2u) * kPlaceInverse % kSampleBins] = h[u].z;
+      ordered[(at + 3u) * kPlaceInverse % kSampleBins] = h[u].w;
+    }
+    __syncthreads();
+    unsigned c[kPer], tot = 0u;
+#pragma unroll
+    for (int u = 0; u < kPer / 4; ++u) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(&ordered[kSampleBins - kPer * (tid + 1) + 4 * u]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        c[4 * u + i] = v[i];
+        tot += v[i];
+      }
+    }
+    if (tid == 0) floor_s = 1u;  // too few positive values in the sample: every one is collected
+    unsigned run = block_incl_scan<kET>(tot, wsum) - tot;
+    if (run < a.target && run + tot >= a.target) {
+#pragma unroll
+      for (int u = kPer - 1; u >= 0; --u) {
+        if (run < a.target && run + c[u] >= a.target)
+          floor_s = max(1u, (unsigned)(kSampleBins - kPer * (tid + 1) + u) << kSampleShift);
+        run += c[u];
+      }
+    }
+    __syncthreads();
+    if (y == 0 && part == 0 && tid == 0) ctl[kFloor] = floor_s;
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb) least[tb] = t0 + 16 * tb + li < a.N ? __uint_as_float(floor_s) : __builtin_nanf("");
+  } else {
+    __syncthreads();
+  }
+  // the wave's activation rows; stores past them (rows past the block, buckets
+  // past F) carry an offset outside the resource and are dropped
+  const int rows = min(kRowTile, a.N - t0);
+  const __amdgpu_buffer_rsrc_t ar = raw_buffer(a.act + ((size_t)g * a.N + (live ? t0 : 0)) * kF,
+                                               kStore && live ? rows * kF * (int)sizeof(float) : 0);
+  uint2* list = a.list + (size_t)g * a.list_cap;
+  unsigned n = 0u;  // the wave's gathered candidates (uniform)
+  auto put = [&](unsigned at, unsigned i) {
+    if (at + i < a.list_cap) list[at + i] = cand[kCollect ? w : 0][i];
+  };
+  auto gather = [&](bool in, unsigned flat, float v) {
+    const unsigned long long m = __ballot(in);
+    if (m) {  // uniform
+      if (in)
+        cand[kCollect ? w : 0][n + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
+            make_uint2(flat, __float_as_uint(v));
+      n += (unsigned)__popcll(m);
+    }
+  };
+  auto flush = [&]() {
+    if (n <= kWaveBuf - 256) return;  // uniform
+    __builtin_amdgcn_wave_barrier();
+    unsigned at = 0u;
+    if (lane == 0) at = atomicAdd(&ctl[kListLen], n);
+    at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+    for (unsigned i = lane; i < n; i += 64) put(at, i);
+    __builtin_amdgcn_wave_barrier();
+    n = 0u;
   };
   int buf = 0;
-  for (int ft = part; ft < kFTiles; ft += parts) {  // uniform
-    const bool more = ft + parts < kFTiles;
-    if (more) load_w(ft + parts, wr);  // in flight while this tile is multiplied
+  for (int ft = first; ft < last; ++ft) {  // uniform
+    const bool more = ft + 1 < last;
+    if (more) load_w(ft + 1, wr);  // in flight while this tile is multiplied
     if (live) {
       const int f0 = ft * kFT;
-      // lane (i, q): buckets f0 + 16 j + 4 q .. + 3; kF is a multiple of 4, so
-      // those 4 buckets are live together
-      float4 bias[kFT / 16], winv[kFT / 16];
-      bool bad_w = false;
-#pragma unroll
-      for (int j = 0; j < kFT / 16; ++j) {
+      f32x4 acc[kTB][kJ];
+      tile_products(ws[buf], xh, xl, acc);
+      // (a bucket past F has a zero row and bias: its 0 is below every floor)
+      tile_values<KT>(a, g, f0, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws[buf] + kET * kWLoads), acc,
+                      [&](int tb, int j, const float (&v)[4]) {
         const int f = f0 + 16 * j + 4 * lq;
-        bias[j] = f < kF ? *reinterpret_cast<const float4*>(bg + f) : make_float4(0.f, 0.f, 0.f, 0.f);
-        winv[j] = *reinterpret_cast<const float4*>(sg + f);
-        bad_w |= winv[j].x == 0.f || winv[j].y == 0.f || winv[j].z == 0.f || winv[j].w == 0.f;
-      }
-      f32x4 acc[kTB][kFT / 16];
+        if constexpr (kStore) {  // relu; NaN is not positive
+          u32x4 p;
 #pragma unroll
-      for (int tb = 0; tb < kTB; ++tb)
-#pragma unroll
-        for (int j = 0; j < kFT / 16; ++j) acc[tb][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const half8* wt = reinterpret_cast<const half8*>(ws[buf]) + lane;
-#pragma unroll
-      for (int kb = 0; kb < kKB; ++kb) {
-        half8 wh[kFT / 16], wl[kFT / 16];
-#pragma unroll
-        for (int j = 0; j < kFT / 16; ++j) {
-          wh[j] = wt[((kb * 2 + 0) * 4 + j) * 64];
-          wl[j] = wt[((kb * 2 + 1) * 4 + j) * 64];
+          for (int r = 0; r < 4; ++r) p[r] = __float_as_uint(v[r] > 0.f ? v[r] : 0.f);
+          __builtin_amdgcn_raw_buffer_store_b128(
+              p, ar, f < kF ? (unsigned)(((16 * tb + li) * kF + f) * (int)sizeof(float)) : ~0u, 0, 0);
         }
-        // eight accumulators interleaved: no MFMA waits on the one before it
+        if constexpr (kCollect) {
 #pragma unroll
-        for (int tb = 0; tb < kTB; ++tb)
-#pragma unroll
-          for (int j = 0; j < kFT / 16; ++j)
-            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
-#pragma unroll
-        for (int tb = 0; tb < kTB; ++tb)
-#pragma unroll
-          for (int j = 0; j < kFT / 16; ++j)
-            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xl[tb][kb], acc[tb][j], 0, 0, 0);
-#pragma unroll
-        for (int tb = 0; tb < kTB; ++tb)
-#pragma unroll
-          for (int j = 0; j < kFT / 16; ++j)
-            acc[tb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], xh[tb][kb], acc[tb][j], 0, 0, 0);
-      }
-      // bias, relu, histogram of the positive values, store
-      if (!bad_rows && !__any(bad_w)) {
-#pragma unroll
-        for (int tb = 0; tb < kTB; ++tb) {
-          const int tok = t0 + 16 * tb + li;
-#pragma unroll
-          for (int j = 0; j < kFT / 16; ++j) {
-            const int f = f0 + 16 * j + 4 * lq;
-            const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
-            const float s4[4] = {winv[j].x, winv[j].y, winv[j].z, winv[j].w};
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              // the scales are powers of two: one rounding, that of the sum with the bias
-              const float s = fmaf(acc[tb][j][r] * xinv[tb], s4[r], b4[r]);
-              v[r] = s > 0.f ? s : 0.f;  // relu; non-positive values are never selected
-            }
-            if (tok < a.N && f < kF) {
-              *reinterpret_cast<float4*>(&ag[(size_t)tok * kF + f]) = make_float4(v[0], v[1], v[2], v[3]);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) take(v[r]);
-            }
-          }
+          for (int r = 0; r < 4; ++r) gather(v[r] >= least[tb], (unsigned)tok[tb] * kF + (unsigned)(f + r), v[r]);
+          flush();
         }
-      } else {
-#pragma unroll 1
-        for (int e = 0; e < kTB * kFT / 4; ++e) {
-          const int tok = t0 + 16 * (e >> 4) + li, f = f0 + 16 * ((e >> 2) & 3) + 4 * lq + (e & 3);
-          if (tok < a.N && f < kF) {
-            const float s = exact_value<KT>(a, g, tok, f), v = s > 0.f ? s : 0.f;
-            ag[(size_t)tok * kF + f] = v;
-            take(v);
-          }
+      }, [&](int tb, int j, int r, float v) {
+        const int f = f0 + 16 * j + 4 * lq + r, t = tb ? tok[1] : tok[0];
+        const bool in = t0 + 16 * tb + li < a.N && f < kF;
+        if constexpr (kStore)
+          if (in) a.act[((size_t)g * a.N + t) * kF + f] = v > 0.f ? v : 0.f;
+        if constexpr (kCollect) {
+          gather(v >= (tb ? least[1] : least[0]), (unsigned)t * kF + (unsigned)f, v);
+          flush();
         }
-      }
+      });
     }
     if (more) {  // the other buffer was last read before the previous barrier
       store_w(buf ^ 1, wr);
@@ -407,10 +684,20 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       buf ^= 1;
     }
   }
-  __syncthreads();
-  unsigned* hg = hist_of(a, g, 0) + ((part + y) % kRep) * kBins;
-  for (int i = tid; i < kBins; i += kET)
-    if (hist[i]) atomicAdd(&hg[i], hist[i]);
+  if constexpr (kCollect) {  // the rest of the 8 waves, one reservation
+    __syncthreads();
+    if (lane == 0) wsum[w] = n;
+    __syncthreads();
+    if (tid == 0) {
+      unsigned total = 0u;
+      for (int i = 0; i < kET / 64; ++i) total += wsum[i];
+      base_s = total ? atomicAdd(&ctl[kListLen], total) : 0u;
+    }
+    __syncthreads();
+    unsigned at = base_s;
+    for (int i = 0; i < w; ++i) at += wsum[i];
+    for (unsigned i = lane; i < n; i += 64) put(at, i);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -440,8 +727,9 @@ __global__ __launch_bounds__(kUT) void digit_kernel(UpdateArgs a, int level) {
     c[u] = s;
     tot += s;
   }
-  const long long total_vals = (long long)a.N * kF;
-  const unsigned count = (unsigned)(a.budget < total_vals ? a.budget : total_vals);
+  if (level == 0 && a.listed)
+    for (int i = tid; i < kSampleBins; i += kUT) a.sample[(size_t)g * kSampleBins + i] = 0u;
+  const unsigned count = budget_of(a);
   const unsigned incl = block_incl_scan<kUT>(tot, wsum);
   unsigned rem, prefix_in;
   if (level == 0) {
@@ -458,8 +746,8 @@ __global__ __launch_bounds__(kUT) void digit_kernel(UpdateArgs a, int level) {
         ctl[kNeed] = 0;
         ctl[kTies] = 0;
         ctl[kOrdered] = 0;
+        ctl[kCut] = 0;
         ctl[kCount] = count;
-        ctl[kListed] = 0;
       }
       return;
     }
@@ -485,13 +773,6 @@ __global__ __launch_bounds__(kUT) void digit_kernel(UpdateArgs a, int level) {
   __syncthreads();
   if (tid == 0) {
     const unsigned prefix = (prefix_in << width) | found_digit;
-    if (level == 0) {
-      // every value the selection can take lies in the first digit's bin or
-      // above it: (count - found_rem) above, found_ties in it.  If they fit,
-      // the first refine pass collects them and the later passes read only them.
-      ctl[kListed] = (unsigned long long)(count - found_rem) + found_ties + kListSlack <= (unsigned long long)a.list_cap;
-      ctl[kListLen] = 0;
-    }
     ctl[kMode] = kModeTopK;
     ctl[kPrefix] = prefix;
     ctl[kRem] = found_rem;
@@ -502,120 +783,230 @@ __global__ __launch_bounds__(kUT) void digit_kernel(UpdateArgs a, int level) {
       ctl[kNeed] = found_rem;
       ctl[kTies] = found_ties;
       ctl[kOrdered] = found_ties > found_rem;
+      ctl[kCut] = ~0u;  // every tie is taken, unless the tie kernels find the last one
+      ctl[kTieLen] = 0u;
     } else {
       ctl[kTau] = 0;
     }
   }
 }
 
-// ---------------------------------------------------------------------------
-// refine: grid (kRefineBlocks, G) x 256; histogram of the next digit of the
-// positive values whose higher bits equal the prefix.  Level 1 reads a and,
-// when the digit kernel found that they fit (ctl kListed), also collects every
-// positive value whose first digit is at or above tau's into the group's
-// compact list: a workgroup gathers its own in LDS (slots by LDS atomics) and
-// reserves its range of the list with one global atomic at its end; once the
-// LDS buffer is full, each wave writes into chunks of kListChunk entries of
-// the list that it reserves one at a time and zero-fills the unused tail of
-// its last one (an index build's candidates, about 8 per key, overflow every
-// buffer).  Level 2 and the emit then read only the list, skipping zero
-// entries.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kUT) void refine_kernel(UpdateArgs a, int level) {
-  const int g = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
-  unsigned* ctl = a.ctl + (size_t)g * kCtl;
-  if (ctl[kMode] != kModeTopK || ctl[kTau] == 0x7f800000u) return;
-  constexpr int kBuf = 1024;  // LDS list entries per workgroup
-  __shared__ unsigned hist[kBins];
-  __shared__ uint2 buf[kBuf];
-  __shared__ unsigned nbuf, first_miss, base_s;
-  for (int i = tid; i < kBins; i += kUT) hist[i] = 0;
-  if (tid == 0) {
-    nbuf = 0u;
-    first_miss = kBuf;
-  }
-  __syncthreads();
-  const unsigned prefix = ctl[kPrefix];
-  const bool listed = ctl[kListed] != 0u;
-  const int shift_hi = level == 1 ? 20 : 9;  // bits above this level's digit
-  const int shift = level == 1 ? 9 : 0;
-  const unsigned dmask = level == 1 ? 0x7ffu : 0x1ffu;
-  uint2* list = a.list + (size_t)g * a.list_cap;
-  if (level == 2 && listed) {
-    const unsigned len = min(ctl[kListLen], a.list_cap);
-    for (unsigned i = blockIdx.x * kUT + tid; i < len; i += gridDim.x * kUT) {
-      const unsigned u = list[i].y;
-      if (u != 0u && (u >> shift_hi) == prefix) atomicAdd(&hist[(u >> shift) & dmask], 1u);
+// The values a pass over a group reads: its candidate list (listed), or the
+// dense activations.  fn(value bits, flat index) is called for each, by NT
+// threads of `blocks` workgroups, kU loads in flight per thread.
+template <int NT, typename Fn>
+__device__ __forceinline__ void each_value(const UpdateArgs& a, int g, bool listed, int block, int blocks, Fn fn) {
+  constexpr int kU = 8;
+  if (listed) {
+    const uint2* list = a.list + (size_t)g * a.list_cap;
+    const unsigned len = a.ctl[(size_t)g * kCtl + kListLen], step = (unsigned)(NT * blocks);
+    for (unsigned i0 = (unsigned)(block * NT) + threadIdx.x; i0 < len; i0 += kU * step) {
+      uint2 e[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) e[u] = list[i0 + u * step < len ? i0 + u * step : i0];
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (i0 + u * step < len) fn(e[u].y, e[u].x);
     }
   } else {
-    const size_t n = (size_t)a.N * kF;
-    const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
-    const bool collect = level == 1 && listed;
-    // this wave's chunk of the list, once the workgroup's buffer is full:
-    // entries [c_at, c_at + c_n) are filled (c_n = kListChunk: none to fill)
-    unsigned c_at = 0u, c_n = (unsigned)kListChunk;
-    for (size_t i = (size_t)blockIdx.x * kUT + tid; i < (n / 4 + kUT - 1) / kUT * kUT;
-         i += (size_t)gridDim.x * kUT) {  // every lane of a wave iterates alike (the list's ballot)
-      const bool in = i < n / 4;
-      const float4 v4 = in ? ag[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+    const size_t n4 = (size_t)a.N * kF / 4, step = (size_t)NT * blocks;
+    const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * a.N * kF);
+    for (size_t i = (size_t)block * NT + threadIdx.x; i < n4; i += step) {
+      const float4 v = ag[i];
+      const float vv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const unsigned u = __float_as_uint(vv[j]);
-        if (vv[j] > 0.f && (u >> shift_hi) == prefix) atomicAdd(&hist[(u >> shift) & dmask], 1u);
-        if (collect) {
-          const bool take = vv[j] > 0.f && (u >> 20) >= prefix;
-          const unsigned long long m = __ballot(take);
-          if (m) {  // uniform
-            const unsigned cnt = (unsigned)__popcll(m), rank = (unsigned)__popcll(m & ((1ull << lane) - 1ull));
-            unsigned at = 0u;
-            if (lane == 0) at = atomicAdd(&nbuf, cnt);
-            at = __shfl(at, 0);
-            if (at + cnt <= (unsigned)kBuf) {  // uniform
-              if (take) buf[at + rank] = make_uint2((unsigned)(4 * i + j), u);
-            } else {
-              // the buffer is full: into the wave's chunk of the list, a new
-              // chunk reserved (one global atomic per kListChunk entries) for
-              // what does not fit.  Reservations come in increasing order, so
-              // every one that fitted the buffer lies below the first that did
-              // not, and the buffer's valid entries are those below it.
-              if (lane == 0) atomicMin(&first_miss, at);
-              const unsigned room = (unsigned)kListChunk - c_n;  // uniform
-              unsigned nat = 0u;
-              if (cnt > room) {  // uniform
-                if (lane == 0) nat = atomicAdd(&ctl[kListLen], (unsigned)kListChunk);
-                nat = __shfl(nat, 0);
-              }
-              if (take) {
-                const unsigned dst = rank < room ? c_at + c_n + rank : nat + (rank - room);
-                if (dst < a.list_cap) list[dst] = make_uint2((unsigned)(4 * i + j), u);
-              }
-              if (cnt > room) {
-                c_at = nat;
-                c_n = cnt - room;
-              } else {
-                c_n += cnt;
-              }
-            }
-          }
-        }
-      }
+      for (int j = 0; j < 4; ++j)
+        if (vv[j] > 0.f) fn(__float_as_uint(vv[j]), (unsigned)(4 * i + j));
     }
-    // the unfilled tail of the wave's chunk reads as no entry (value bits 0)
-    for (unsigned e = c_n + lane; e < (unsigned)kListChunk; e += 64)
-      if (c_at + e < a.list_cap) list[c_at + e] = make_uint2(0u, 0u);
   }
+}
+
+// ---------------------------------------------------------------------------
+// hist0 / refine: grid (kRefineBlocks, G) x 256; histogram of the first digit
+// of the positive values, and of the next digit of those whose higher bits
+// equal the prefix.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void level_hist(const UpdateArgs& a, int level, int shift_hi, unsigned prefix, int shift,
+                                           unsigned dmask) {
+  const int g = blockIdx.y, tid = threadIdx.x;
+  __shared__ unsigned hist[kBins];
+  for (int i = tid; i < kBins; i += kUT) hist[i] = 0;
+  __syncthreads();
+  each_value<kUT>(a, g, list_ok(a, g), blockIdx.x, gridDim.x, [&](unsigned u, unsigned) {
+    if ((u >> shift_hi) == prefix) atomicAdd(&hist[(u >> shift) & dmask], 1u);
+  });
   __syncthreads();
   unsigned* hg = hist_of(a, g, level) + (blockIdx.x % kRep) * kBins;
   for (int i = tid; i < kBins; i += kUT)
     if (hist[i]) atomicAdd(&hg[i], hist[i]);
-  // the workgroup's buffered candidates
-  const unsigned nb = min(nbuf, first_miss);
-  if (nb == 0u) return;  // uniform
-  if (tid == 0) base_s = atomicAdd(&ctl[kListLen], nb);
+}
+
+__global__ __launch_bounds__(kUT) void hist0_kernel(UpdateArgs a) { level_hist(a, 0, 31, 0u, 20, 0x7ffu); }
+
+__global__ __launch_bounds__(kUT) void refine_kernel(UpdateArgs a, int level) {
+  const unsigned* ctl = a.ctl + (size_t)blockIdx.y * kCtl;
+  if (ctl[kMode] != kModeTopK || ctl[kTau] == 0x7f800000u) return;
+  level_hist(a, level, level == 1 ? 20 : 9, ctl[kPrefix], level == 1 ? 9 : 0, level == 1 ? 0x7ffu : 0x1ffu);
+}
+
+// One level of a radix search in LDS: the digit of the rem-th largest key among
+// the `bins` counted ones; rem becomes its rank inside the digit's bin, whose
+// count is returned in `ties`.  NT threads; the result is uniform.
+struct Found {
+  unsigned digit, rem, ties;
+};
+template <int NT>
+__device__ __forceinline__ Found find_digit(const unsigned* hist, int bins, unsigned rem, unsigned* wsum, Found* out) {
+  const int tid = threadIdx.x, per = (bins + NT - 1) / NT;
+  unsigned tot = 0u;
+  for (int u = 0; u < per; ++u) {
+    const int d = bins - 1 - (tid * per + u);
+    tot += d >= 0 ? hist[d] : 0u;
+  }
+  unsigned run = block_incl_scan<NT>(tot, wsum) - tot;
+  if (run < rem && run + tot >= rem)
+    for (int u = 0; u < per; ++u) {
+      const int d = bins - 1 - (tid * per + u);
+      const unsigned c = d >= 0 ? hist[d] : 0u;
+      if (run < rem && run + c >= rem) *out = Found{(unsigned)d, rem - run, c};
+      run += c;
+    }
   __syncthreads();
-  for (unsigned i = tid; i < nb; i += kUT)
-    if (base_s + i < a.list_cap) list[base_s + i] = buf[i];
+  const Found f = *out;
+  __syncthreads();
+  return f;
+}
+
+// ---------------------------------------------------------------------------
+// select: grid G x 1024, calls of up to kSelectMax keys: tau and the cut of its
+// ties in one launch, where the levels of hist0 / digit / refine and the tie
+// kernels are nine of about 4.5 us each.  One pass over the list counts 13-bit
+// digits, a second gathers tau's bin (3% of tau wide: about a fifth of the
+// budget) in LDS, where the other 18 bits and the flat indices of the ties are
+// searched: 13.5 us at 1024 keys, 30 at 4096 (16384 keys took 127: there the
+// levels' own launches, over 256 workgroups per group, are the better ones).
+// A bin that does not fit (ties by the thousand), or a list that
+// cannot be used, is searched by passes over the list or the activations.
+// ---------------------------------------------------------------------------
+constexpr int kST = 1024;
+constexpr int kSelBuf = 8192;
+
+__global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
+  const int g = blockIdx.x, tid = threadIdx.x;
+  __shared__ unsigned hist[kSampleBins];
+  __shared__ uint2 bin[kSelBuf];
+  __shared__ unsigned wsum[kST / 64], nbin;
+  __shared__ Found found;
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  const bool listed = list_ok(a, g);
+  const unsigned count = budget_of(a);
+  for (int i = tid; i < kSampleBins; i += kST) a.sample[(size_t)g * kSampleBins + i] = 0u;  // for the next call
+  if (tid == 0) nbin = 0u;
+  // The listed values lie within a few octaves above the floor, 32 digits each,
+  // so they are counted in kRel digits from the floor's on, 8 replicas of each
+  // (64 lanes meet in some 25 digits: one replica took 15 us of atomics for the
+  // list of 4096 keys); a value beyond them, or an unlisted call, in all 8192.
+  constexpr unsigned kRel = kSampleBins / 8;
+  Found f;
+  unsigned npos = 0u;
+  for (bool rel = listed;; rel = false) {  // uniform
+    const unsigned base = rel ? ctl[kFloor] >> kSampleShift : 0u;
+    __syncthreads();
+    for (int i = tid; i < kSampleBins; i += kST) hist[i] = 0u;
+    __syncthreads();
+    each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned) {
+      const unsigned d = (u >> kSampleShift) - base;
+      atomicAdd(&hist[rel ? 8u * min(d, kRel - 1u) + (tid & 7) : d], 1u);
+    });
+    __syncthreads();
+    if (rel) {
+      unsigned c = 0u;
+      if (tid < (int)kRel)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) c += hist[8 * tid + r];
+      __syncthreads();
+      if (tid < (int)kRel) hist[tid] = c;
+      __syncthreads();
+    }
+    const int bins = rel ? (int)kRel : kSampleBins;
+    npos = 0u;
+    for (int i = tid; i < bins; i += kST) npos += hist[i];
+    block_incl_scan<kST>(npos, wsum);
+    npos = 0u;
+    for (int i = 0; i < kST / 64; ++i) npos += wsum[i];
+    __syncthreads();
+    if (npos < count) {  // fewer positives than the budget: every one is kept (core.py:22-26)
+      if (tid == 0) {
+        ctl[kTau] = 0u;
+        ctl[kCut] = 0u;
+      }
+      return;
+    }
+    f = find_digit<kST>(hist, bins, count, wsum, &found);
+    if (!rel) break;
+    if (f.digit < kRel - 1u) {
+      f.digit += base;
+      break;
+    }
+  }
+  const unsigned top = f.digit;
+  const bool gathered = f.ties <= (unsigned)kSelBuf;
+  if (gathered) {
+    each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
+      if ((u >> kSampleShift) == top) bin[atomicAdd(&nbin, 1u)] = make_uint2(flat, u);
+    });
+    __syncthreads();
+  }
+  // counts the digit (key >> shift) & mask of the values of tau's bin for which in(u, flat)
+  auto count_digits = [&](int bins, auto in, auto digit) {
+    for (int i = tid; i < bins; i += kST) hist[i] = 0u;
+    __syncthreads();
+    if (gathered) {
+      for (unsigned i = tid; i < nbin; i += kST)
+        if (in(bin[i].y)) atomicAdd(&hist[digit(bin[i].y, bin[i].x)], 1u);
+    } else {
+      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
+        if (in(u)) atomicAdd(&hist[digit(u, flat)], 1u);
+      });
+    }
+    __syncthreads();
+  };
+  unsigned prefix = top;
+  for (int shift = 9; shift >= 0; shift -= 9) {
+    count_digits(512, [&](unsigned u) { return (u >> (shift + 9)) == prefix; },
+                 [&](unsigned u, unsigned) { return (u >> shift) & 511u; });
+    f = find_digit<kST>(hist, 512, f.rem, wsum, &found);
+    prefix = (prefix << 9) | f.digit;
+  }
+  unsigned cut = ~0u;
+  if (f.ties > f.rem) {  // the rem-th smallest flat index of the ties = the rem-th largest complement
+    unsigned key = 0u;
+    const int width[3] = {11, 11, 10};
+    int shift = 32;
+    for (int l = 0; l < 3; ++l) {
+      shift -= width[l];
+      const unsigned mask = (1u << width[l]) - 1u;
+      const int hi = shift + width[l];
+      for (int i = tid; i < (1 << width[l]); i += kST) hist[i] = 0u;
+      __syncthreads();
+      auto tie = [&](unsigned u, unsigned flat) {
+        const unsigned c = ~flat;
+        if (u == prefix && (hi == 32 || (c >> hi) == key)) atomicAdd(&hist[(c >> shift) & mask], 1u);
+      };
+      if (gathered)
+        for (unsigned i = tid; i < nbin; i += kST) tie(bin[i].y, bin[i].x);
+      else
+        each_value<kST>(a, g, listed, 0, 1, tie);
+      __syncthreads();
+      f = find_digit<kST>(hist, 1 << width[l], f.rem, wsum, &found);
+      key = (key << width[l]) | f.digit;
+    }
+    cut = ~key;
+  }
+  if (tid == 0) {
+    ctl[kTau] = prefix;
+    ctl[kCut] = cut;
+  }
 }
 
 __device__ __forceinline__ void set_member(const UpdateArgs& a, int g, unsigned flat) {
@@ -625,46 +1016,25 @@ __device__ __forceinline__ void set_member(const UpdateArgs& a, int g, unsigned 
 }
 
 // ---------------------------------------------------------------------------
-// emit: grid (kRefineBlocks, G) x 256 over a.
+// emit: grid (blocks, G) x 256: the bit of every value above tau and of the ties
+// up to the cut.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kUT) void emit_kernel(UpdateArgs a) {
-  const int g = blockIdx.y, tid = threadIdx.x;
+  const int g = blockIdx.y;
   const unsigned* ctl = a.ctl + (size_t)g * kCtl;
-  const unsigned mode = ctl[kMode];
-  const float tau = __uint_as_float(ctl[kTau]);
-  const bool take_ties = mode == kModeTopK && !ctl[kOrdered] && tau > 0.f;
-  if (mode == kModeTopK && ctl[kListed]) {  // every candidate is in the compact list
-    const uint2* list = a.list + (size_t)g * a.list_cap;
-    const unsigned len = min(ctl[kListLen], a.list_cap);
-    for (unsigned i = blockIdx.x * kUT + tid; i < len; i += gridDim.x * kUT) {
-      const uint2 e = list[i];
-      const float v = __uint_as_float(e.y);
-      if (e.y != 0u && (v > tau || (take_ties && v == tau))) set_member(a, g, e.x);
-    }
-    return;
-  }
-  const size_t n = (size_t)a.N * kF;
-  const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
-  for (size_t i = (size_t)blockIdx.x * kUT + tid; i < n / 4; i += (size_t)gridDim.x * kUT) {
-    const float4 v4 = ag[i];
-    const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float v = vv[j];
-      const bool sel = mode == kModeAllPositive ? v > 0.f : ((v > tau && v > 0.f) || (take_ties && v == tau));
-      if (sel) set_member(a, g, (unsigned)(4 * i + j));
-    }
-  }
+  const unsigned tau = ctl[kTau], cut = ctl[kCut];
+  each_value<kUT>(a, g, list_ok(a, g), blockIdx.x, gridDim.x, [&](unsigned u, unsigned flat) {
+    if (u > tau || (u == tau && flat <= cut)) set_member(a, g, flat);
+  });
 }
 
 // ---------------------------------------------------------------------------
-// ties, only when the ties at tau overflow the budget: the first `need` of
-// them in ascending flat index (core.py:23-24).  The activations of a group
-// are cut into tie_blocks contiguous ranges [r L, (r + 1) L), dealt to the
-// workgroups r = x, x + kTieGrid, ...  tie_count_kernel counts each range's
-// ties; tie_take_kernel skips the ties of the lower ranges and takes the
-// range's own in flat order (4 consecutive values per thread) while the
-// budget lasts.  Grid (min(tie_blocks, kTieGrid), G) x 256 each.
+// ties, only when the ties at tau overflow the budget: the flat index of the
+// last of the first `need` in ascending flat index (core.py:23-24).
+// tie_count_kernel, grid (blocks, G) x 256: gathers the ties' flat indices from
+// the list, or counts the ties of each contiguous range [r L, (r + 1) L) of the
+// dense activations.  tie_cut_kernel, grid G x 1024: a radix search over the
+// gathered indices, or the range that holds the need-th tie and a scan of it.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bool ordered_ties(const UpdateArgs& a, int g) {
   const unsigned* ctl = a.ctl + (size_t)g * kCtl;
@@ -675,7 +1045,16 @@ __global__ __launch_bounds__(kUT) void tie_count_kernel(UpdateArgs a) {
   const int g = blockIdx.y, tid = threadIdx.x;
   if (!ordered_ties(a, g)) return;
   __shared__ unsigned wsum[kUT / 64];
-  const float tau = __uint_as_float(a.ctl[(size_t)g * kCtl + kTau]);
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  if (list_ok(a, g)) {
+    const unsigned tau = ctl[kTau];
+    unsigned* ties = a.ties + (size_t)g * a.list_cap;
+    each_value<kUT>(a, g, true, blockIdx.x, gridDim.x, [&](unsigned u, unsigned flat) {
+      if (u == tau) ties[atomicAdd(&ctl[kTieLen], 1u)] = flat;
+    });
+    return;
+  }
+  const float tau = __uint_as_float(ctl[kTau]);
   const size_t n = (size_t)a.N * kF;
   const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
   for (int r = blockIdx.x; r < a.tie_blocks; r += gridDim.x) {  // uniform
@@ -701,179 +1080,236 @@ __global__ __launch_bounds__(kUT) void tie_count_kernel(UpdateArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kUT) void tie_take_kernel(UpdateArgs a) {
-  const int g = blockIdx.y, tid = threadIdx.x;
+__global__ __launch_bounds__(kST) void tie_cut_kernel(UpdateArgs a) {
+  const int g = blockIdx.x, tid = threadIdx.x;
   if (!ordered_ties(a, g)) return;
-  __shared__ unsigned wsum[kUT / 64];
-  const unsigned* ctl = a.ctl + (size_t)g * kCtl;
-  const float tau = __uint_as_float(ctl[kTau]);  // > 0: only positive values reach the histogram
-  const unsigned need = ctl[kNeed];
-  const size_t n = (size_t)a.N * kF;
-  const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
-  for (int r = blockIdx.x; r < a.tie_blocks; r += gridDim.x) {  // uniform
-    unsigned below = 0;
-    for (int j = tid; j < r; j += kUT) below += a.tcount[(size_t)g * a.tie_blocks + j];
-    block_incl_scan<kUT>(below, wsum);
-    unsigned taken = wsum[0] + wsum[1] + wsum[2] + wsum[3];  // ties of the lower ranges, all ranked first
-    __syncthreads();  // every thread has read wsum before the next scan rewrites it
-    const size_t lo = min(n, (size_t)r * a.tie_len), hi = min(n, lo + a.tie_len);
-    for (size_t base = lo / 4; base < hi / 4 && taken < need; base += kUT) {  // uniform condition
-      const size_t i = base + tid;
-      const float4 v = i < hi / 4 ? ag[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const bool h[4] = {v.x == tau, v.y == tau, v.z == tau, v.w == tau};
-      const unsigned c = (unsigned)h[0] + (unsigned)h[1] + (unsigned)h[2] + (unsigned)h[3];
-      const unsigned incl = block_incl_scan<kUT>(c, wsum);
-      unsigned rank = taken + incl - c;  // rank of this thread's first tie among all ties
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (h[j]) {
-          if (rank < need) set_member(a, g, (unsigned)(4 * i + j));
-          ++rank;
-        }
-      taken += wsum[0] + wsum[1] + wsum[2] + wsum[3];
-      __syncthreads();  // wsum is rewritten by the next scan
+  __shared__ unsigned hist[kBins], wsum[kST / 64], range_s, below_s;
+  __shared__ Found found;
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  const unsigned need = ctl[kNeed];  // >= 1
+  if (list_ok(a, g)) {
+    const unsigned* ties = a.ties + (size_t)g * a.list_cap;
+    const unsigned len = ctl[kTieLen];
+    unsigned key = 0u, rem = need;
+    const int width[3] = {11, 11, 10};
+    int shift = 32;
+    for (int l = 0; l < 3; ++l) {
+      shift -= width[l];
+      const unsigned mask = (1u << width[l]) - 1u;
+      const int hi = shift + width[l];
+      for (int i = tid; i < kBins; i += kST) hist[i] = 0u;
+      __syncthreads();
+      for (unsigned i = tid; i < len; i += kST) {
+        const unsigned c = ~ties[i];
+        if (hi == 32 || (c >> hi) == key) atomicAdd(&hist[(c >> shift) & mask], 1u);
+      }
+      __syncthreads();
+      const Found f = find_digit<kST>(hist, 1 << width[l], rem, wsum, &found);
+      key = (key << width[l]) | f.digit;
+      rem = f.rem;
     }
+    if (tid == 0) ctl[kCut] = ~key;
+    return;
+  }
+  const float tau = __uint_as_float(ctl[kTau]);
+  constexpr int kPer = kMaxTieBlocks / kST;
+  unsigned c[kPer], tot = 0u;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int r = tid * kPer + u;
+    c[u] = r < a.tie_blocks ? a.tcount[(size_t)g * a.tie_blocks + r] : 0u;
+    tot += c[u];
+  }
+  unsigned run = block_incl_scan<kST>(tot, wsum) - tot;
+  if (run < need && run + tot >= need)
+    for (int u = 0; u < kPer; ++u) {
+      if (run < need && run + c[u] >= need) {
+        range_s = (unsigned)(tid * kPer + u);
+        below_s = run;
+      }
+      run += c[u];
+    }
+  __syncthreads();
+  const size_t n = (size_t)a.N * kF;
+  const size_t lo = min(n, (size_t)range_s * a.tie_len), hi = min(n, lo + a.tie_len);
+  const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
+  unsigned taken = below_s;
+  for (size_t base = lo / 4; base < hi / 4 && taken < need; base += kST) {  // uniform condition
+    const size_t i = base + tid;
+    const float4 v = i < hi / 4 ? ag[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool h[4] = {v.x == tau, v.y == tau, v.z == tau, v.w == tau};
+    const unsigned k = (unsigned)h[0] + (unsigned)h[1] + (unsigned)h[2] + (unsigned)h[3];
+    const unsigned incl = block_incl_scan<kST>(k, wsum);
+    unsigned rank = taken + incl - k;  // rank of this thread's first tie among all ties
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (h[j] && ++rank == need) ctl[kCut] = (unsigned)(4 * i + j);
+    for (int j = 0; j < kST / 64; ++j) taken += wsum[j];
+    __syncthreads();  // wsum is rewritten by the next scan
   }
 }
 
 // ---------------------------------------------------------------------------
-// moments: grid (kChunks, G) x 256.  Wave w handles buckets 32c + 8w + j:
+// moments: grid (kChunks, G) x 512.  Wave w handles buckets 32c + 4w + j:
 // members from the bitmap, two-pass moments of their keys; then the tile
 // merge, thread = (dim k, bucket col) pairs of mean row k and var row 128+k.
+// Bound by memory round trips, by the 49 MB of moments read and rewritten (8
+// groups) and by the fetching of its own instructions, so the buckets are a
+// loop that 24 waves per CU run side by side, not one unrolled over a wave's
+// buckets (171 registers, 35 us at 1024 keys).  Lane l owns dims 2l, 2l + 1
+// of every member, so no sum crosses lanes, and the first 8 members of a
+// bucket (at a budget of 8 per key, 3 at 1024 keys and 11 at 4096 on average)
+// are requested together and kept for the second pass; the tile's old moments
+// are requested before the first of them.  15.9 us at 1024 keys, 40 at 4096
+// (16 members kept: 22 and 46, registers spilled at 6 waves per SIMD).
 // ---------------------------------------------------------------------------
-constexpr int kMaxBlock = 4096;  // new tokens per update (LDS member list per wave)
-constexpr int kMomBatch = 16;    // member key words requested at once
+constexpr int kMaxBlock = 4096;  // new tokens per update
+constexpr int kMT = 512;
+constexpr int kMomSlot = 512;    // members listed at once: 16 bitmap words hold no more
+constexpr int kMomRound = 8;     // member key words requested at once
+constexpr int kMomCols = kChunk / (kMT / 64);  // buckets per wave (4)
 
-__device__ __forceinline__ float merge_mean(float a, float b, float den, float ma, float mb) {
+// The update's merge (core.py:194-199) for bucket sizes a (old) and b (block),
+// den = max(a + b, 1): every rounding of (a x + b y) / den + ..., with the
+// quotients by divide_by.
+__device__ __forceinline__ float merge_mean(float a, float b, float den, float rden, float ma, float mb) {
 #pragma clang fp contract(off)
-  return (a * ma + b * mb) / den;
+  return divide_by(a * ma + b * mb, den, rden);
 }
-__device__ __forceinline__ float merge_var(float a, float b, float den, float ma, float mb, float va, float vb) {
+__device__ __forceinline__ float merge_var(float a, float b, float den, float rden, float ab, float ma, float mb, float va,
+                                           float vb) {
 #pragma clang fp contract(off)
-  const float v = (a * va + b * vb) / den;
+  const float v = divide_by(a * va + b * vb, den, rden);
   const float d = ma - mb;
-  return v + ((a * b) / (den * den)) * (d * d);
+  return v + ab * (d * d);
 }
 
 template <typename KT>
-__global__ __launch_bounds__(kUT) void moments_kernel(UpdateArgs a) {
+__global__ __launch_bounds__(kMT, 6) void moments_kernel(UpdateArgs a) {
   const int c = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  __shared__ float nm[kChunk][kD], nv[kChunk][kD];
+  __shared__ float nm[kChunk][kD + 1], nv[kChunk][kD + 1];
   __shared__ int nb[kChunk];
-  // the wave's member list, in dynamic LDS sized by the block (N tokens per
-  // wave at most), so that several workgroups share a CU
-  extern __shared__ int toks_all[];
-  int* toks = toks_all + (size_t)w * a.N;
-  const int w_lo = a.H >> 5, w_hi = (a.H + a.N - 1) >> 5;
+  __shared__ uint16_t toks_all[kMT / 64][kMomSlot];  // tokens of the block, from its first word's on
+  uint16_t* toks = toks_all[w];
   typedef KeyLoad<KT> KL;
-  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks;
-  // the first 64 bitmap words of the wave's 8 buckets, all requested at once
-  // (the whole block's words up to 2016 tokens)
-  constexpr int kCols = kChunk / 4;
-  uint32_t first[kCols];
-#pragma unroll
-  for (int j = 0; j < kCols; ++j) {
-    const int f = c * kChunk + w * kCols + j;
-    const int wd = w_lo + lane;
-    first[j] = f < kF && wd <= w_hi ? a.bits[((size_t)g * kF + f) * a.row_words + wd] : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < kCols; ++j) {
-    const int col = w * kCols + j, f = c * kChunk + col;
-    int b = 0;
-    if (f < kF) {
-      const uint32_t* row = a.bits + ((size_t)g * kF + f) * a.row_words;
-      for (int w0 = w_lo; w0 <= w_hi; w0 += 64) {
-        const int wd = w0 + lane;
-        uint32_t m = w0 == w_lo ? first[j] : (wd <= w_hi ? row[wd] : 0u);
-        if (wd == w_lo) m &= ~0u << (a.H & 31);                               // tokens before H
-        if (wd == w_hi && ((a.H + a.N) & 31)) m &= (1u << ((a.H + a.N) & 31)) - 1u;  // tokens past H+N
-        const int pc = __popc(m);
-        const int incl = (int)wave_incl_scan((unsigned)pc);
-        int at = b + incl - pc;
-        while (m) {
-          toks[at++] = wd * 32 + (int)__builtin_ctz(m);
-          m &= m - 1u;
-        }
-        b += __shfl(incl, 63);
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_s_waitcnt(0);
-    // two-pass moments of the ORIGINAL keys (core.py:84-88); lane owns dims
-    // 2l, 2l+1.  Members are summed in ascending order; their key words are
-    // requested kMomBatch at a time, and a bucket of at most kMomBatch members
-    // keeps them in registers for the second pass.
-    auto key_word = [&](int i) { return KL::load2(kg + (size_t)toks[i] * kD + 2 * lane); };
-    float s0 = 0.f, s1 = 0.f;
-    typename KL::Raw2 kept[kMomBatch];
-    for (int i0 = 0; i0 < b; i0 += kMomBatch) {  // uniform
-      typename KL::Raw2 r[kMomBatch];
-#pragma unroll
-      for (int u = 0; u < kMomBatch; ++u) r[u] = key_word(min(i0 + u, b - 1));  // unconditional: one round trip
-#pragma unroll
-      for (int u = 0; u < kMomBatch; ++u) {
-        if (i0 + u < b) {
-          s0 += KL::lo(r[u]);
-          s1 += KL::hi(r[u]);
-        }
-        kept[u] = r[u];
-      }
-    }
-    const float m0 = b ? s0 / (float)b : 0.f, m1 = b ? s1 / (float)b : 0.f;
-    float q0 = 0.f, q1 = 0.f;
-    if (b <= kMomBatch) {
-#pragma unroll
-      for (int u = 0; u < kMomBatch; ++u)
-        if (u < b) {
-          const float d0 = KL::lo(kept[u]) - m0, d1 = KL::hi(kept[u]) - m1;
-          q0 += d0 * d0;
-          q1 += d1 * d1;
-        }
-    } else {
-      for (int i0 = 0; i0 < b; i0 += kMomBatch) {
-        typename KL::Raw2 r[kMomBatch];
-#pragma unroll
-        for (int u = 0; u < kMomBatch; ++u) r[u] = key_word(min(i0 + u, b - 1));
-#pragma unroll
-        for (int u = 0; u < kMomBatch; ++u)
-          if (i0 + u < b) {
-            const float d0 = KL::lo(r[u]) - m0, d1 = KL::hi(r[u]) - m1;
-            q0 += d0 * d0;
-            q1 += d1 * d1;
-          }
-      }
-    }
-    nm[col][2 * lane] = m0;
-    nm[col][2 * lane + 1] = m1;
-    nv[col][2 * lane] = b ? q0 / (float)b : 0.f;
-    nv[col][2 * lane + 1] = b ? q1 / (float)b : 0.f;
-    if (lane == 0) nb[col] = b;
-    __builtin_amdgcn_wave_barrier();
-  }
-  __syncthreads();
+  const int w_lo = a.H >> 5, w_hi = (a.H + a.N - 1) >> 5;
+  // the block's key rows, from its first bitmap word's token on (32-bit offsets)
+  constexpr unsigned kRowBytes = kD * sizeof(KT);
+  const __amdgpu_buffer_rsrc_t kr =
+      raw_buffer(static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)w_lo * 32 * kD,
+                 (int)((unsigned)(a.H + a.N - 32 * w_lo) * kRowBytes));
+  const unsigned at_dims = 2u * lane * (unsigned)sizeof(KT);
+  const int f0 = c * kChunk + w * kMomCols;
+  const uint32_t* rows = a.bits + ((size_t)g * kF + f0) * a.row_words;
+  // Word wd of the wave's bucket j, tokens of the block only.
+  auto word = [&](int j, int wd) {
+    uint32_t m = f0 + j < kF && wd <= w_hi ? rows[(size_t)j * a.row_words + wd] : 0u;
+    if (wd == w_lo) m &= ~0u << (a.H & 31);                                      // tokens before H
+    if (wd == w_hi && ((a.H + a.N) & 31)) m &= (1u << ((a.H + a.N) & 31)) - 1u;  // tokens past H + N
+    return m;
+  };
+  uint32_t next = word(0, w_lo + lane);
   float* tile = a.moments + (size_t)(g * kChunks + c) * kRow * kChunk;
   const int col = tid & (kChunk - 1), f = c * kChunk + col;
-  if (f >= kF) return;  // padding columns stay zero
-  const int na = a.counts[(size_t)g * kFP + f], nbn = nb[col];
-  const float fa = (float)na, fb = (float)nbn;
-  const float total = fa + fb, den = total < 1.f ? 1.f : total;
-  // every old mean and variance of the thread's 16 dims is requested before
-  // the first merge, so the tile costs one memory round trip
-  constexpr int kRowsPerThread = kD / (kUT / kChunk);  // 16
+  constexpr int kRowsPerThread = kD / (kMT / kChunk);  // 8
   float ma[kRowsPerThread], va[kRowsPerThread];
 #pragma unroll
   for (int i = 0; i < kRowsPerThread; ++i) {
-    const int k = (tid >> 5) + (kUT / kChunk) * i;
+    const int k = (tid >> 5) + (kMT / kChunk) * i;
     ma[i] = tile[k * kChunk + col];
     va[i] = tile[(kD + k) * kChunk + col];
   }
+  const int na = a.counts[(size_t)g * kFP + f];
+#pragma unroll 1
+  for (int j = 0; j < kMomCols; ++j) {
+    const uint32_t head = next;  // the bucket's first 64 words: the whole block up to 2017 tokens
+    if (j + 1 < kMomCols) next = word(j + 1, w_lo + lane);
+    // members of words [w0, w0 + 64) in ascending order to toks[n ..], up to kMomSlot; n grows by their number
+    auto list_words = [&](uint32_t m, int w0, int n) {
+      const int incl = (int)wave_incl_scan((unsigned)__popc(m));
+      int at = n + incl - __popc(m);
+      __builtin_amdgcn_wave_barrier();
+      for (; m && at < kMomSlot; m &= m - 1u) toks[at++] = (uint16_t)((w0 + lane - w_lo) * 32 + (int)__builtin_ctz(m));
+      __builtin_amdgcn_wave_barrier();
+      return n + __builtin_amdgcn_readlane(incl, 63);
+    };
+    // two-pass moments of the ORIGINAL keys (core.py:84-88)
+    float m0 = 0.f, m1 = 0.f, v0 = 0.f, v1 = 0.f;
+    auto sum = [&](typename KL::Raw2 r) {
+      m0 += KL::lo(r);
+      m1 += KL::hi(r);
+    };
+    auto dev = [&](typename KL::Raw2 r) {
+      const float d0 = KL::lo(r) - m0, d1 = KL::hi(r) - m1;
+      v0 += d0 * d0;
+      v1 += d1 * d1;
+    };
+    auto pass = [&](int i0, int n, auto add) {
+      for (; i0 < n; i0 += kMomRound) {  // uniform
+        typename KL::Raw2 r[kMomRound];
+#pragma unroll
+        for (int u = 0; u < kMomRound; ++u) r[u] = KL::load2(kr, toks[min(i0 + u, n - 1)] * kRowBytes + at_dims);
+#pragma unroll
+        for (int u = 0; u < kMomRound; ++u)
+          if (i0 + u < n) add(r[u]);
+      }
+    };
+    int b = list_words(head, w_lo, 0);
+    for (int w0 = w_lo + 64; w0 <= w_hi; w0 += 64) b = list_words(word(j, w0 + lane), w0, b);
+    if (b <= kMomSlot) {  // uniform: the list is whole
+      if (b > 0) {
+        typename KL::Raw2 kept[kMomRound];
+#pragma unroll
+        for (int u = 0; u < kMomRound; ++u) kept[u] = KL::load2(kr, toks[min(u, b - 1)] * kRowBytes + at_dims);
+        const float n = (float)b, rn = 1.0f / n;
+#pragma unroll
+        for (int u = 0; u < kMomRound; ++u)
+          if (u < b) sum(kept[u]);
+        pass(kMomRound, b, sum);
+        m0 = divide_by(m0, n, rn);
+        m1 = divide_by(m1, n, rn);
+#pragma unroll
+        for (int u = 0; u < kMomRound; ++u)
+          if (u < b) dev(kept[u]);
+        pass(kMomRound, b, dev);
+        v0 = divide_by(v0, n, rn);
+        v1 = divide_by(v1, n, rn);
+      }
+    } else {  // 16 words (at most 512 members) at a time, once for each pass
+      b = 0;
+      for (int w0 = w_lo; w0 <= w_hi; w0 += 16) {
+        const int n = list_words(lane < 16 ? word(j, w0 + lane) : 0u, w0, 0);
+        pass(0, n, sum);
+        b += n;
+      }
+      if (b > 0) {
+        const float n = (float)b, rn = 1.0f / n;
+        m0 = divide_by(m0, n, rn);
+        m1 = divide_by(m1, n, rn);
+        for (int w0 = w_lo; w0 <= w_hi; w0 += 16) 
+          pass(0, list_words(lane < 16 ? word(j, w0 + lane) : 0u, w0, 0), dev);
+        v0 = divide_by(v0, n, rn);
+        v1 = divide_by(v1, n, rn);
+      }
+    }
+    const int o = w * kMomCols + j;
+    nm[o][2 * lane] = m0;
+    nm[o][2 * lane + 1] = m1;
+    nv[o][2 * lane] = v0;
+    nv[o][2 * lane + 1] = v1;
+    if (lane == 0) nb[o] = b;
+  }
+  __syncthreads();
+  if (f >= kF) return;  // padding columns stay zero
+  const int nbn = nb[col];
+  const float fa = (float)na, fb = (float)nbn;
+  const float total = fa + fb, den = total < 1.f ? 1.f : total, rden = 1.0f / den, ab = (fa * fb) / (den * den);
 #pragma unroll
   for (int i = 0; i < kRowsPerThread; ++i) {
-    const int k = (tid >> 5) + (kUT / kChunk) * i;
+    const int k = (tid >> 5) + (kMT / kChunk) * i;
     const float mb = nm[col][k], vb = nv[col][k];
-    tile[k * kChunk + col] = merge_mean(fa, fb, den, ma[i], mb);
-    tile[(kD + k) * kChunk + col] = merge_var(fa, fb, den, ma[i], mb, va[i], vb);
+    tile[k * kChunk + col] = merge_mean(fa, fb, den, rden, ma[i], mb);
+    tile[(kD + k) * kChunk + col] = merge_var(fa, fb, den, rden, ab, ma[i], mb, va[i], vb);
   }
   if (tid < kChunk) a.counts[(size_t)g * kFP + f] = na + nbn;
 }
@@ -934,133 +1370,162 @@ __global__ __launch_bounds__(kUT) void clear_bits_kernel(UpdateArgs a) {
 // ---------------------------------------------------------------------------
 // build_moments: grid (F, G) x 256, one workgroup per bucket f, any member
 // count.  Members are the set bits of the bucket's bitmap row below N (a
-// build indexes K rows = bitmap columns [0, N)).  Chunks of 256 words (one
-// per thread) are compacted into an LDS token list; while the whole list
-// fits in kList tokens it is kept and both passes read it, otherwise each
-// pass re-scans the row chunk by chunk.  Thread = (member slot tid >> 4 of
-// 16, dims 8 (tid & 15) ..): 16 key rows per step with 16-byte loads,
-// double accumulation, fixed order.  mean = sum / n rounded to fp32; var =
-// sum (x - mean)^2 / n with that rounded mean; empty bucket -> 0
-// (core.py:84-88).  Counts and moments are written, not merged.
+// build indexes K rows = bitmap columns [0, N)).  The row is compacted into an
+// LDS token list, 2048 words (64K keys) requested at once; a list of more than
+// kList tokens is rebuilt 64 words at a time in each pass.  Workgroup x takes
+// bucket 375 (x % 8) + x / 8: consecutive workgroups go to the 8 XCDs in turn,
+// so each XCD works through consecutive buckets and its L2 joins their 4-byte
+// columns of the moment tiles before they are written back.  Thread = (member slot tid >> 4 of 16, dims 8 (tid & 15)
+// ..), double accumulation, fixed order: the slots of a wave by shuffles, then
+// the 4 waves.  The first 192 members (a 64K build has 175 on average; 96 of
+// fp32) are requested together and kept packed in registers, so the second pass reads
+// no memory.  mean = sum / n rounded to fp32; var = sum (x - mean)^2 / n
+// with that rounded mean; empty bucket -> 0 (core.py:84-88).  Counts and
+// moments are written, not merged.
 // ---------------------------------------------------------------------------
-constexpr int kList = 8192;
+constexpr int kList = 2048;
 constexpr int kSlots = kUT / 16;
+template <typename KT>
+constexpr int kKeep = sizeof(KT) == 2 ? 12 : 6;  // members per slot kept in registers (48 of them)
 
 struct BuildMomentsLds {
   int toks[kList];
-  double red[kSlots][kD];
+  double red[kUT / 64][kD];
   unsigned wsum[kUT / 64];
   float mean[kD];
 };
 
-// Members among words [w0, w0 + 256) of the row -> toks[at ..] when they all
-// fit below kList.  Returns the chunk's member count (uniform); the caller
-// barriers before the list is read and before the next chunk.
-__device__ __forceinline__ unsigned compact_chunk(const uint32_t* row, int w0, int nw, int N, int* toks, unsigned at,
+// Members among words [w0, w0 + 256 W) of the row below word w1, W consecutive
+// words per thread (8: the row is 16-byte aligned, as a build's is and a
+// caller's of summarize need not be) ->
+// toks[at ..] when they all fit below kList.  Returns their count (uniform);
+// the caller barriers before the list is read and before the next chunk.
+template <int W>
+__device__ __forceinline__ unsigned compact_chunk(const uint32_t* row, int w0, int w1, int N, int* toks, unsigned at,
                                                   unsigned* wsum) {
-  const int wd = w0 + threadIdx.x;
-  uint32_t m = wd < nw ? row[wd] : 0u;
-  if (wd == nw - 1 && (N & 31)) m &= (1u << (N & 31)) - 1u;
-  const unsigned pc = (unsigned)__popc(m);
+  const int wd = w0 + W * (int)threadIdx.x, nw = (N + 31) >> 5;
+  uint32_t m[W];
+#pragma unroll
+  for (int i = 0; i < W; ++i) m[i] = 0u;
+  if constexpr (W == 8) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (wd + 4 * h < w1) {  // (row_words is a multiple of 4)
+        const uint4 v = *reinterpret_cast<const uint4*>(row + wd + 4 * h);
+        m[4 * h] = v.x; m[4 * h + 1] = v.y; m[4 * h + 2] = v.z; m[4 * h + 3] = v.w;
+      }
+  } else if (wd < w1) {
+    m[0] = row[wd];
+  }
+  unsigned pc = 0u;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    if (wd + i >= nw) m[i] = 0u;
+    if (wd + i == nw - 1 && (N & 31)) m[i] &= (1u << (N & 31)) - 1u;
+    pc += (unsigned)__popc(m[i]);
+  }
   const unsigned incl = block_incl_scan<kUT>(pc, wsum);
   const unsigned total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
   if (at + total <= (unsigned)kList) {
     unsigned p = at + incl - pc;
-    while (m) {
-      toks[p++] = wd * 32 + (int)__builtin_ctz(m);
-      m &= m - 1u;
-    }
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+      for (; m[i]; m[i] &= m[i] - 1u) toks[p++] = (wd + i) * 32 + (int)__builtin_ctz(m[i]);
   }
   return total;
 }
 
-template <bool kDev, typename KT>
-__device__ __forceinline__ void accumulate_rows(const KT* kg, const int* toks, unsigned n, int slot, int d0,
-                                                const float (&m)[8], double (&acc)[8]) {
-#pragma unroll 4
-  for (unsigned i = slot; i < n; i += kSlots) {
-    float x[8];
-    KeyLoad<KT>::load8(kg + (size_t)toks[i] * kD + d0, x);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if constexpr (kDev) {
-        const double t = (double)x[j] - (double)m[j];
-        acc[j] += t * t;
-      } else {
-        acc[j] += (double)x[j];
-      }
-    }
-  }
+// v of lane l ^ M, M = 16 or 32.
+template <int M>
+__device__ __forceinline__ double xor_d(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const unsigned x = M == 16 ? xor16_u(lo) : xor32_u(lo), y = M == 16 ? xor16_u(hi) : xor32_u(hi);
+  return __longlong_as_double((long long)(((unsigned long long)y << 32) | x));
 }
 
-// One pass over the members (kDev: squared deviations from m), reduced over
-// the slots into red[0][..] order-fixed sums for tid < kD (returned).
-template <bool kDev, typename KT>
-__device__ double bucket_pass(BuildMomentsLds& L, const uint32_t* row, const KT* kg, int nw, int N, bool kept,
-                              unsigned n, const float (&m)[8]) {
-  const int tid = threadIdx.x, slot = tid >> 4, d0 = (tid & 15) * 8;
-  double acc[8];
+// One pass's order-fixed sum over the slots: of dim tid for tid < kD.
+__device__ __forceinline__ double slot_sum(BuildMomentsLds& L, double (&acc)[8]) {
+  const int tid = threadIdx.x, lane = tid & 63;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] = 0.0;
-  if (kept) {
-    accumulate_rows<kDev>(kg, L.toks, n, slot, d0, m, acc);
-  } else {
-    for (int w0 = 0; w0 < nw; w0 += kUT) {
-      __syncthreads();  // the previous chunk's list has been read
-      const unsigned c = compact_chunk(row, w0, nw, N, L.toks, 0u, L.wsum);  // <= 8192: always fits
-      __syncthreads();
-      accumulate_rows<kDev>(kg, L.toks, c, slot, d0, m, acc);
-    }
+  for (int j = 0; j < 8; ++j) {
+    acc[j] += xor_d<16>(acc[j]);
+    acc[j] += xor_d<32>(acc[j]);
   }
+  if (lane < 16)
 #pragma unroll
-  for (int j = 0; j < 8; ++j) L.red[slot][d0 + j] = acc[j];
+    for (int j = 0; j < 8; ++j) L.red[tid >> 6][8 * lane + j] = acc[j];
   __syncthreads();
-  double t = 0.0;
-  if (tid < kD)
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) t += L.red[i][tid];
+  const double t = tid < kD ? (L.red[0][tid] + L.red[1][tid]) + (L.red[2][tid] + L.red[3][tid]) : 0.0;
   __syncthreads();  // red is free again
   return t;
 }
 
 template <typename KT>
-__global__ __launch_bounds__(kUT) void build_moments_kernel(UpdateArgs a) {
-  const int f = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+__global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
+  static_assert(kF % 8 == 0, "buckets in 8 equal runs");
+  const int f = (int)(blockIdx.x & 7u) * (kF / 8) + (int)(blockIdx.x >> 3), g = blockIdx.y;
+  const int tid = threadIdx.x, slot = tid >> 4, d0 = (tid & 15) * 8;
   __shared__ BuildMomentsLds L;
+  typedef KeyLoad<KT> KL;
   const uint32_t* row = a.bits + ((size_t)g * kF + f) * a.row_words;
-  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks;
+  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + d0;
   const int nw = (a.N + 31) >> 5;
   // count the members, keeping the list while it fits
   unsigned n = 0;
-  bool kept = true;
-  for (int w0 = 0; w0 < nw; w0 += kUT) {
-    const unsigned c = compact_chunk(row, w0, nw, a.N, L.toks, n, L.wsum);
+  bool listed = true;
+  const bool wide = ((a.row_words & 3) | (int64_t)(reinterpret_cast<uintptr_t>(a.bits) & 15u)) == 0;
+  for (int w0 = 0; w0 < nw; w0 += wide ? 8 * kUT : kUT) {  // uniform
+    const unsigned c = wide ? compact_chunk<8>(row, w0, nw, a.N, L.toks, n, L.wsum)
+                            : compact_chunk<1>(row, w0, nw, a.N, L.toks, n, L.wsum);
+    listed = listed && n + c <= (unsigned)kList;
     __syncthreads();
-    if (n + c > (unsigned)kList) {
-      kept = false;
-      n = 0;
-      for (int w1 = 0; w1 < nw; w1 += kUT) {  // count only: the list is rebuilt per chunk in the passes
-        const int wd = w1 + tid;
-        uint32_t m = wd < nw ? row[wd] : 0u;
-        if (wd == nw - 1 && (a.N & 31)) m &= (1u << (a.N & 31)) - 1u;
-        block_incl_scan<kUT>((unsigned)__popc(m), L.wsum);
-        n += L.wsum[0] + L.wsum[1] + L.wsum[2] + L.wsum[3];
-        __syncthreads();
-      }
-      break;
-    }
     n += c;
   }
-  float zero[8];
+  auto key_row = [&](unsigned i) { return KL::raw8(kg + (size_t)L.toks[i] * kD); };
+  typename KL::Raw8 kept[kKeep<KT>];
+  if (listed)
 #pragma unroll
-  for (int j = 0; j < 8; ++j) zero[j] = 0.f;
-  const double sum = bucket_pass<false>(L, row, kg, nw, a.N, kept, n, zero);
+    for (int u = 0; u < kKeep<KT>; ++u)
+      if (kSlots * u < (int)n) kept[u] = key_row(min((unsigned)(slot + kSlots * u), n - 1u));  // uniform
+  double acc[8];
+  auto each_member = [&](auto add) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0;
+    if (listed) {
+#pragma unroll
+      for (int u = 0; u < kKeep<KT>; ++u)
+        if (slot + kSlots * u < (int)n) add(kept[u]);
+#pragma unroll 4
+      for (unsigned i = slot + kSlots * kKeep<KT>; i < n; i += kSlots) add(key_row(i));
+    } else {
+      for (int w0 = 0; w0 < nw; w0 += kList / 32) {
+        __syncthreads();  // the previous chunk's list has been read
+        const unsigned c = compact_chunk<1>(row, w0, min(nw, w0 + kList / 32), a.N, L.toks, 0u, L.wsum);  // always fits
+        __syncthreads();
+#pragma unroll 4
+        for (unsigned i = slot; i < c; i += kSlots) add(key_row(i));
+      }
+    }
+  };
+  each_member([&](const typename KL::Raw8& r) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += (double)KL::at(r, j);
+  });
+  const double sum = slot_sum(L, acc);
   if (tid < kD) L.mean[tid] = n ? (float)(sum / (double)n) : 0.f;
   __syncthreads();
   float m[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) m[j] = L.mean[(tid & 15) * 8 + j];
-  const double dev = bucket_pass<true>(L, row, kg, nw, a.N, kept, n, m);
+  for (int j = 0; j < 8; ++j) m[j] = L.mean[d0 + j];
+  each_member([&](const typename KL::Raw8& r) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const double t = (double)KL::at(r, j) - (double)m[j];
+      acc[j] += t * t;
+    }
+  });
+  const double dev = slot_sum(L, acc);
   if (tid < kD) {
     float* tile = a.moments + (size_t)(g * kChunks + f / kChunk) * kRow * kChunk;
     const int col = f % kChunk;
@@ -1081,26 +1546,6 @@ __global__ __launch_bounds__(kUT) void build_moments_kernel(UpdateArgs a) {
 // each range's strict values and ties (tcount[2r], tcount[2r + 1]),
 // flat_emit_kernel writes them after the lower ranges' ones.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kUT) void hist0_kernel(UpdateArgs a) {
-  const int g = blockIdx.y, tid = threadIdx.x;
-  __shared__ unsigned hist[kBins];
-  for (int i = tid; i < kBins; i += kUT) hist[i] = 0;
-  __syncthreads();
-  const size_t n = (size_t)a.N * kF;
-  const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * n);
-  for (size_t i = (size_t)blockIdx.x * kUT + tid; i < n / 4; i += (size_t)gridDim.x * kUT) {
-    const float4 v4 = ag[i];
-    const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (vv[j] > 0.f) atomicAdd(&hist[__float_as_uint(vv[j]) >> 20], 1u);
-  }
-  __syncthreads();
-  unsigned* hg = hist_of(a, g, 0) + (blockIdx.x % kRep) * kBins;
-  for (int i = tid; i < kBins; i += kUT)
-    if (hist[i]) atomicAdd(&hg[i], hist[i]);
-}
-
 struct FlatRule {
   float tau;
   bool all_pos, ties;
@@ -1226,7 +1671,7 @@ using namespace prismkv;
 // therefore serves every smaller block: no call finds another call's
 // activations or list where it expects zeroed histograms.
 struct UpdateLayout {
-  size_t hist, ctl, tcount, part, wsplit, wscale, act, list, total;
+  size_t hist, ctl, tcount, part, wsplit, sample, act, list, ties, total;
   unsigned list_cap;
   UpdateLayout(int groups, int N) {
     size_t o = 0;
@@ -1236,12 +1681,12 @@ struct UpdateLayout {
     tcount = take((size_t)groups * kMaxTieBlocks * 2 * sizeof(unsigned));
     part = take((size_t)groups * kCenterParts * kD * sizeof(double));
     wsplit = take((size_t)groups * kFTiles * kWTile * sizeof(_Float16));
-    wscale = take((size_t)groups * kFTiles * kFT * sizeof(float));
+    sample = take((size_t)groups * kSampleBins * sizeof(unsigned));
     act = take((size_t)groups * N * kF * sizeof(float));
-    // the compact list: room for 16 candidates per key (twice the 8 H
-    // budget of an index build) plus the chunk tails, at least 2^19
-    list_cap = N > 0 ? std::max(1u << 19, 16u * (unsigned)N + kListSlack) : 0u;
+    // the candidate list: six times the 8 N budget of an index build, at least 2^19
+    list_cap = N > 0 ? std::max(1u << 19, (unsigned)kListPerKey * (unsigned)N + kListSlack) : 0u;
     list = take((size_t)groups * list_cap * sizeof(uint2));
+    ties = take((size_t)groups * list_cap * sizeof(unsigned));
     total = o;
   }
 };
@@ -1263,12 +1708,15 @@ static UpdateArgs make_args(uint64_t k, uint64_t W, uint64_t b, uint64_t center,
   a.moments = reinterpret_cast<float*>(moments);
   a.act = reinterpret_cast<float*>(w + L.act);
   a.wsplit = reinterpret_cast<_Float16*>(w + L.wsplit);
-  a.wscale = reinterpret_cast<float*>(w + L.wscale);
   a.hist = reinterpret_cast<unsigned*>(w + L.hist);
   a.ctl = reinterpret_cast<unsigned*>(w + L.ctl);
   a.tcount = reinterpret_cast<unsigned*>(w + L.tcount);
   a.list = reinterpret_cast<uint2*>(w + L.list);
   a.list_cap = L.list_cap;
+  a.sample = reinterpret_cast<unsigned*>(w + L.sample);
+  a.ties = reinterpret_cast<unsigned*>(w + L.ties);
+  a.listed = 0;
+  a.target = 0;
   a.H = H;
   a.N = N;
   a.budget = (long long)N * key_mean;
@@ -1299,23 +1747,48 @@ static int encode_parts(int rows) {
   return best;
 }
 
-// encode .. ties: the exact batch-wide positive Top-k of the N keys' activations
-// and their bitmap bits.
+// Sample tokens of a call over N keys: every key up to 128, 128 of up to 2048
+// (each of the 47 tiles' workgroups splits their rows again), 256 of up to
+// 16384, 1/64 beyond, at most 2048.
+static int sample_tokens(int N) {
+  if (N <= 2048) return std::min(N, kEncTokens / 2);
+  return std::min(2048, std::max(kEncTokens, N / 64 / kEncTokens * kEncTokens));
+}
+
+// sample .. emit: the exact batch-wide positive Top-k of the N keys' activations
+// and their bitmap bits.  `keep`: the activations are left in the workspace.
 template <typename KT>
-static void launch_selection(const UpdateArgs& a, int groups, hipStream_t s) {
+static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s) {
+  // Candidates are collected when the list holds three times the budget: the
+  // floor aims at 2 (select) or 1.5 times it, with up to 28% of a bin's width
+  // and what the sample does not count on top.
+  a.listed = 3 * a.budget <= (long long)a.list_cap;
+  const int S = a.listed ? sample_tokens(a.N) : 0;
+  const bool one = a.listed && a.N <= kSelectMax;
+  a.target = (unsigned)((one ? 4 : 3) * ((long long)S * (a.budget / a.N)) / 2);
   const int token_tiles = (a.N + kEncTokens - 1) / kEncTokens;
-  hipLaunchKernelGGL(wsplit_kernel, dim3(kFTiles, groups), dim3(kUT), 0, s, a);
-  hipLaunchKernelGGL(encode_kernel<KT>, dim3(token_tiles, encode_parts(token_tiles * groups), groups), dim3(kET), 0, s,
-                     a);
-  hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, 0);
-  for (int level = 1; level < kLevels; ++level) {
-    hipLaunchKernelGGL(refine_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a, level);
-    hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, level);
+  const dim3 grid(token_tiles, encode_parts(token_tiles * groups), groups);
+  hipLaunchKernelGGL(sample_kernel<KT>, dim3(std::max(1, (S + kEncTokens - 1) / kEncTokens), kFTiles, groups),
+                     dim3(kET), 0, s, a, S);
+  if (a.listed && keep) {
+    hipLaunchKernelGGL((encode_kernel<KT, true, true>), grid, dim3(kET), 0, s, a);
+  } else {
+    if (a.listed) hipLaunchKernelGGL((encode_kernel<KT, false, true>), grid, dim3(kET), 0, s, a);
+    hipLaunchKernelGGL((encode_kernel<KT, true, false>), grid, dim3(kET), 0, s, a);
+  }
+  if (one) {
+    hipLaunchKernelGGL(select_kernel, dim3(groups), dim3(kST), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(hist0_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
+    hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, 0);
+    for (int level = 1; level < kLevels; ++level) {
+      hipLaunchKernelGGL(refine_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a, level);
+      hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, level);
+    }
+    hipLaunchKernelGGL(tie_count_kernel, dim3(kTieGrid, groups), dim3(kUT), 0, s, a);
+    hipLaunchKernelGGL(tie_cut_kernel, dim3(groups), dim3(kST), 0, s, a);
   }
   hipLaunchKernelGGL(emit_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
-  const int tie_grid = std::min(a.tie_blocks, kTieGrid);
-  hipLaunchKernelGGL(tie_count_kernel, dim3(tie_grid, groups), dim3(kUT), 0, s, a);
-  hipLaunchKernelGGL(tie_take_kernel, dim3(tie_grid, groups), dim3(kUT), 0, s, a);
 }
 
 template <typename KT>
@@ -1337,14 +1810,8 @@ static int update_impl(uint64_t k, uint64_t W, uint64_t b, uint64_t center, uint
   const UpdateArgs a = make_args(k, W, b, center, scale, bits, counts, moments, work, groups, H, N, key_mean, ks,
                                  row_words, L);
   hipStream_t s = (hipStream_t)stream;
-  launch_selection<KT>(a, groups, s);
-  // member lists: N ints per wave of dynamic LDS (up to 64 KB, allowed once per key type)
-  static const hipError_t lds_ok = hipFuncSetAttribute(reinterpret_cast<const void*>(moments_kernel<KT>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)(kUT / 64 * kMaxBlock * sizeof(int)));
-  if (lds_ok != hipSuccess) return (int)lds_ok;
-  hipLaunchKernelGGL(moments_kernel<KT>, dim3(kChunks, groups), dim3(kUT), (size_t)(kUT / 64) * N * sizeof(int), s,
-                     a);
+  launch_selection<KT>(a, groups, true, s);
+  hipLaunchKernelGGL(moments_kernel<KT>, dim3(kChunks, groups), dim3(kMT), 0, s, a);
   return (int)hipGetLastError();
 }
 
@@ -1355,7 +1822,7 @@ static int build_impl(uint64_t k, uint64_t W, uint64_t b, uint64_t center, uint6
   if (groups < 1 || groups > 65535 || batch < 1 || batch > groups || H < 1 || H > kMaxBuild || key_mean < 1 ||
       key_mean > kF)
     return kBadSize;
-  if (flags & ~kBuildCenter) return kBadMode;
+  if (flags & ~(kBuildCenter | kBuildNoAct)) return kBadMode;
   if (ks < (int64_t)H * kD || row_words < (H + 31) / 32 || (row_words & 3)) return kBadSize;
   if (!k || !W || !b || !center || !scale || !bits || !counts || !moments || !work) return kBadSize;
   if (!aligned16<KT>(k, ks) || ((bits | W | b) & 15u)) return kBadSize;
@@ -1379,7 +1846,7 @@ static int build_impl(uint64_t k, uint64_t W, uint64_t b, uint64_t center, uint6
                          reinterpret_cast<float*>(cg));
     }
     hipLaunchKernelGGL(clear_bits_kernel, dim3(512, nb), dim3(kUT), 0, s, a);
-    launch_selection<KT>(a, nb, s);
+    launch_selection<KT>(a, nb, !(flags & kBuildNoAct), s);
     hipLaunchKernelGGL(build_moments_kernel<KT>, dim3(kF, nb), dim3(kUT), 0, s, a);
   }
   return (int)hipGetLastError();

@@ -204,14 +204,14 @@ class Native8B:
         with torch.cuda.device(k.device):
             obj._allocate(history, capacity, library, k.device, center)
             obj.set_encoder_tables(W, b, key_scale, key_mean)
-            flags = 0
+            flags = 0 if keep_activations else 4  # 4: they need not be left in the workspace
             if obj.center is None:
                 obj.center = torch.zeros(GROUPS, DIM, dtype=torch.float32, device=k.device)
-                flags = 1  # the device computes the centers
+                flags |= 1  # the device computes the centers
             per_group = obj.lib.query("prismkv_build_work_bytes", 1, history)
             batch = max(1, min(GROUPS, int(work_limit) // per_group))
-            work = torch.zeros(obj.lib.query("prismkv_build_work_bytes", batch, history), dtype=torch.uint8,
-                               device=k.device)
+            work = _lib.selection_work(obj.lib.query("prismkv_build_work_bytes", batch, history),
+                                       obj.lib.query("prismkv_update_act_offset", batch), k.device)
             obj.lib.call("prismkv_build", k.data_ptr(), obj.W_enc.data_ptr(), obj.b_enc.data_ptr(),
                          obj.center.data_ptr(), obj.key_scale.data_ptr(), obj.bits.data_ptr(), obj.n.data_ptr(),
                          obj.moments.data_ptr(), work.data_ptr(), GROUPS, batch, history, obj.key_mean, flags,
@@ -571,8 +571,9 @@ class Native8B:
         if self.history + block > self.capacity:
             raise ValueError("capacity exceeded: rebuild with a larger capacity")
         if block > self.update_block:
-            self.update_work = torch.zeros(self.lib.query("prismkv_update_work_bytes", GROUPS, block),
-                                           dtype=torch.uint8, device=self.out.device)
+            self.update_work = _lib.selection_work(self.lib.query("prismkv_update_work_bytes", GROUPS, block),
+                                                   self.lib.query("prismkv_update_act_offset", GROUPS),
+                                                   self.out.device)
             self.update_block = block
         self.lib.call("prismkv_update", k.data_ptr(), self.W_enc.data_ptr(), self.b_enc.data_ptr(),
                       self.center.data_ptr(), self.key_scale.data_ptr(), self.bits.data_ptr(), self.n.data_ptr(),
