@@ -346,6 +346,11 @@ size_t prismkv_topk_work_bytes(void);
 int prismkv_topk(uint64_t act, uint64_t out, uint64_t out_len, uint64_t work, int N, int64_t count,
                  size_t work_bytes, uint64_t stream);
 
+/* The id checks of attend (core.py:176-179) for one group's ids i64 [n]: out
+ * i32 [n] <- the ids (clamped into [0, H)), meta i32 [2] <- n, and 1 if an id lies
+ * outside [0, H) | 2 if an id comes twice.  H in [1, 2^20]. */
+int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int H, uint64_t stream);
+
 /* summarize (core.py:76-89) of every group from its bitmap rows: counts and
  * the tiled moments get each bucket's member count and the population mean
  * and variance of the member K rows (bit t of row f: row t of K, t < H);

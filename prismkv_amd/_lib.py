@@ -51,6 +51,7 @@ SIGNATURES = {
     "prismkv_route_scores": ([_U64] * 8 + [_I32, _SZ], True, _I32),
     "prismkv_topk_work_bytes": ([], False, _SZ),
     "prismkv_topk": ([_U64] * 4 + [_I32, _I64, _SZ], True, _I32),
+    "prismkv_check_ids": ([_U64] * 3 + [_I64, _I32], True, _I32),
     "prismkv_summarize_work_bytes": ([_I32], False, _SZ),
     "prismkv_summarize": ([_U64] * 6 + [_I32, _I32, _I32, _I64, _I64, _SZ], True, _I32),
     "prismkv_route_qact_work_bytes": ([_I32], False, _SZ),
@@ -124,8 +125,14 @@ def selection_work(nbytes_: int, head: int, device):
 
 
 def load(path=None) -> Library:
-    key = str(Path(path or DEFAULT_LIBRARY).resolve())
-    lib = _loaded.get(key)
+    # by the path as given first: resolving one takes 15 us, and core's functions ask on every call
+    given = str(path or DEFAULT_LIBRARY)
+    lib = _loaded.get(given)
     if lib is None:
-        lib = _loaded[key] = Library(key)
+        key = str(Path(given).resolve())
+        lib = _loaded.get(key)
+        if lib is None:
+            lib = _loaded[key] = Library(key)
+        if Path(given).is_absolute():  # (a relative path's meaning goes with the working folder)
+            _loaded[given] = lib
     return lib

@@ -303,7 +303,17 @@ def _check_q(q):
 QA_WIDTH = 64  # the q_activation selection: up to 4 heads x 16 buckets
 
 
-def _route_qact(q, index, sae, query_scale, scores):
+# One selection's small outputs, in one buffer so that the host reads them with
+# one copy: features i64 [64], valid f32 [64], raw and count i32, then the
+# router's valid f32 [64] before a cap rewrites it, then the union's workspace.
+_VALID, _RAW, _COUNT, _RANKED, _UNION = 512, 768, 772, 1024, 1280
+
+
+def _selection(device, union_bytes=0):
+    return torch.zeros(_UNION + union_bytes, dtype=torch.uint8, device=device)
+
+
+def _route_qact(q, index, sae, query_scale, scores, sel):
     t = _tables(index)
     q1, suffix = _check_q(q)
     _check_sae(sae)
@@ -311,29 +321,22 @@ def _route_qact(q, index, sae, query_scale, scores):
     device = q1.device
     W, b = _encoder(sae, device)
     qs = torch.tensor([float(query_scale)], dtype=torch.float32, device=device)
-    features = torch.zeros(1, QA_WIDTH, dtype=torch.int64, device=device)
-    valid = torch.zeros(1, QA_WIDTH, device=device)
-    raw = torch.zeros(1, dtype=torch.int32, device=device)
     work = _work("route_qact", lib.query("prismkv_route_qact_work_bytes", 1), device)
+    at = sel.data_ptr()
     lib.call("prismkv_route_qact" + suffix, q1.data_ptr(), W.data_ptr(), b.data_ptr(), qs.data_ptr(), t.n.data_ptr(),
-             work.data_ptr(), features.data_ptr(), valid.data_ptr(), raw.data_ptr(), scores.data_ptr(), 1,
-             _lib.nbytes(work), stream=_stream())
-    return t, features, valid, raw
+             work.data_ptr(), at, at + _VALID, at + _RAW, scores.data_ptr(), 1, _lib.nbytes(work), stream=_stream())
+    return t
 
 
-def _route(q, index, scores):
+def _route(q, index, scores, sel):
     t = _tables(index)
     q1, suffix = _check_q(q)
     lib = _lib_()
-    device = q1.device
-    features = torch.zeros(1, TOPK, dtype=torch.int64, device=device)
-    valid = torch.zeros(1, TOPK, device=device)
-    raw = torch.zeros(1, dtype=torch.int32, device=device)
-    work = _work("route", lib.query("prismkv_route_work_bytes", 1), device)
+    work = _work("route", lib.query("prismkv_route_work_bytes", 1), q1.device)
+    at = sel.data_ptr()
     lib.call("prismkv_route_scores" + suffix, q1.data_ptr(), t.moments.data_ptr(), t.n.data_ptr(), work.data_ptr(),
-             features.data_ptr(), valid.data_ptr(), raw.data_ptr(), scores.data_ptr(), 1, _lib.nbytes(work),
-             stream=_stream())
-    return t, features, valid, raw
+             at, at + _VALID, at + _RAW, scores.data_ptr(), 1, _lib.nbytes(work), stream=_stream())
+    return t
 
 
 def _check_router(router="moments", sae=None, query_scale=None, query_topk=16,
@@ -358,12 +361,13 @@ def bucket_scores(q, index, *, router="moments", sae=None, query_scale=None, que
     scores of the 4 queries' top-16 SAE activations, normalised per query,
     and every live bucket of positive score (up to 64), same order."""
     _check_router(router, sae, query_scale, query_topk, terms)
-    scores = torch.zeros(1, FEATURES, device=q.device)
+    scores = torch.empty(1, FEATURES, device=q.device)
+    sel = _selection(q.device)
     if router == "moments":
-        _, features, valid, _ = _route(q, index, scores)
+        _route(q, index, scores, sel)
     else:
-        _, features, valid, _ = _route_qact(q, index, sae, query_scale, scores)
-    return scores[0], features[0][valid[0] > 0]
+        _route_qact(q, index, sae, query_scale, scores, sel)
+    return scores[0], sel[:_VALID].view(torch.int64)[sel[_VALID:_RAW].view(torch.float32) > 0]
 
 
 @torch.no_grad()
@@ -377,33 +381,31 @@ def select_buckets(q, index, *, unique_cap=None, **kwargs):
         raise ValueError("unique_cap must be a fraction in [0,1]")
     router = _check_router(**kwargs)
     H = index.history
-    scores = torch.zeros(1, FEATURES, device=q.device)
-    if router == "q_activation":
-        t, features, valid, raw = _route_qact(q, index, kwargs["sae"], kwargs["query_scale"], scores)
-        width = QA_WIDTH
-    else:
-        t, features, valid, raw = _route(q, index, scores)
-        width = TOPK
-    candidates = int((valid[0] > 0).sum())
-    limit = H if unique_cap is None else math.floor(H * unique_cap)
+    scores = torch.empty(1, FEATURES, device=q.device)
     lib = _lib_()
+    sel = _selection(q.device, lib.query("prismkv_union_work_bytes", 1, max(H, 1)))
+    if router == "q_activation":
+        t, width = _route_qact(q, index, kwargs["sae"], kwargs["query_scale"], scores, sel), QA_WIDTH
+    else:
+        t, width = _route(q, index, scores, sel), TOPK
+    at = sel.data_ptr()
+    limit = H if unique_cap is None else math.floor(H * unique_cap)
     if unique_cap is not None:
-        lib.call("prismkv_select_cap_n", t.bits.data_ptr(), t.n.data_ptr(), features.data_ptr(), valid.data_ptr(),
-                 raw.data_ptr(), 1, H, limit, t.row_words, width, stream=_stream())
-    ids = torch.zeros(1, max(H, 1), dtype=torch.int32, device=q.device)
-    count = torch.zeros(1, dtype=torch.int32, device=q.device)
-    work = _work("union", lib.query("prismkv_union_work_bytes", 1, H), q.device)
-    lib.call("prismkv_union_n", t.bits.data_ptr(), features.data_ptr(), valid.data_ptr(), work.data_ptr(),
-             ids.data_ptr(), count.data_ptr(), 1, H, t.row_words, ids.shape[1], width, _lib.nbytes(work),
-             stream=_stream())
-    n = int(count.item())
-    if int(work[:4].view(torch.int32).item()):  # a bounded wait of the union gave up
-        work.zero_()
-        raise RuntimeError("prismkv_union_n: a bounded inter-workgroup wait gave up; the workspace was reset")
-    kept = features[0][valid[0] > 0].tolist()
+        sel[_RANKED:_UNION] = sel[_VALID:_RAW]
+        lib.call("prismkv_select_cap_n", t.bits.data_ptr(), t.n.data_ptr(), at, at + _VALID, at + _RAW, 1, H, limit,
+                 t.row_words, width, stream=_stream())
+    ids = torch.empty(1, max(H, 1), dtype=torch.int32, device=q.device)
+    lib.call("prismkv_union_n", t.bits.data_ptr(), at, at + _VALID, at + _UNION, ids.data_ptr(), at + _COUNT, 1, H,
+             t.row_words, ids.shape[1], width, sel.numel() - _UNION, stream=_stream())
+    host = sel[:_UNION + 4].cpu()  # one copy: everything the caller gets as Python numbers
+    if int(host[_UNION:].view(torch.int32)):  # a bounded wait of the union gave up
+        raise RuntimeError("prismkv_union_n: a bounded inter-workgroup wait gave up")
+    valid = host[_VALID:_RAW].view(torch.float32) > 0
+    raw, n = host[_RAW:_COUNT + 4].view(torch.int32).tolist()
+    candidates = valid if unique_cap is None else host[_RANKED:_UNION].view(torch.float32) > 0
     assert n <= limit
-    return ids[0, :n].long(), dict(features=kept, raw=int(raw.item()), unique=n, limit=limit,
-                                   candidate_buckets=candidates, scores=scores[0])
+    return ids[0, :n].long(), dict(features=host[:_VALID].view(torch.int64)[valid].tolist(), raw=raw, unique=n,
+                                   limit=limit, candidate_buckets=int(candidates.sum()), scores=scores[0])
 
 
 @torch.no_grad()
@@ -413,10 +415,19 @@ def attend(q, keys, values, old_ids, history):
     [history, len(keys)), fp32 accumulation, output in q's dtype."""
     if keys.shape != values.shape or not 0 <= history <= len(keys):
         raise ValueError("invalid KV/history")
-    if len(old_ids) and (old_ids.min() < 0 or old_ids.max() >= history):
-        raise ValueError("old_ids must address old history only")
-    if len(old_ids.unique()) != len(old_ids):
-        raise ValueError("deduplicate history before attention")
+    # on the device, the id checks run in one launch beside the attention and
+    # are read back once, after it; a call that the kernels would refuse, or
+    # ids elsewhere, are checked first, as the reference does
+    fused = (isinstance(old_ids, torch.Tensor) and old_ids.dtype == torch.int64 and old_ids.ndim == 1
+             and 0 < len(old_ids) and 1 <= history <= MAX_KEYS and tuple(q.shape) == (HEADS, DIM)
+             and keys.ndim == 2 and keys.shape[-1] == DIM
+             and all(x.device == q.device and x.device.type == "cuda" for x in (old_ids, keys, values))
+             and all(x.dtype.is_floating_point for x in (q, keys, values)))
+    if not fused:
+        if len(old_ids) and (old_ids.min() < 0 or old_ids.max() >= history):
+            raise ValueError("old_ids must address old history only")
+        if len(old_ids.unique()) != len(old_ids):
+            raise ValueError("deduplicate history before attention")
     if len(old_ids) + len(keys) - history == 0:
         return q.new_zeros(q.shape)
     _native(tuple(q.shape) == (HEADS, DIM), "GQA groups of 4 query heads of head_dim 128")
@@ -431,16 +442,27 @@ def attend(q, keys, values, old_ids, history):
     q1 = q1.reshape(1, HEADS, DIM)
     L = len(keys)
     lib = _lib_()
-    # an id row as wide as the history (the entry point's row stride), first len(old_ids) used
-    ids = torch.zeros(1, max(history, len(old_ids), 1), dtype=torch.int32, device=q.device)
-    ids[0, :len(old_ids)] = old_ids.to(device=q.device, dtype=torch.int32)
-    count = torch.tensor([len(old_ids)], dtype=torch.int32, device=q.device)
+    # an id row as wide as the history (the entry point's row stride), first
+    # len(old_ids) used; the two words before it are their count and the checks' result
+    row = torch.empty(2 + max(history, len(old_ids), 1), dtype=torch.int32, device=q.device)
+    meta, ids = row.data_ptr(), row.data_ptr() + 8
+    if fused:
+        old_ids = old_ids.contiguous()
+        lib.call("prismkv_check_ids", old_ids.data_ptr(), ids, meta, len(old_ids), history, stream=_stream())
+    else:
+        row[2:2 + len(old_ids)] = old_ids.to(device=q.device, dtype=torch.int32)
+        row[:1] = len(old_ids)
     out = torch.empty(1, HEADS, DIM, dtype=dtype, device=q.device)
     work = _work("attend", lib.query("prismkv_attend_work_bytes", 1, ATTEND_SPLITS), q.device)
-    lib.call("prismkv_attend" + suffix, q1.data_ptr(), keys.data_ptr(), values.data_ptr(), ids.data_ptr(),
-             count.data_ptr(), work.data_ptr(), out.data_ptr(), 1, history, L - history, L * DIM, L * DIM,
-             ids.shape[1], ATTEND_SPLITS, _lib.nbytes(work), stream=_stream())
-    code = int(work[:4].view(torch.int32).item())
+    lib.call("prismkv_attend" + suffix, q1.data_ptr(), keys.data_ptr(), values.data_ptr(), ids, meta,
+             work.data_ptr(), out.data_ptr(), 1, history, L - history, L * DIM, L * DIM,
+             row.numel() - 2, ATTEND_SPLITS, _lib.nbytes(work), stream=_stream())
+    bad = row[:2].tolist()[1] if fused else 0
+    if bad:
+        work.zero_()  # (more ids than the history has leave an error word)
+        raise ValueError("old_ids must address old history only" if bad & 1 else
+                         "deduplicate history before attention")
+    code = int(work[:4].view(torch.int32).item()) if bf16 else 0  # the fp32 kernel waits for nothing
     if code:  # a bounded wait of the attention gave up (ids were checked above)
         work.zero_()
         raise RuntimeError(f"prismkv_attend{suffix}: {ERROR_MESSAGES.get(code, ERROR_MESSAGES[ERR_WAIT])}; "

@@ -149,6 +149,50 @@ __global__ __launch_bounds__(kAT) void attend_merge(const float* __restrict__ st
   merge_group(state, S, blockIdx.x, out, lds.wts);
 }
 
+// The id checks of core.attend (core.py:176-179) in one launch of one
+// workgroup: every id in [0, H), none twice (an LDS bitmap of the history, 128
+// KB at 2^20 tokens), and the ids as the attention reads them (32 bits, clamped
+// into the history) with their count.  As a minimum, a maximum and a sorted
+// unique, each read back, they and the selection's read-backs took two thirds of
+// a 480 us call pair (core.select_buckets + core.attend at 1024 + 32 tokens, fp32;
+// 150 us with this kernel and one read-back each).  Bound by the one CU's reads:
+// 8 in flight per thread.
+constexpr int kIdThreads = 1024;
+constexpr int kMaxCheckedHistory = 1 << 20;
+constexpr int kIdRange = 1, kIdTwice = 2;  // meta[1]
+
+__global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __restrict__ ids, int n, int H,
+                                                               int32_t* __restrict__ out, int* __restrict__ meta) {
+  extern __shared__ unsigned seen[];
+  __shared__ int bad_s;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < (H + 31) / 32; i += kIdThreads) seen[i] = 0u;
+  if (tid == 0) bad_s = 0;
+  __syncthreads();
+  constexpr int kU = 8;
+  int bad = 0;
+  for (int i0 = tid; i0 < n; i0 += kU * kIdThreads) {
+    int64_t v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) v[u] = ids[i0 + u * kIdThreads < n ? i0 + u * kIdThreads : i0];
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (i0 + u * kIdThreads < n) {
+        const bool in = v[u] >= 0 && v[u] < H;
+        const int id = in ? (int)v[u] : 0;
+        out[i0 + u * kIdThreads] = id;
+        if (!in) bad |= kIdRange;
+        else if (atomicOr(&seen[id >> 5], 1u << (id & 31)) >> (id & 31) & 1u) bad |= kIdTwice;
+      }
+  }
+  if (bad) atomicOr(&bad_s, bad);
+  __syncthreads();
+  if (tid == 0) {
+    meta[0] = n;
+    meta[1] = bad_s;
+  }
+}
+
 }  // namespace
 }  // namespace prismkv
 
@@ -209,6 +253,21 @@ int prismkv_attend_f32(uint64_t q, uint64_t k, uint64_t v, uint64_t ids, uint64_
     return kBadSize;
   if (work_bytes < prismkv_attend_work_bytes(groups, splits)) return kBadSize;
   return attend_split_launch<float>(q, k, v, ids, count, work, out, groups, H, T, ks, vs, ids_stride, splits, stream);
+}
+
+int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int H, uint64_t stream) {
+  if (n < 0 || n > INT32_MAX || H < 1 || H > kMaxCheckedHistory || !out || !meta || (n && !ids)) return kBadSize;
+  const int lds = (H + 31) / 32 * (int)sizeof(unsigned);
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(check_ids_kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             kMaxCheckedHistory / 32 * (int)sizeof(unsigned));
+    if (e != hipSuccess) return (int)e;
+  }
+  hipLaunchKernelGGL(check_ids_kernel, dim3(1), dim3(kIdThreads), lds, (hipStream_t)stream,
+                     reinterpret_cast<const int64_t*>(ids), (int)n, H, reinterpret_cast<int32_t*>(out),
+                     reinterpret_cast<int*>(meta));
+  return (int)hipGetLastError();
 }
 
 // kernels/ppu_8b/av_tuned.cu:62-67 contract; state is the caller's

@@ -189,3 +189,30 @@ def test_attend_edges():
                              ids.cpu().numpy(), H)
         err = expect.attention_errors(bf16_bits(out), want)
         assert err["rel_l2"] <= 2e-3, err
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,n", [(1, 1), (31, 31), (1025, 1024), (5000, 777), (600000, 9000)])
+def test_attend_id_checks(H, n, dtype):
+    from prismkv_amd import core
+    # the checks of core.py:176-179 on the device: the same messages, and the call after a refused one is exact
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    k = torch.randn(H + 3, 128, generator=gen, device="cuda").to(dtype)
+    v = torch.randn(H + 3, 128, generator=gen, device="cuda").to(dtype)
+    q = torch.randn(4, 128, generator=gen, device="cuda").to(dtype)
+    ids = torch.randperm(H, generator=gen, device="cuda")[:n]
+    for at, value, message in ((n - 1, H, "old history only"), (0, -1, "old history only"), (n // 2, 1 << 40, "old history only")):
+        wrong = ids.clone()
+        wrong[at] = value
+        with pytest.raises(ValueError, match=message):
+            core.attend(q, k, v, wrong, H)
+    with pytest.raises(ValueError, match="deduplicate"):
+        core.attend(q, k, v, torch.cat((ids, ids[-1:])), H)
+    got = core.attend(q, k, v, ids, H)
+    rows = torch.cat((ids, torch.arange(H, H + 3, device="cuda")))
+    p = torch.softmax(q.double() @ k[rows].double().T / 128 ** 0.5, dim=-1)
+    want = p @ v[rows].double()
+    assert got.dtype == dtype
+    assert float((got.double() - want).norm() / want.norm()) < (4e-3 if dtype == torch.bfloat16 else 1e-5)
+    strided = torch.stack((ids, ids), dim=1)[:, 0]  # a view with a stride
+    assert torch.equal(core.attend(q, k, v, strided, H), got)
