@@ -327,6 +327,19 @@ int prismkv_route_qact(uint64_t q, uint64_t W, uint64_t b, uint64_t qscale, uint
                        uint64_t features, uint64_t valid, uint64_t raw, uint64_t scores, int groups, size_t work_bytes,
                        uint64_t stream);
 
+/* The decode step of the q_activation router (core.py:131-139, :142-183 with cap
+ * None) in two launches: prismkv_route_qact's candidates, then its ranking with
+ * prismkv_union_n's and prismkv_attend's work over the up to 64 buckets.  Writes
+ * the same features / valid [G][64], raw, ids and count as those, and out to
+ * rounding.  `qact_work` is prismkv_route_qact's workspace (scratch), `decode_work`
+ * prismkv_decode's; its limits and the -1 for a group that cannot be resident are
+ * prismkv_decode's. */
+int prismkv_decode_qact(uint64_t q, uint64_t W, uint64_t b, uint64_t qscale, uint64_t counts, uint64_t bits, uint64_t k,
+                        uint64_t v, uint64_t qact_work, uint64_t decode_work, uint64_t features, uint64_t valid, uint64_t raw,
+                        uint64_t ids, uint64_t count, uint64_t out, int groups, int H, int T, int capacity,
+                        int64_t row_words, int64_t ks, int64_t vs, int64_t ids_stride, size_t qact_work_bytes,
+                        size_t decode_work_bytes, uint64_t stream);
+
 /* prismkv_union / prismkv_select_cap over selections of `width` rows per
  * group (features / valid [G][width]), width 16 or 64. */
 int prismkv_union_n(uint64_t bits, uint64_t features, uint64_t valid, uint64_t work, uint64_t ids, uint64_t count,

@@ -56,6 +56,7 @@ SIGNATURES = {
     "prismkv_summarize": ([_U64] * 6 + [_I32, _I32, _I32, _I64, _I64, _SZ], True, _I32),
     "prismkv_route_qact_work_bytes": ([_I32], False, _SZ),
     "prismkv_route_qact": ([_U64] * 10 + [_I32, _SZ], True, _I32),
+    "prismkv_decode_qact": ([_U64] * 16 + [_I32] * 4 + [_I64] * 4 + [_SZ, _SZ], True, _I32),
     "prismkv_build_f32": ([_U64] * 9 + [_I32] * 5 + [_I64, _I64, _SZ], True, _I32),
     "prismkv_update_f32": ([_U64] * 9 + [_I32] * 4 + [_I64, _I64, _SZ], True, _I32),
     "prismkv_summarize_f32": ([_U64] * 6 + [_I32, _I32, _I32, _I64, _I64, _SZ], True, _I32),

@@ -254,6 +254,10 @@ size_t attend_list_work_bytes(int groups);
 int attend_list(uint64_t q, uint64_t k, uint64_t v, uint64_t ids, uint64_t count, uint64_t work, uint64_t out,
                 int groups, int H, int T, int64_t ks, int64_t vs, int64_t ids_stride, uint64_t stream);
 
+// The candidates of the q_activation router (defined in route.hip): each head's
+// 16 best keys of each bucket range, into `work` (prismkv_route_qact_work_bytes).
+int qact_candidates(uint64_t q, uint64_t W, uint64_t b, uint64_t qscale, uint64_t work, int groups, uint64_t stream);
+
 // Error words.  A workspace's first 32-bit word is its sticky error word; its
 // 8-byte slot at byte offset 8 optionally holds the device address of a
 // host-mapped 32-bit word (0 = none), so a host binding can notice an error

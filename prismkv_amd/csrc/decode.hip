@@ -15,7 +15,9 @@
 // unique cap has walked it) or phases 6-9 on a given id list (prismkv_attend);
 // the capped variant runs the budgeted walk between phases 4 and 6
 // (prismkv_decode_capped); the route-only variant stops after the ids
-// (prismkv_route_union).
+// (prismkv_route_union); the q_activation variant ranks that router's
+// candidates in every workgroup and runs phases 5-9 on its up to 64 buckets
+// (prismkv_decode_qact).
 //
 // Grid (S, G) x 512, S = clamp(256 / G, 32, 256) (32 for 8 groups: the whole
 // launch is resident at once, one workgroup per CU, at any history).  Workgroup p
@@ -65,6 +67,7 @@
 #include <mutex>
 
 #include "attend_mfma.h"
+#include "qact.h"
 #include "score.h"
 
 // The attention phase runs on the matrix cores (v_mfma_f32_16x16x32_bf16 for
@@ -127,6 +130,8 @@ struct DecodeArgs {
   // replace the selection and the union; ids / count are then not written
   const int32_t* ids_in;
   const int32_t* count_in;
+  // the q_activation router's candidates (qact_part_kernel's)
+  const unsigned long long* qcand;
 };
 
 // The tile's selected tokens live in dynamic LDS after this struct, sized
@@ -995,8 +1000,11 @@ __device__ __forceinline__ void route_finish(const DecodeArgs& a, int g, int p, 
 
 // kWide: union tiles of 65-128 words (the host's choice when tw > 64), whose
 // two chunks' words phase 4 requests.
+// kQact (with kGiven): the selected rows come from the q_activation router's
+// candidates, in every workgroup of the group (a launch of its own for the
+// ranking took 8 us, the union's 9.7).
 template <int KW, bool kGiven = false, bool kCap = false, bool kEarlyTail = false, bool kRouteOnly = false,
-          bool kWide = false>
+          bool kWide = false, bool kQact = false>
 __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
   const int p = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   __shared__ DecodeLds lds;
@@ -1018,8 +1026,50 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
   uint4 ek[1][4], ev[1][4];
 
   // attention over a given id list: no selection, no union (uniform)
-  const bool id_list = kGiven && a.ids_in != nullptr;
-  if constexpr (kGiven) {
+  const bool id_list = kGiven && !kQact && a.ids_in != nullptr;
+  if constexpr (kQact) {
+    // ---- 1-4. the rows of the q_activation router's selection: wave h takes
+    // head h's 16 buckets of positive weight (a bucket that two heads chose
+    // counts once in an OR, and an empty one has no bit set, so the union needs
+    // neither the scores nor their order: the group's last workgroup ranks them
+    // for the caller after its attention), and wave w ORs rows w, w + 8, ...
+    // over the tile's first 128 words
+    int* sel64 = reinterpret_cast<int*>(lds.sel.best);  // -1: none
+    static_assert(kQaSel * sizeof(int) <= sizeof(lds.sel.best) && kQaSel * sizeof(unsigned long long) <= sizeof(lds.tl),
+                  "the heads' buckets, and their keys kept for the ranking");
+    if (w < kHq) {
+      const unsigned long long best = qact_head_top(a.qcand, g, w);
+      const float weight = qact_weight(best);
+      if (lane < kTop) {
+        reinterpret_cast<unsigned long long*>(lds.tl)[kTop * w + lane] = best;
+        sel64[kTop * w + lane] = weight > 0.f ? row_of(best) : -1;
+      }
+    }
+    __syncthreads();
+    if (a.tw <= 2 * kTileWords) {
+      constexpr int kRows = kQaSel / (kDT / 64);
+      const int words = (a.H + 31) / 32, wd = p * a.tw + lane;
+      const bool in = lane < a.tw && wd < words, in2 = lane + kTileWords < a.tw && wd + kTileWords < words;
+      uint32_t v[kRows], v2[kRows];
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        const int row = __builtin_amdgcn_readfirstlane(sel64[w + kDT / 64 * i]);
+        const __amdgpu_buffer_rsrc_t res = raw_buffer(a.bits + ((size_t)g * kF + max(row, 0)) * a.row_words,
+                                                      row >= 0 ? (int)a.row_words * 4 : 0);  // past the row: 0
+        v[i] = load_nt4_buf(res, in ? (unsigned)wd * 4u : ~0u);
+        v2[i] = a.tw > kTileWords ? load_nt4_buf(res, in2 ? (unsigned)(wd + kTileWords) * 4u : ~0u) : 0u;
+      }
+      uint32_t m = 0u, m2 = 0u;
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        m |= v[i];
+        m2 |= v2[i];
+      }
+      lds.sel.ors[w][lane] = m;
+      lds.sel.ors2[w][lane] = m2;
+      __syncthreads();
+    }
+  } else if constexpr (kGiven) {
     // ---- 1-4. the given selection: the valid, in-range buckets in order (an
     // out-of-range id selects nothing, as in union_kernel); no row is
     // prefetched, so the union loads every selected row
@@ -1107,7 +1157,7 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
         m |= lds.sel.ors[k][lane];
         covered |= lds.cover[k];
       }
-      const unsigned missing = ((1u << nr) - 1u) & ~covered;  // winners' ranks no wave prefetched (uniform)
+      const unsigned missing = kQact ? 0u : ((1u << nr) - 1u) & ~covered;  // winners' ranks no wave prefetched (uniform)
       if (missing && lane < a.tw && wd < nw) {
         // one round of loads: every rank loads (a covered one repeats the first
         // missing row) and only the missing ones are kept
@@ -1139,7 +1189,24 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
     uint32_t m = 0u;
     int n = 0, incl = 0;
     if (w < chunks) {
-      if constexpr (kPfChunks > 1) {
+      if constexpr (kQact) {
+        // up to two chunks: the waves' ORs; more: every row's words of chunk w, 16 rows at a time
+        if (chunks <= 2) {
+#pragma unroll
+          for (int k = 0; k < kDT / 64; ++k) m |= w ? lds.sel.ors2[k][lane] : lds.sel.ors[k][lane];
+        } else if (cw < a.tw && wd < nw) {
+          const int* sel64 = reinterpret_cast<const int*>(lds.sel.best);
+          const uint32_t* gb = a.bits + (size_t)g * kF * a.row_words + wd;
+          for (int r0 = 0; r0 < kQaSel; r0 += kTop) {
+            uint32_t v[kTop];
+#pragma unroll
+            for (int r = 0; r < kTop; ++r)
+              v[r] = __builtin_nontemporal_load(gb + (size_t)max(sel64[r0 + r], 0) * a.row_words);
+#pragma unroll
+            for (int r = 0; r < kTop; ++r) m |= sel64[r0 + r] >= 0 ? v[r] : 0u;
+          }
+        }
+      } else if constexpr (kPfChunks > 1) {
         // chunk w < 2 (both prefetched): the waves' ORs, then one round of
         // loads for the winners no wave prefetched (every rank loads, a
         // covered one repeating the first missing row, and only the missing
@@ -1517,6 +1584,21 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
     if (p == a.S - 1 && w == 0)
       write_selection(lds.win, lds.need, a.counts + (size_t)g * kFP, a.features + (size_t)g * kTop,
                       a.valid + (size_t)g * kTop, a.raw + g);
+  if constexpr (kQact)
+    if (p == a.S - 1 && w == 0) {
+      int bucket;
+      float score;
+      bool first;
+      const int* cg = a.counts + (size_t)g * kFP;
+      const unsigned long long key =
+          qact_rank(reinterpret_cast<const unsigned long long*>(lds.tl), cg, bucket, score, first);
+      const int n = __popcll(__ballot(key != 0ull));
+      const int f = lane < n ? row_of(key) : 0;
+      a.features[(size_t)g * kQaSel + lane] = f;
+      a.valid[(size_t)g * kQaSel + lane] = lane < n ? 1.f : 0.f;
+      const int sum = wave_sum_i(lane < n ? cg[f] : 0);
+      if (lane == 0) a.raw[g] = sum;
+    }
   // ---- 9. workgroups 0..15 each merge one (head, 32-dim slice) of the S
   // split states into out[g] and clear the words they read; workgroup 0
   // also clears the group's statistics, candidates and tile counts (every
@@ -1611,6 +1693,10 @@ static int resident_workgroups() {
                          reinterpret_cast<const void*>(decode_kernel<2, true>),
                          reinterpret_cast<const void*>(decode_kernel<4, true>),
                          reinterpret_cast<const void*>(decode_kernel<8, true>),
+                         reinterpret_cast<const void*>(decode_kernel<1, true, false, false, false, false, true>),
+                         reinterpret_cast<const void*>(decode_kernel<2, true, false, false, false, false, true>),
+                         reinterpret_cast<const void*>(decode_kernel<4, true, false, false, false, false, true>),
+                         reinterpret_cast<const void*>(decode_kernel<8, true, false, false, false, false, true>),
                          reinterpret_cast<const void*>(decode_kernel<1, false, true>),
                          reinterpret_cast<const void*>(decode_kernel<2, false, true>),
                          reinterpret_cast<const void*>(decode_kernel<4, false, true>),
@@ -1670,13 +1756,13 @@ static int decode_check(uint64_t q, uint64_t moments, uint64_t counts, uint64_t 
 // One fused variant's launch for S workgroups per group: KW = ceil(S / 32)
 // 64-key candidate sets per wave (the wide variant is never taken above
 // S = 128, so it has no KW = 8 instantiation).
-template <bool kGiven, bool kCap, bool kEarlyTail, bool kRouteOnly, bool kWide>
+template <bool kGiven, bool kCap, bool kEarlyTail, bool kRouteOnly, bool kWide, bool kQact = false>
 static void launch_decode(int S, dim3 grid, size_t dyn, hipStream_t s, const DecodeArgs& a) {
   const dim3 block(kDT);
-  if (S <= 32) hipLaunchKernelGGL((decode_kernel<1, kGiven, kCap, kEarlyTail, kRouteOnly, kWide>), grid, block, dyn, s, a);
-  else if (S <= 64) hipLaunchKernelGGL((decode_kernel<2, kGiven, kCap, kEarlyTail, kRouteOnly, kWide>), grid, block, dyn, s, a);
-  else if (S <= 128) hipLaunchKernelGGL((decode_kernel<4, kGiven, kCap, kEarlyTail, kRouteOnly, kWide>), grid, block, dyn, s, a);
-  else if constexpr (!kWide) hipLaunchKernelGGL((decode_kernel<8, kGiven, kCap, kEarlyTail, kRouteOnly, false>), grid, block, dyn, s, a);
+  if (S <= 32) hipLaunchKernelGGL((decode_kernel<1, kGiven, kCap, kEarlyTail, kRouteOnly, kWide, kQact>), grid, block, dyn, s, a);
+  else if (S <= 64) hipLaunchKernelGGL((decode_kernel<2, kGiven, kCap, kEarlyTail, kRouteOnly, kWide, kQact>), grid, block, dyn, s, a);
+  else if (S <= 128) hipLaunchKernelGGL((decode_kernel<4, kGiven, kCap, kEarlyTail, kRouteOnly, kWide, kQact>), grid, block, dyn, s, a);
+  else if constexpr (!kWide) hipLaunchKernelGGL((decode_kernel<8, kGiven, kCap, kEarlyTail, kRouteOnly, false, kQact>), grid, block, dyn, s, a);
 }
 
 // Enqueues a decode launch whose arguments decode_check accepted.
@@ -1684,7 +1770,7 @@ static int decode_launch(uint64_t q, uint64_t moments, uint64_t counts, uint64_t
                          uint64_t work, uint64_t features, uint64_t valid, uint64_t raw, uint64_t ids, uint64_t count,
                          uint64_t out, const int* tail_dev, bool given, int groups, int H, int T, int64_t row_words,
                          int64_t ks, int64_t vs, int64_t ids_stride, uint64_t stream, unsigned* err, int64_t limit,
-                         bool route_only = false) {
+                         bool route_only = false, uint64_t qcand = 0) {
   const int S = decode_splits(groups);
   const DecodeWorkLayout L(groups, S);
   char* w = reinterpret_cast<char*>(work);
@@ -1726,13 +1812,16 @@ static int decode_launch(uint64_t q, uint64_t moments, uint64_t counts, uint64_t
   a.out = reinterpret_cast<uint16_t*>(out);
   a.ids_in = nullptr;
   a.count_in = nullptr;
+  a.qcand = reinterpret_cast<const unsigned long long*>(qcand);
   const dim3 grid(S, groups);
   hipStream_t s = (hipStream_t)stream;
   const size_t rows_bytes = (size_t)32 * a.tw * sizeof(int);  // the tile's row list (dynamic LDS)
   // wide: union tiles of 65-128 words, both chunks prefetched (S <= 128 at
   // every history the single launch takes, 8 groups above 64K)
   const bool wide = a.tw > kTileWords && a.tw <= kPrefetchChunks * kTileWords && S <= 128;
-  if (route_only) {
+  if (qcand) {
+    launch_decode<true, false, false, false, false, true>(S, grid, rows_bytes, s, a);
+  } else if (route_only) {
     if (wide) launch_decode<false, false, false, true, true>(S, grid, rows_bytes, s, a);
     else launch_decode<false, false, false, true, false>(S, grid, rows_bytes, s, a);
   } else if (limit >= 0) {
@@ -1856,6 +1945,8 @@ __global__ __launch_bounds__(256) void clear_words(uint4* p, size_t n16) {
 
 extern "C" {
 
+size_t prismkv_route_qact_work_bytes(int groups);
+
 size_t prismkv_scratch_bytes(void) { return kScratchBytes; }
 
 int prismkv_decode_noalloc(uint64_t q, uint64_t moments, uint64_t counts, uint64_t bits, uint64_t k, uint64_t v,
@@ -1906,6 +1997,24 @@ int prismkv_decode(uint64_t q, uint64_t moments, uint64_t counts, uint64_t bits,
                    int64_t ids_stride, size_t work_bytes, uint64_t stream) {
   return decode_impl(q, moments, counts, bits, k, v, work, features, valid, raw, ids, count, out, nullptr, false, groups,
                      H, T, capacity, row_words, ks, vs, ids_stride, work_bytes, stream);
+}
+
+int prismkv_decode_qact(uint64_t q, uint64_t W, uint64_t b, uint64_t qscale, uint64_t counts, uint64_t bits, uint64_t k,
+                        uint64_t v, uint64_t qact_work, uint64_t work, uint64_t features, uint64_t valid, uint64_t raw,
+                        uint64_t ids, uint64_t count, uint64_t out, int groups, int H, int T, int capacity,
+                        int64_t row_words, int64_t ks, int64_t vs, int64_t ids_stride, size_t qact_work_bytes,
+                        size_t work_bytes, uint64_t stream) {
+  if (groups < 1 || groups > 65535) return kBadSize;
+  if (work_bytes < DecodeWorkLayout(groups, decode_splits(groups)).total) return kBadSize;
+  if (qact_work_bytes < prismkv_route_qact_work_bytes(groups)) return kBadSize;
+  if (!W || !b || !qscale || !counts || !qact_work || !raw || (W & 15u)) return kBadSize;
+  int rc = decode_check(q, 0, counts, bits, k, v, work, features, valid, raw, ids, count, out, true, groups, H, T,
+                        capacity, row_words, ks, vs, ids_stride, -1);
+  if (rc) return rc;
+  rc = qact_candidates(q, W, b, qscale, qact_work, groups, stream);
+  if (rc) return rc;
+  return decode_launch(q, 0, counts, bits, k, v, work, features, valid, raw, ids, count, out, nullptr, true, groups, H, T,
+                       row_words, ks, vs, ids_stride, stream, nullptr, -1, false, qact_work);
 }
 
 int prismkv_union_attend(uint64_t q, uint64_t bits, uint64_t k, uint64_t v, uint64_t work, uint64_t features,

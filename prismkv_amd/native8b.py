@@ -501,11 +501,21 @@ class Native8B:
                           k.shape[1] - self.history, self.capacity, self.row_words, k.stride(0), v.stride(0),
                           self.capacity, _lib.nbytes(self.decode_work), stream=self._stream())
             return self.out
-        if self.history > FUSED_MAX_HISTORY or self.router != "moments":
-            # very long histories exceed one launch's group size; the q_activation
-            # router selects up to 64 buckets
+        if self.history > FUSED_MAX_HISTORY or (self.router != "moments" and self.unique_cap is not None):
+            # very long histories exceed one launch's group size; the
+            # q_activation router's up to 64 buckets are walked by cap_kernel
             self.route(q)
             return self.attention(q, k, v, **kwargs)
+        if self.router != "moments":
+            # two launches: the queries' activations, then ranking, union and attention
+            self.lib.call("prismkv_decode_qact", q.data_ptr(), self.W_query.data_ptr(), self.b_query.data_ptr(),
+                          self.query_scale.data_ptr(), self.n.data_ptr(), self.bits.data_ptr(), k.data_ptr(),
+                          v.data_ptr(), self.qact_work.data_ptr(), self.decode_work.data_ptr(),
+                          self.features.data_ptr(), self.valid.data_ptr(), self.raw.data_ptr(), self.ids.data_ptr(),
+                          self.count.data_ptr(), self.out.data_ptr(), GROUPS, self.history, k.shape[1] - self.history,
+                          self.capacity, self.row_words, k.stride(0), v.stride(0), self.capacity,
+                          _lib.nbytes(self.qact_work), _lib.nbytes(self.decode_work), stream=self._stream())
+            return self.out
         if self.unique_cap is not None:
             # the budgeted walk runs between selection and union, on the same launch
             self.lib.call("prismkv_decode_capped", q.data_ptr(), self.moments.data_ptr(), self.n.data_ptr(),

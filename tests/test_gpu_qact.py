@@ -140,3 +140,57 @@ def test_hf_q_activation_decode():
     log(f"  hf q_activation decode: {err}")
     assert err["rel_l2"] <= 2e-3 and err["max_abs"] < 0.05, err
     session.close()
+
+
+@pytest.mark.parametrize("H,T", [(1, 0), (40, 3), (2047, 1), (65536, 300), (65537, 0), (131072, 5), (140001, 700),
+                                 (524288, 2)])
+def test_fused_q_activation_equals_the_separate_launches(H, T):
+    # one to eight union chunks per workgroup (words past 64, 128): features, raw,
+    # ids and count bit for bit, out to the rounding of another partition
+    from prismkv_amd import Native8B
+    gen = torch.Generator(device="cuda").manual_seed(H + T)
+    k, v = (torch.randn(8, H + T, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(8, 4, 128, generator=gen, device="cuda").to(torch.bfloat16)
+    W = torch.randn(8, 3000, 128, generator=gen, device="cuda") / 128 ** 0.5
+    b = 0.05 * torch.randn(8, 3000, generator=gen, device="cuda")
+    # random bucket lists: every token in 8 random buckets, two of them shared by all groups
+    tok = torch.arange(H, device="cuda").repeat_interleave(8)
+    feat = torch.randint(0, 3000, (8 * H,), generator=gen, device="cuda")
+    order = (feat * H + tok).unique()
+    feat, tok = order // H, order % H
+    n = torch.bincount(feat, minlength=3000)
+    csr = tok.int().expand(8, -1).contiguous()
+    offsets = torch.cat((torch.zeros(1, dtype=torch.int64, device="cuda"), n.cumsum(0))).int().expand(8, -1).contiguous()
+    zeros = torch.zeros(8, 3000, 128, device="cuda")
+    op = Native8B.from_tables(H, n.expand(8, -1), zeros, zeros, csr, offsets)
+    op.set_query_encoders(W, b, torch.linspace(0.5, 1.5, 8))
+    op.router = "q_activation"
+    op.route(q)
+    want_out = op.attention(q, k, v).clone()
+    names = ("features", "valid", "raw", "count")
+    want = {x: getattr(op, x).clone() for x in names}
+    ids = [op.ids[g, :op.count[g]].clone() for g in range(8)]
+    for x in names + ("ids", "out"):
+        getattr(op, x).fill_(3)
+    for _ in range(2):
+        got = op(q, k, v)
+        for x in names:
+            assert torch.equal(getattr(op, x), want[x]), x
+        for g in range(8):
+            assert torch.equal(op.ids[g, :op.count[g]], ids[g]), g
+        # bf16 outputs of two exact softmaxes: at most a rounding of 2^-9 apart
+        assert float((got.float() - want_out.float()).norm()) <= 4e-3 * float(want_out.float().norm()) + 1e-6
+    assert op.decode_errors() == 0
+
+
+def test_fused_q_activation_refuses_what_the_decode_refuses():
+    from prismkv_amd import _lib
+    lib = _lib.load()
+    need, qneed = lib.query("prismkv_decode_work_bytes", 8, 100), lib.query("prismkv_route_qact_work_bytes", 8)
+    call = getattr(lib.cdll, "prismkv_decode_qact")
+    good = [*[16] * 16, 8, 100, 4, 100, 4, 104 * 128, 104 * 128, 100, qneed, need, 0]
+    for at, value in ((24, qneed - 1), (25, need - 1), (17, 0), (17, 524289), (18, -1), (19, 99), (20, 3), (21, 103 * 128),
+                      (1, 20), (1, 0), (8, 0)):
+        args = list(good)
+        args[at] = value
+        assert call(*args) == -1, (at, value)
