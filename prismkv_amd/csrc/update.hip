@@ -27,7 +27,7 @@
 // `interval` tokens, its cost is amortised):
 //   sample   W as pairs of f16 in the encode's operand order, and a histogram
 //            (13 bits) of the positive activations of a few hundred tokens;
-//   encode   the GEMM on the f16 matrix cores, 256 tokens x 64 buckets per
+//   encode   the GEMM on the f16 matrix cores, 512 buckets x 16 tokens per
 //            workgroup and step, a = relu(...): the values at or above a floor
 //            read off the sample (about twice the budget of them) go to the
 //            group's candidate list as (flat index, value), and, where the
@@ -192,10 +192,9 @@ __device__ __forceinline__ unsigned* hist_of(const UpdateArgs& a, int g, int lev
 // The split W of tile ft (64 buckets) is 32 fragments of 1 KB,
 // [kb (4)][hi, lo][j (4)], lane (i, q) = (l % 16, l / 16) of a fragment holding
 // bucket 64 ft + 16 j + i, dims 32 kb + 8 q .. + 7 (an MFMA A operand), then
-// the buckets' biases and inverse scales, so that the encode's loop has no
-// other load that would wait behind the stores of the tile before.  It is
-// made once per call, by the sample kernel, and not in each encode workgroup:
-// that takes it off the encode's VALU, which its epilogue already fills.
+// the buckets' biases and inverse scales.  It is made once per call, by the
+// sample kernel, and not in each encode workgroup: that takes it off the
+// encode's VALU, which its epilogue already fills.
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -214,21 +213,21 @@ __device__ __forceinline__ float2 row_scale(float m) {
   return make_float2(__uint_as_float((unsigned)(127 + k) << 23), __uint_as_float((unsigned)(127 - k) << 23));
 }
 
-__device__ __forceinline__ void split8(const float (&x)[8], float scale, half8& hi, half8& lo) {
+template <typename Fn>
+__device__ __forceinline__ void split8(const float (&x)[8], Fn scaled, half8& hi, half8& lo) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float v = x[j] * scale;
+    const float v = scaled(x[j]);
     hi[j] = (_Float16)v;
     lo[j] = (_Float16)(v - (float)hi[j]);
   }
 }
 
-constexpr int kET = 512;                          // encode workgroup
-constexpr int kTB = 2;                            // 16-token blocks per wave
+constexpr int kET = 512;                          // sample and encode workgroups
+constexpr int kTB = 2;                            // sample: 16-token blocks per wave,
 constexpr int kRowTile = 16 * kTB;                // tokens per wave
-constexpr int kEncTokens = kET / 64 * kRowTile;   // tokens per workgroup (256)
-constexpr int kWLoads = kFT * kD * 4 / 16 / kET;  // 16-byte loads of a W tile per thread (4),
-constexpr int kWTail = kFT * 8 / 16;              // and of its biases and scales, by the first threads (32)
+constexpr int kSampleTile = kET / 64 * kRowTile;   // and per workgroup (256)
+constexpr int kWLoads = kFT * kD * 4 / 16 / kET;  // 16-byte words of a W tile's fragments per thread (4)
 constexpr int kWRows = kWTile * 2 / 16;           // 16-byte words of a tile
 constexpr int kJ = kFT / 16;                      // 16-bucket columns of a tile (4)
 
@@ -293,7 +292,7 @@ __device__ __forceinline__ bool split_rows(const RowsRaw<KT>& raw, half8 (&xh)[k
     xinv[tb] = s2.y;
     bad |= s2.y == 0.f;
 #pragma unroll
-    for (int kb = 0; kb < kKB; ++kb) split8(x[kb], s2.x, xh[tb][kb], xl[tb][kb]);
+    for (int kb = 0; kb < kKB; ++kb) split8(x[kb], [&](float v) { return v * s2.x; }, xh[tb][kb], xl[tb][kb]);
   }
   return __any(bad);
 }
@@ -420,7 +419,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
   const int y = blockIdx.x, ft = blockIdx.y, g = blockIdx.z, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   __shared__ __align__(16) u32x4 ws[kWRows];
   __shared__ unsigned hist[kSampleBins];
-  const int r0 = y * kEncTokens + w * kRowTile;  // the wave's first sample row
+  const int r0 = y * kSampleTile + w * kRowTile;  // the wave's first sample row
   const bool live = r0 < S;                      // uniform per wave
   int tok[kTB];
   RowsRaw<KT> raw;
@@ -453,7 +452,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
 #pragma unroll
     for (int kb = 0; kb < kKB; ++kb) {
       half8 hi, lo;
-      split8(x[kb], sc.x, hi, lo);
+      split8(x[kb], [&](float v) { return v * sc.x; }, hi, lo);
       lds[((kb * 2 + 0) * kJ + w) * 64] = hi;
       lds[((kb * 2 + 1) * kJ + w) * 64] = lo;
       if (y == 0) {
@@ -502,79 +501,127 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
 }
 
 // ---------------------------------------------------------------------------
-// encode: grid (ceil(N / 256), P, G) x 512.  Workgroup (y, part) takes the
-// tokens [256 y, 256 y + 256), wave w the 32 rows 256 y + 32 w + 16 tb + i, and
-// the bucket tiles part, part + P, ... (64 buckets each).  The wave's x is
-// computed and split once, into registers (64 of them), and each bucket tile's
-// split W streams through LDS, double-buffered: the next tile is requested into
-// registers while the current one is multiplied.  32 tokens per wave, because
-// a wave reads the whole 32 KB tile from LDS whatever its tokens: at 16 the 8
-// waves' reads took as long as their products.  P is chosen on the host
-// (encode_parts).
+// encode: grid (G, 6, R) x 512.  Workgroup (g, part, y) takes range y of the
+// group's tokens, whole 16-token steps, and wave w the bucket tile 8 part + w,
+// whose split W it holds in registers (128 of them) from start to end; the 47
+// tiles leave the last part's last wave to the splitting only.  The keys go
+// through LDS: 64 tokens at a time (a stage) are loaded, made x = (k - center) /
+// key_scale, split and written as MFMA operands, double-buffered, and every wave
+// multiplies the stage's four steps by its tile.  A group's workgroups lie 8
+// blocks apart, with 8 groups on one XCD, whose L2 then holds that group's W.
+//
+// The other way round (x in registers, W tiles streamed through LDS, a barrier
+// per tile) every wave read 32 KB of LDS per 96 MFMAs; here it is 16 KB, a
+// barrier per 192, and no load of the loop but the next stage's rows.  1024 /
+// 4096 keys with the activations stored: 38 / 121 us then, 35.5 / 111 now; 65536
+// without: 1.33 ms, now 1.17 (2.07 GHz under this load, 1.03 PFLOP/s; the
+// products alone took 0.90 ms, and a large f16 library product runs at 1.2).
+// Neither a higher priority for some of the waves nor the epilogue's values
+// placed one by one between the next step's products changed that.
 //
 // kCollect: the values at or above the group's floor, the lower edge of the
 // sample histogram's bin that holds the target-th largest value, go to the
 // candidate list: each wave gathers its own in LDS (places from a ballot, no
 // atomics) and moves them to a range of the list that it reserves with one
 // atomic; the workgroup's rest goes out together at the end.  An LDS histogram
-// of every positive value instead, 1024 per wave and tile on some thirty bins,
-// took longer than the products (64K keys, 8 groups: 3.0 ms and a 1.3 ms pass
-// over the stored activations; now 1.33 ms and no pass).  The products alone
-// take 0.90 ms of it (1.3 PFLOP/s; a large f16 library product reaches 1.2),
-// the epilogue's multiply-add, compare and branch per value the rest.
+// of every positive value instead took longer than the products.
 // kStore: every activation is written, one 16-byte store per lane and column.
 // Without kCollect the kernel is the dense path of a call that collects no
 // candidates, or whose list turned out unusable (else it returns at once).
 // ---------------------------------------------------------------------------
-constexpr int kWaveBuf = 512;  // candidates a wave gathers; a column of 4 values adds at most 256
+constexpr int kEW = kET / 64;                           // waves, a bucket tile each
+constexpr int kEParts = (kFTiles + kEW - 1) / kEW;      // 6
+constexpr int kStage = 64;                              // tokens split at a time
+constexpr int kSteps = kStage / 16;
+constexpr int kWaveBuf = 512;  // candidates a wave gathers
 
 template <typename KT, bool kStore, bool kCollect>
 __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
-  const int y = blockIdx.x, part = blockIdx.y, parts = gridDim.y, g = blockIdx.z, tid = threadIdx.x;
-  const int w = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
-  __shared__ __align__(16) u32x4 ws[2][kWRows];  // [buffer][a split W tile]
-  __shared__ uint2 cand[kCollect ? kET / 64 : 1][kCollect ? kWaveBuf : 1];
-  __shared__ unsigned wsum[kET / 64], floor_s, base_s;
+  const int g = blockIdx.x, part = blockIdx.y, y = blockIdx.z, ranges = gridDim.z, tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, lq = lane >> 4;
+  __shared__ __align__(16) half8 xs[2][kSteps * kKB * 2 * 64];  // [buffer][step][dim block][hi, lo][lane]
+  __shared__ __align__(16) float xinv[2][kStage];               // inverse scales; 0: a row that is not split
+  __shared__ __align__(16) float center[kD];
+  __shared__ uint2 cand[kCollect ? kEW : 1][kCollect ? kWaveBuf + 64 : 1];  // the wave's, and a dump per lane
+  __shared__ unsigned wsum[kEW], floor_s, base_s;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
   if constexpr (!kCollect)
     if (list_ok(a, g)) return;  // uniform
-  const int t0 = y * kEncTokens + w * kRowTile;  // the wave's first token
-  const bool live = t0 < a.N;                    // uniform per wave: a wave without tokens only moves W
-  const u32x4* wg = reinterpret_cast<const u32x4*>(a.wsplit + (size_t)g * kFTiles * kWTile);
-  auto load_w = [&](int ft, u32x4 (&r)[kWLoads + 1]) {
-#pragma unroll
-    for (int u = 0; u < kWLoads; ++u) r[u] = wg[(size_t)ft * kWRows + tid + kET * u];
-    r[kWLoads] = wg[(size_t)ft * kWRows + kET * kWLoads + (tid & (kWTail - 1))];
+  // the workgroup's tokens, the wave's bucket tile
+  const int blocks = (a.N + 15) / 16;
+  const int t0 = 16 * (int)((long long)blocks * y / ranges), t1 = min(a.N, 16 * (int)((long long)blocks * (y + 1) / ranges));
+  const int ft = part * kEW + w, f0 = ft * kFT + 4 * lq;
+  const bool live = ft < kFTiles;  // uniform per wave: the last part's last wave only splits rows
+  // rows of a stage: thread (row 8 w + l % 8, dims 16 (l / 8) .. + 15)
+  const int sr = 8 * w + (lane & 7), sp = lane >> 3;
+  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + 16 * sp;
+  const float scale = a.scale[g], rscale = 1.0f / scale;
+  // (the scale's own range bounds what divide_by may meet)
+  const bool scaled = fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
+  typename KeyLoad<KT>::Raw8 raw[2];
+  auto load_rows = [&](int t) {
+    const KT* p = kg + (size_t)(a.H + min(t + sr, a.N - 1)) * kD;
+    raw[0] = KeyLoad<KT>::raw8(p);
+    raw[1] = KeyLoad<KT>::raw8(p + 8);
   };
-  auto store_w = [&](int buf, const u32x4 (&r)[kWLoads + 1]) {
+  auto split_rows = [&](int buf) {
+    float x[2][8], m = 0.f;
 #pragma unroll
-    for (int u = 0; u < kWLoads; ++u) ws[buf][tid + kET * u] = r[u];
-    if (tid < kWTail) ws[buf][kET * kWLoads + tid] = r[kWLoads];
+    for (int h = 0; h < 2; ++h) {
+      const f32x4 c0 = *reinterpret_cast<const f32x4*>(center + 16 * sp + 8 * h);
+      const f32x4 c1 = *reinterpret_cast<const f32x4*>(center + 16 * sp + 8 * h + 4);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        x[h][t] = KeyLoad<KT>::at(raw[h], t) - (t < 4 ? c0[t & 3] : c1[t & 3]);
+        m = fmaxf(m, fabsf(x[h][t]));  // NaN is passed over: its sums are NaN either way
+      }
+    }
+    m = fmaxf(m, __shfl_xor(m, 8));
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    const float2 s2 = row_scale(fabsf(divide_by(m, scale, rscale)));  // the largest |x|; NaN for an infinite m
+    // (d / s) times the row's power of two: the quotient and its remainder scale exactly
+    const float rs = rscale * s2.x, ss = scale * s2.y;
+    half8* out = &xs[buf][((sr >> 4) * kKB + (sp >> 1)) * 2 * 64 + (2 * (sp & 1)) * 16 + (sr & 15)];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      half8 hi, lo;
+      split8(x[h], [&](float d) { return divide_by(d, ss, rs); }, hi, lo);
+      out[16 * h] = hi;
+      out[64 + 16 * h] = lo;
+    }
+    // (a quotient's remainder stays in the normal range)
+    if (sp == 0) xinv[buf][sr] = scaled && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
   };
-  // the part's bucket tiles: consecutive ones, whose stores meet in the lines of a token's row
-  const int first = part * kFTiles / parts, last = (part + 1) * kFTiles / parts;
-  u32x4 wr[kWLoads + 1];
-  load_w(first, wr);
-  half8 xh[kTB][kKB], xl[kTB][kKB];
-  float xinv[kTB];
-  int tok[kTB];
-  bool bad_rows = false;
-  if (live) {
-    RowsRaw<KT> raw;
+  load_rows(t0);
+  if (tid < kD) center[tid] = a.center[(size_t)g * kD + tid];
+  const _Float16* wt = a.wsplit + ((size_t)g * kFTiles + min(ft, kFTiles - 1)) * kWTile;
+  half8 wf[kKB][2][kJ];
 #pragma unroll
-    for (int tb = 0; tb < kTB; ++tb)
-      tok[tb] = min(t0 + 16 * tb + li, a.N - 1);  // rows past the block repeat the last one (masked below)
-    raw.load(a, g, tok);
-    bad_rows = split_rows<KT>(raw, xh, xl, xinv);
+  for (int kb = 0; kb < kKB; ++kb)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) wf[kb][p][j] = reinterpret_cast<const half8*>(wt)[((kb * 2 + p) * kJ + j) * 64 + lane];
+  f32x4 bias[kJ], winv[kJ];
+  bool bad_w = false;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const float* tail = reinterpret_cast<const float*>(wt + kFT * kD * 2) + 16 * j + 4 * lq;
+    bias[j] = *reinterpret_cast<const f32x4*>(tail);
+    winv[j] = *reinterpret_cast<const f32x4*>(tail + kFT);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bad_w |= winv[j][r] == 0.f;
   }
-  store_w(0, wr);
-  float least[kTB];  // the lane's floor per token: NaN (nothing is collected) for rows past the block
+  bad_w = __any(bad_w);
+  float least = 0.f;  // the floor
   if constexpr (kCollect) {
     // every workgroup reads the same histogram and puts its bins in order, in
-    // the buffer of the second W tile; then thread t has the 16 bins below 8192 - 16 t
+    // the buffer of the second stage; then thread t has the 16 bins below 8192 - 16 t
     constexpr int kPer = kSampleBins / kET;
+    static_assert(kSampleBins * sizeof(unsigned) <= sizeof(xs[1]), "room for the histogram");
     const uint4* sh = reinterpret_cast<const uint4*>(a.sample + (size_t)g * kSampleBins);
-    unsigned* ordered = reinterpret_cast<unsigned*>(ws[1]);
+    unsigned* ordered = reinterpret_cast<unsigned*>(xs[1]);
     uint4 h[kPer / 4];
 #pragma unroll
     for (int u = 0; u < kPer / 4; ++u) h[u] = sh[tid + kET * u];
@@ -609,27 +656,34 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     }
     __syncthreads();
     if (y == 0 && part == 0 && tid == 0) ctl[kFloor] = floor_s;
-#pragma unroll
-    for (int tb = 0; tb < kTB; ++tb) least[tb] = t0 + 16 * tb + li < a.N ? __uint_as_float(floor_s) : __builtin_nanf("");
+    least = __uint_as_float(floor_s);
   } else {
     __syncthreads();
   }
-  // the wave's activation rows; stores past them (rows past the block, buckets
-  // past F) carry an offset outside the resource and are dropped
-  const int rows = min(kRowTile, a.N - t0);
-  const __amdgpu_buffer_rsrc_t ar = raw_buffer(a.act + ((size_t)g * a.N + (live ? t0 : 0)) * kF,
-                                               kStore && live ? rows * kF * (int)sizeof(float) : 0);
+  split_rows(0);
+  // W is awaited here: left pending into the loop, its first use there waited in every
+  // step for the stores of the step before
+#pragma unroll
+  for (int kb = 0; kb < kKB; ++kb)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) asm volatile("" ::"v"(wf[kb][p][j]));
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) asm volatile("" ::"v"(bias[j]), "v"(winv[j]));
+  __syncthreads();
   uint2* list = a.list + (size_t)g * a.list_cap;
   unsigned n = 0u;  // the wave's gathered candidates (uniform)
   auto put = [&](unsigned at, unsigned i) {
     if (at + i < a.list_cap) list[at + i] = cand[kCollect ? w : 0][i];
   };
+  auto place = [&](unsigned long long m) {
+    return n + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+  };
   auto gather = [&](bool in, unsigned flat, float v) {
     const unsigned long long m = __ballot(in);
     if (m) {  // uniform
-      if (in)
-        cand[kCollect ? w : 0][n + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] =
-            make_uint2(flat, __float_as_uint(v));
+      if (in) cand[kCollect ? w : 0][place(m)] = make_uint2(flat, __float_as_uint(v));
       n += (unsigned)__popcll(m);
     }
   };
@@ -644,42 +698,100 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     n = 0u;
   };
   int buf = 0;
-  for (int ft = first; ft < last; ++ft) {  // uniform
-    const bool more = ft + 1 < last;
-    if (more) load_w(ft + 1, wr);  // in flight while this tile is multiplied
+  for (int t = t0; t < t1; t += kStage) {  // uniform
+    const bool more = t + kStage < t1;
+    if (more) load_rows(t + kStage);  // in flight while this stage is multiplied
+    // the stage's activation rows; stores past them (rows past the block, buckets
+    // past F) carry an offset outside the resource and are dropped
+    const __amdgpu_buffer_rsrc_t ar = raw_buffer(a.act + ((size_t)g * a.N + t) * kF,
+                                                 kStore ? min(kStage, t1 - t) * kF * (int)sizeof(float) : 0);
     if (live) {
-      const int f0 = ft * kFT;
-      f32x4 acc[kTB][kJ];
-      tile_products(ws[buf], xh, xl, acc);
-      // (a bucket past F has a zero row and bias: its 0 is below every floor)
-      tile_values<KT>(a, g, f0, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws[buf] + kET * kWLoads), acc,
-                      [&](int tb, int j, const float (&v)[4]) {
-        const int f = f0 + 16 * j + 4 * lq;
-        if constexpr (kStore) {  // relu; NaN is not positive
+#pragma unroll 1
+      for (int s = 0; s < kSteps && t + 16 * s < t1; ++s) {  // uniform
+        const int tok = t + 16 * s + li;
+        const half8* x = &xs[buf][s * kKB * 2 * 64 + lane];
+        half8 xh = x[0], xl = x[64];
+        f32x4 acc[kJ];
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < kKB; ++kb) {
+          // the next dim block's rows are requested before this one's products
+          const half8 yh = x[(kb + 1) % kKB * 2 * 64], yl = x[((kb + 1) % kKB * 2 + 1) * 64];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][1][j], xh, acc[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][0][j], xl, acc[j], 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][0][j], xh, acc[j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          xh = yh;
+          xl = yl;
+        }
+        const float inv = xinv[buf][16 * s + li];
+        const unsigned flat = (unsigned)tok * kF + (unsigned)f0;
+        if (bad_w || __any(inv == 0.f)) {  // uniform
+#pragma unroll 1
+          for (int e = 0; e < kJ * 4; ++e) {
+            const int f = 16 * (e >> 2) + (e & 3);
+            const bool in = tok < t1 && f0 + f < kF;
+            const float v = in ? exact_value<KT>(a, g, tok, f0 + f) : 0.f;
+            if constexpr (kStore)
+              if (in) a.act[(size_t)g * a.N * kF + flat + f] = v > 0.f ? v : 0.f;
+            if constexpr (kCollect) {
+              gather(in && v >= least, flat + (unsigned)f, v);
+              flush();
+            }
+          }
+          continue;
+        }
+        // the scales are powers of two: one rounding, that of the sum with the bias
+        float most = -INFINITY;
+        unsigned hits = 0u;
+        // NaN (nothing is collected) for rows past the range; a bucket past F has a
+        // zero row and bias: its 0 is below every floor
+        const float from = tok < t1 ? least : __builtin_nanf("");
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
           u32x4 p;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) p[r] = __float_as_uint(v[r] > 0.f ? v[r] : 0.f);
-          __builtin_amdgcn_raw_buffer_store_b128(
-              p, ar, f < kF ? (unsigned)(((16 * tb + li) * kF + f) * (int)sizeof(float)) : ~0u, 0, 0);
+          for (int r = 0; r < 4; ++r) {
+            const float v = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
+            acc[j][r] = v;
+            p[r] = __float_as_uint(v > 0.f ? v : 0.f);  // relu; NaN is not positive
+            // hits = 2 hits + (v >= from), in two instructions
+            if constexpr (kCollect)
+              asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(hits) : "v"(v), "v"(from) : "vcc");
+            most = fmaxf(most, v);
+          }
+          if constexpr (kStore)
+            __builtin_amdgcn_raw_buffer_store_b128(
+                p, ar, f0 + 16 * j < kF ? (unsigned)(((16 * s + li) * kF + f0 + 16 * j) * (int)sizeof(float)) : ~0u, 0, 0);
         }
         if constexpr (kCollect) {
+          // a lane's one candidate is its largest value
+          const bool one = hits != 0u && (hits & (hits - 1u)) == 0u;
+          const unsigned long long m = __ballot(one);
+          const unsigned e = (unsigned)__clz((int)hits) & 15u;  // bit 15 is the first value
+          cand[w][one ? place(m) : kWaveBuf + lane] = make_uint2(flat + 4u * (e & 12u) + (e & 3u), __float_as_uint(most));
+          n += (unsigned)__popcll(m);
+          const bool several = hits != 0u && !one;
+          if (__any(several)) {  // uniform
 #pragma unroll
-          for (int r = 0; r < 4; ++r) gather(v[r] >= least[tb], (unsigned)tok[tb] * kF + (unsigned)(f + r), v[r]);
+            for (int j = 0; j < kJ; ++j) {
+              flush();
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                gather(several && (hits >> (15 - 4 * j - r) & 1u), flat + (unsigned)(16 * j + r), acc[j][r]);
+            }
+          }
           flush();
         }
-      }, [&](int tb, int j, int r, float v) {
-        const int f = f0 + 16 * j + 4 * lq + r, t = tb ? tok[1] : tok[0];
-        const bool in = t0 + 16 * tb + li < a.N && f < kF;
-        if constexpr (kStore)
-          if (in) a.act[((size_t)g * a.N + t) * kF + f] = v > 0.f ? v : 0.f;
-        if constexpr (kCollect) {
-          gather(v >= (tb ? least[1] : least[0]), (unsigned)t * kF + (unsigned)f, v);
-          flush();
-        }
-      });
+      }
     }
-    if (more) {  // the other buffer was last read before the previous barrier
-      store_w(buf ^ 1, wr);
+    if (more) {
+      split_rows(buf ^ 1);  // last read before the previous barrier
       __syncthreads();
       buf ^= 1;
     }
@@ -690,7 +802,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     __syncthreads();
     if (tid == 0) {
       unsigned total = 0u;
-      for (int i = 0; i < kET / 64; ++i) total += wsum[i];
+      for (int i = 0; i < kEW; ++i) total += wsum[i];
       base_s = total ? atomicAdd(&ctl[kListLen], total) : 0u;
     }
     __syncthreads();
@@ -1730,29 +1842,30 @@ static UpdateArgs make_args(uint64_t k, uint64_t W, uint64_t b, uint64_t center,
   return a;
 }
 
-// Bucket-tile parts of an encode over `rows` (token tiles x groups) workgroups
-// per part: one workgroup runs per CU, so a launch takes ceil(rows P / 256)
-// rounds of ceil(47 / P) tiles each plus about two tiles' time to load and
-// split its keys; the P of the least total.
-static int encode_parts(int rows) {
-  int best = 1;
-  long long least = -1;
-  for (int p = 1; p <= kFTiles; ++p) {
-    const long long cost = ((long long)rows * p + 255) / 256 * ((kFTiles + p - 1) / p + 2);
+// Token ranges R of an encode: one workgroup runs per CU, so a launch takes
+// rounds of 256 of its 6 G R workgroups, each its 16-token steps plus about six
+// steps' time to load its W, find the floor and split its first rows; of the
+// R that fill 1 .. 8 rounds the one of the least total.
+static int encode_ranges(int N, int groups) {
+  const long long blocks = (N + 15) / 16, per = (long long)groups * kEParts;
+  long long best = 1, least = -1;
+  for (int q = 1; q <= 8; ++q) {
+    const long long r = std::min(blocks, std::max(1ll, 256ll * q / per));
+    const long long cost = (per * r + 255) / 256 * ((blocks + r - 1) / r + 6);
     if (least < 0 || cost < least) {
       least = cost;
-      best = p;
+      best = r;
     }
   }
-  return best;
+  return (int)best;
 }
 
 // Sample tokens of a call over N keys: every key up to 128, 128 of up to 2048
 // (each of the 47 tiles' workgroups splits their rows again), 256 of up to
 // 16384, 1/64 beyond, at most 2048.
 static int sample_tokens(int N) {
-  if (N <= 2048) return std::min(N, kEncTokens / 2);
-  return std::min(2048, std::max(kEncTokens, N / 64 / kEncTokens * kEncTokens));
+  if (N <= 2048) return std::min(N, kSampleTile / 2);
+  return std::min(2048, std::max(kSampleTile, N / 64 / kSampleTile * kSampleTile));
 }
 
 // sample .. emit: the exact batch-wide positive Top-k of the N keys' activations
@@ -1766,9 +1879,8 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
   const int S = a.listed ? sample_tokens(a.N) : 0;
   const bool one = a.listed && a.N <= kSelectMax;
   a.target = (unsigned)((one ? 4 : 3) * ((long long)S * (a.budget / a.N)) / 2);
-  const int token_tiles = (a.N + kEncTokens - 1) / kEncTokens;
-  const dim3 grid(token_tiles, encode_parts(token_tiles * groups), groups);
-  hipLaunchKernelGGL(sample_kernel<KT>, dim3(std::max(1, (S + kEncTokens - 1) / kEncTokens), kFTiles, groups),
+  const dim3 grid(groups, kEParts, encode_ranges(a.N, groups));
+  hipLaunchKernelGGL(sample_kernel<KT>, dim3(std::max(1, (S + kSampleTile - 1) / kSampleTile), kFTiles, groups),
                      dim3(kET), 0, s, a, S);
   if (a.listed && keep) {
     hipLaunchKernelGGL((encode_kernel<KT, true, true>), grid, dim3(kET), 0, s, a);

@@ -103,3 +103,25 @@ def test_encode_rows_and_buckets_that_are_not_split():
     assert torch.equal(act[5, rows, 2999], torch.where(x[rows] > 0, float("inf"), 0.0))
     rest = [r for r in range(290) if r not in (7, 40, 41)]
     check(k, W, b, center, scale, act, rows=rest, buckets=[f for f in range(F) if f != 2999])
+
+
+@pytest.mark.parametrize("block", [16, 17, 63, 65, 80, 81, 129, 1023, 1041, 2000])
+def test_encode_steps_and_stages(block):
+    # token ranges of whole 16-token steps, rows split 64 at a time: blocks that end inside either
+    k, W, b, center, scale = inputs(block, 900 + block)
+    op, act = run_append(k, W, b, center, scale, block)
+    check(k, W, b, center, scale, act)
+    assert int(op.n.sum()) == G * 8 * block
+
+
+@pytest.mark.parametrize("exponent", [-59, -40, 40, 59])
+def test_encode_key_scales(exponent):
+    # the row's power of two is folded into the division by the key scale; where the
+    # divisor would leave the normal range the plain fp32 chains take over
+    k, W, b, center, scale = inputs(100, 33)
+    center.zero_()
+    k[:, H:] = (k[:, H:].float() * 2.0 ** exponent).to(torch.bfloat16)
+    k[:, H + 1::4] = (k[:, H + 1::4].float() * 2.0 ** (exponent // 2)).to(torch.bfloat16)
+    scale = scale * 2.0 ** exponent
+    _, act = run_append(k, W, b, center, scale, 100)
+    check(k, W, b, center, scale, act)
