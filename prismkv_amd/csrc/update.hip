@@ -224,9 +224,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], Fn scaled, half8& hi
 }
 
 constexpr int kET = 512;                          // sample and encode workgroups
-constexpr int kTB = 2;                            // sample: 16-token blocks per wave,
-constexpr int kRowTile = 16 * kTB;                // tokens per wave
-constexpr int kSampleTile = kET / 64 * kRowTile;   // and per workgroup (256)
+constexpr int kSampleFew = kET / 64 * 16;         // sample tokens per workgroup at 16 per wave (128); at 32, twice as many
 constexpr int kWLoads = kFT * kD * 4 / 16 / kET;  // 16-byte words of a W tile's fragments per thread (4)
 constexpr int kWRows = kWTile * 2 / 16;           // 16-byte words of a tile
 constexpr int kJ = kFT / 16;                      // 16-bucket columns of a tile (4)
@@ -234,7 +232,7 @@ constexpr int kJ = kFT / 16;                      // 16-bucket columns of a tile
 // The wave's key rows and its center, as loaded: lane (i, q) takes dims
 // 32 kb + 8 q .. + 7 of its own tokens.  All of it is requested before any is
 // used, so the split below waits for one memory round trip.
-template <typename KT>
+template <typename KT, int kTB>
 struct RowsRaw {
   typename KeyLoad<KT>::Raw8 k[kTB][kKB];
   f32x4 c[kKB][2];
@@ -269,8 +267,8 @@ __device__ __forceinline__ float divide_by(float d, float s, float r) {
 // The split x = (k - center) / key_scale (fp32, core.py:98) of the wave's
 // tokens.  xinv: the inverse of each row's scale; returns whether a row of the
 // wave is not split.
-template <typename KT>
-__device__ __forceinline__ bool split_rows(const RowsRaw<KT>& raw, half8 (&xh)[kTB][kKB], half8 (&xl)[kTB][kKB],
+template <typename KT, int kTB>
+__device__ __forceinline__ bool split_rows(const RowsRaw<KT, kTB>& raw, half8 (&xh)[kTB][kKB], half8 (&xl)[kTB][kKB],
                                            float (&xinv)[kTB]) {
   const float s = raw.scale, rs = 1.0f / s;
   // (the scale's own range bounds what divide_by may meet)
@@ -301,6 +299,7 @@ __device__ __forceinline__ bool split_rows(const RowsRaw<KT>& raw, half8 (&xh)[k
 // v_mfma_f32_16x16x32_f16, lane (i, q) feeding A[i][8 q + t] and B[8 q + t][i],
 // t = 0..7, and holding D[4 q + r][i].  A is W (bucket rows), B is x (token
 // columns), so lane (i, q) ends with buckets 16 j + 4 q + r of token i.
+template <int kTB>
 __device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)[kTB][kKB], const half8 (&xl)[kTB][kKB],
                                               f32x4 (&acc)[kTB][kJ]) {
   const half8* wt = reinterpret_cast<const half8*>(ws) + (threadIdx.x & 63);
@@ -353,7 +352,7 @@ __device__ float exact_value(const UpdateArgs& a, int g, int tok, int f) {
 // four(tb, j, v) gets lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3,
 // in rolled form one(tb, j, r, v) where a row or bucket is not split.  `tok` is
 // the lane's two tokens; sg the tile's biases, then its inverse bucket scales.
-template <typename KT, typename Four, typename One>
+template <typename KT, int kTB, typename Four, typename One>
 __device__ __forceinline__ void tile_values(const UpdateArgs& a, int g, int f0, const int (&tok)[kTB],
                                             const float (&xinv)[kTB], bool bad_rows, const float* sg,
                                             const f32x4 (&acc)[kTB][kJ], Four four, One one) {
@@ -384,7 +383,7 @@ __device__ __forceinline__ void tile_values(const UpdateArgs& a, int g, int f0, 
 #pragma unroll 1
     for (int e = 0; e < kTB * kJ * 4; ++e) {
       const int tb = e >> 4, j = (e >> 2) & 3, f = f0 + 16 * j + 4 * lq + (e & 3);
-      one(tb, j, e & 3, f < kF ? exact_value<KT>(a, g, tb ? tok[1] : tok[0], f) : 0.f);
+      one(tb, j, e & 3, f < kF ? exact_value<KT>(a, g, tb ? tok[kTB - 1] : tok[0], f) : 0.f);
     }
   }
 }
@@ -405,7 +404,7 @@ static_assert((kPlace * kPlaceInverse) % kSampleBins == 1u, "inverse places");
 __device__ __forceinline__ unsigned sample_place(unsigned bin) { return bin * kPlace % kSampleBins; }
 
 // ---------------------------------------------------------------------------
-// sample: grid (max(ceil(S / 256), 1), kFTiles, G) x 512.  Splits bucket tile
+// sample: grid (max(ceil(S / (128 kTB)), 1), kFTiles, G) x 512.  Splits bucket tile
 // ft of W (the first token tile's workgroups write it for the encode), and adds
 // to the group's histogram, for each of S sample tokens and each 16 buckets of
 // the tile (a lane's), the largest activation if it is positive.  Around tau a
@@ -414,15 +413,15 @@ __device__ __forceinline__ unsigned sample_place(unsigned bin) { return bin * kP
 // for 188 at most, and the floor stays one that serves the others.  S = 0 only
 // splits.
 // ---------------------------------------------------------------------------
-template <typename KT>
+template <typename KT, int kTB>
 __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
   const int y = blockIdx.x, ft = blockIdx.y, g = blockIdx.z, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   __shared__ __align__(16) u32x4 ws[kWRows];
-  __shared__ unsigned hist[kSampleBins];
-  const int r0 = y * kSampleTile + w * kRowTile;  // the wave's first sample row
+  __shared__ __align__(16) unsigned hist[kSampleBins];
+  const int r0 = y * kSampleFew * kTB + w * 16 * kTB;  // the wave's first sample row
   const bool live = r0 < S;                      // uniform per wave
   int tok[kTB];
-  RowsRaw<KT> raw;
+  RowsRaw<KT, kTB> raw;
   if (live) {
 #pragma unroll
     for (int tb = 0; tb < kTB; ++tb) tok[tb] = sample_token(min(r0 + 16 * tb + (lane & 15), S - 1), S, a.N);
@@ -477,17 +476,19 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
   half8 xh[kTB][kKB], xl[kTB][kKB];
   float xinv[kTB];
   bool bad_rows = false;
-  if (live) bad_rows = split_rows<KT>(raw, xh, xl, xinv);
+  if (live) bad_rows = split_rows<KT, kTB>(raw, xh, xl, xinv);
   __syncthreads();
   if (live) {
     f32x4 acc[kTB][kJ];
     tile_products(ws, xh, xl, acc);
-    float most[kTB] = {0.f, 0.f};
-    tile_values<KT>(a, g, ft * kFT, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws + kET * kWLoads), acc,
+    float most[kTB];
+#pragma unroll
+    for (int tb = 0; tb < kTB; ++tb) most[tb] = 0.f;
+    tile_values<KT, kTB>(a, g, ft * kFT, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws + kET * kWLoads), acc,
                     [&](int tb, int j, const float (&v)[4]) {
       most[tb] = fmaxf(most[tb], fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
     }, [&](int tb, int j, int r, float v) {
-      if (tb) most[1] = fmaxf(most[1], v); else most[0] = fmaxf(most[0], v);
+      if (tb) most[kTB - 1] = fmaxf(most[kTB - 1], v); else most[0] = fmaxf(most[0], v);
     });
 #pragma unroll
     for (int tb = 0; tb < kTB; ++tb)
@@ -496,8 +497,16 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
   }
   __syncthreads();
   unsigned* sh = a.sample + (size_t)g * kSampleBins;
-  for (int i = tid; i < kSampleBins; i += kET)
-    if (hist[i]) atomicAdd(&sh[sample_place(i)], hist[i]);
+#pragma unroll
+  for (int u = 0; u < kSampleBins / 4 / kET; ++u) {
+    const int i = 4 * (tid + kET * u);
+    const u32x4 c = *reinterpret_cast<const u32x4*>(&hist[i]);
+    if (c[0] | c[1] | c[2] | c[3]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c[e]) atomicAdd(&sh[sample_place(i + e)], c[e]);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -513,7 +522,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
 // The other way round (x in registers, W tiles streamed through LDS, a barrier
 // per tile) every wave read 32 KB of LDS per 96 MFMAs; here it is 16 KB, a
 // barrier per 192, and no load of the loop but the next stage's rows.  1024 /
-// 4096 keys with the activations stored: 38 / 121 us then, 35.5 / 111 now; 65536
+// 4096 keys with the activations stored: 38 / 121 us then, 35 / 109 now; 65536
 // without: 1.33 ms, now 1.17 (2.07 GHz under this load, 1.03 PFLOP/s; the
 // products alone took 0.90 ms, and a large f16 library product runs at 1.2).
 // Neither a higher priority for some of the waves nor the epilogue's values
@@ -697,6 +706,14 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     __builtin_amdgcn_wave_barrier();
     n = 0u;
   };
+  const unsigned flat0 = (unsigned)li * kF + (unsigned)f0;
+  // The lane's offsets in a step's rows; 2^31 is outside.  (The step's own part is
+  // added to them and not given as the instruction's scalar offset: four-word
+  // stores with one lost their last word to the vector instruction that
+  // followed, which the compiler takes to need no wait.)
+  unsigned column[kJ];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) column[j] = f0 + 16 * j < kF ? (flat0 + 16u * j) * (unsigned)sizeof(float) : 1u << 31;
   int buf = 0;
   for (int t = t0; t < t1; t += kStage) {  // uniform
     const bool more = t + kStage < t1;
@@ -711,6 +728,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
         const int tok = t + 16 * s + li;
         const half8* x = &xs[buf][s * kKB * 2 * 64 + lane];
         half8 xh = x[0], xl = x[64];
+        const float inv = xinv[buf][16 * s + li];
         f32x4 acc[kJ];
 #pragma unroll
         for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -729,8 +747,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
           xh = yh;
           xl = yl;
         }
-        const float inv = xinv[buf][16 * s + li];
-        const unsigned flat = (unsigned)tok * kF + (unsigned)f0;
+        const unsigned flat = flat0 + (unsigned)(t + 16 * s) * kF;
         if (bad_w || __any(inv == 0.f)) {  // uniform
 #pragma unroll 1
           for (int e = 0; e < kJ * 4; ++e) {
@@ -766,8 +783,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
             most = fmaxf(most, v);
           }
           if constexpr (kStore)
-            __builtin_amdgcn_raw_buffer_store_b128(
-                p, ar, f0 + 16 * j < kF ? (unsigned)(((16 * s + li) * kF + f0 + 16 * j) * (int)sizeof(float)) : ~0u, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(p, ar, column[j] + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
         }
         if constexpr (kCollect) {
           // a lane's one candidate is its largest value
@@ -1860,12 +1876,12 @@ static int encode_ranges(int N, int groups) {
   return (int)best;
 }
 
-// Sample tokens of a call over N keys: every key up to 128, 128 of up to 2048
-// (each of the 47 tiles' workgroups splits their rows again), 256 of up to
-// 16384, 1/64 beyond, at most 2048.
+// Sample tokens of a call over N keys: every key up to 128, 128 of up to 4096
+// (the count at the floor is then good to a few percent, whatever N is), 256 of
+// up to 16384, 1/64 beyond, at most 2048.
 static int sample_tokens(int N) {
-  if (N <= 2048) return std::min(N, kSampleTile / 2);
-  return std::min(2048, std::max(kSampleTile, N / 64 / kSampleTile * kSampleTile));
+  if (N <= kSelectMax) return std::min(N, kSampleFew);
+  return std::min(2048, std::max(2 * kSampleFew, N / 64 / (2 * kSampleFew) * (2 * kSampleFew)));
 }
 
 // sample .. emit: the exact batch-wide positive Top-k of the N keys' activations
@@ -1880,8 +1896,14 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
   const bool one = a.listed && a.N <= kSelectMax;
   a.target = (unsigned)((one ? 4 : 3) * ((long long)S * (a.budget / a.N)) / 2);
   const dim3 grid(groups, kEParts, encode_ranges(a.N, groups));
-  hipLaunchKernelGGL(sample_kernel<KT>, dim3(std::max(1, (S + kSampleTile - 1) / kSampleTile), kFTiles, groups),
-                     dim3(kET), 0, s, a, S);
+  // 16 tokens per wave while that is one workgroup per tile: all 8 waves share the
+  // rows' splitting, where 32 left it to four (1024 keys: 19.5 us, now 14); beyond,
+  // 32, as every workgroup splits its W tile again
+  if (S <= kSampleFew)
+    hipLaunchKernelGGL((sample_kernel<KT, 1>), dim3(1, kFTiles, groups), dim3(kET), 0, s, a, S);
+  else
+    hipLaunchKernelGGL((sample_kernel<KT, 2>), dim3((S + 2 * kSampleFew - 1) / (2 * kSampleFew), kFTiles, groups), dim3(kET),
+                       0, s, a, S);
   if (a.listed && keep) {
     hipLaunchKernelGGL((encode_kernel<KT, true, true>), grid, dim3(kET), 0, s, a);
   } else {
