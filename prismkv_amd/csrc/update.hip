@@ -32,10 +32,13 @@
 //            read off the sample (about twice the budget of them) go to the
 //            group's candidate list as (flat index, value), and, where the
 //            caller reads them, all of them to [G][N][F];
-//   select   one workgroup per group finds tau, the budget-th largest value,
-//            in the list and, when ties at tau overflow the budget, the flat
-//            index of the last one taken;
-//   emit     sets the members' bitmap bits;
+//   split    finds the digit of the candidates' values that holds tau, the
+//            budget-th largest (the encode has counted them): the candidates
+//            above it are members, whose bitmap bits it sets, those in it go to
+//            a short list;
+//   select   one workgroup per group finds tau in that list and, when ties at
+//            tau overflow the budget, the flat index of the last one taken, and
+//            sets the rest of the bits;
 //   moments  per 32-bucket tile: new members from the bitmap, two-pass
 //            moments of their keys, merge, counts += new.
 // The sample decides only how long the list is.  Where it misjudged (fewer
@@ -48,7 +51,7 @@
 // The build runs the same selection over all H keys of a group (in batches
 // of groups, so the activations of one batch fit the workspace) after a
 // center pass and a bitmap clear, with select's work spread over many
-// workgroups for long histories (histogram / digit / refine, three levels),
+// workgroups for long histories (histogram / digit / refine, three levels, emit),
 // and computes every bucket's moments from scratch (build_moments: one
 // workgroup per bucket, any member count).  Unless the caller keeps them, a
 // build never writes its activations (12 KB per key) at all.
@@ -74,6 +77,7 @@ constexpr unsigned kListSlack = 1u << 18;  // list entries beyond kListPerKey pe
 constexpr int kListPerKey = 48;
 constexpr int kSampleShift = 18, kSampleBins = 1 << (31 - kSampleShift);  // 13-bit digits of positive floats: 3.1% each
 constexpr int kSelectMax = 4096;  // keys up to which one workgroup per group selects
+constexpr int kFineShift = 12;     // the candidates' own digits: 2^12 bit patterns each (0.05%), kBins of them from the floor on
 constexpr int kMaxBuild = 1 << 20;   // keys per group of a build (N * F < 2^32 flat indices)
 constexpr int kBuildCenter = 1;      // prismkv_build flag: compute the center (else it is an input)
 constexpr int kBuildNoAct = 4;       // prismkv_build flag: the activations need not be left in the workspace
@@ -149,6 +153,7 @@ struct UpdateArgs {
   unsigned list_cap;  // entries per group
   unsigned target;    // sample values at or above the floor, at least
   int listed;         // whether the call collects candidates
+  int fine;           // whether the encode counts them in fine digits (hist level 0), for split_kernel
   int H, N;          // first key row / bitmap column, keys indexed
   long long budget;  // N * key_mean
   int tie_blocks;
@@ -172,6 +177,10 @@ __device__ __forceinline__ bool list_ok(const UpdateArgs& a, int g) {
 
 __device__ __forceinline__ unsigned* hist_of(const UpdateArgs& a, int g, int level) {
   return a.hist + ((size_t)g * kLevels + level) * kRep * kBins;
+}
+
+__device__ __forceinline__ unsigned fine_digit(unsigned u, unsigned floor) {
+  return min((u - floor) >> kFineShift, (unsigned)kBins - 1u);
 }
 
 // ---------------------------------------------------------------------------
@@ -470,7 +479,10 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
       }
     }
   }
-  if (y == 0 && ft == 0 && tid == 0) a.ctl[(size_t)g * kCtl + kListLen] = 0u;
+  if (y == 0 && ft == 0 && tid == 0) {
+    a.ctl[(size_t)g * kCtl + kListLen] = 0u;
+    a.ctl[(size_t)g * kCtl + kTieLen] = 0u;
+  }
   if (S == 0) return;  // uniform
   for (int i = tid; i < kSampleBins; i += kET) hist[i] = 0u;
   half8 xh[kTB][kKB], xl[kTB][kKB];
@@ -552,6 +564,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   __shared__ __align__(16) float xinv[2][kStage];               // inverse scales; 0: a row that is not split
   __shared__ __align__(16) float center[kD];
   __shared__ uint2 cand[kCollect ? kEW : 1][kCollect ? kWaveBuf + 64 : 1];  // the wave's, and a dump per lane
+  __shared__ unsigned fine[kCollect ? kBins : 1];  // the candidates' fine digits
   __shared__ unsigned wsum[kEW], floor_s, base_s;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
   if constexpr (!kCollect)
@@ -654,6 +667,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       }
     }
     if (tid == 0) floor_s = 1u;  // too few positive values in the sample: every one is collected
+    for (int i = tid; i < kBins; i += kET) fine[i] = 0u;
     unsigned run = block_incl_scan<kET>(tot, wsum) - tot;
     if (run < a.target && run + tot >= a.target) {
 #pragma unroll
@@ -684,7 +698,9 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   uint2* list = a.list + (size_t)g * a.list_cap;
   unsigned n = 0u;  // the wave's gathered candidates (uniform)
   auto put = [&](unsigned at, unsigned i) {
-    if (at + i < a.list_cap) list[at + i] = cand[kCollect ? w : 0][i];
+    const uint2 e = cand[kCollect ? w : 0][i];
+    if (at + i < a.list_cap) list[at + i] = e;
+    if (a.fine) atomicAdd(&fine[kCollect ? fine_digit(e.y, floor_s) : 0u], 1u);
   };
   auto place = [&](unsigned long long m) {
     return n + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
@@ -825,6 +841,12 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     unsigned at = base_s;
     for (int i = 0; i < w; ++i) at += wsum[i];
     for (unsigned i = lane; i < n; i += 64) put(at, i);
+    if (a.fine) {  // uniform
+      __syncthreads();
+      unsigned* hg = hist_of(a, g, 0);
+      for (int i = tid; i < kBins; i += kET)
+        if (fine[i]) atomicAdd(&hg[i], fine[i]);
+    }
   }
 }
 
@@ -1005,19 +1027,56 @@ __device__ __forceinline__ Found find_digit(const unsigned* hist, int bins, unsi
   return f;
 }
 
+__device__ __forceinline__ void set_member(const UpdateArgs& a, int g, unsigned flat) {
+  const int tok = (int)(flat / kF), f = (int)(flat % kF);
+  const int t = a.H + tok;
+  atomicOr(a.bits + ((size_t)g * kF + f) * a.row_words + (t >> 5), 1u << (t & 31));
+}
+
 // ---------------------------------------------------------------------------
-// select: grid G x 1024, calls of up to kSelectMax keys: tau and the cut of its
-// ties in one launch, where the levels of hist0 / digit / refine and the tie
-// kernels are nine of about 4.5 us each.  One pass over the list counts 13-bit
-// digits, a second gathers tau's bin (3% of tau wide: about a fifth of the
-// budget) in LDS, where the other 18 bits and the flat indices of the ties are
-// searched: 13.5 us at 1024 keys, 30 at 4096 (16384 keys took 127: there the
-// levels' own launches, over 256 workgroups per group, are the better ones).
-// A bin that does not fit (ties by the thousand), or a list that
-// cannot be used, is searched by passes over the list or the activations.
+// Calls of up to kSelectMax keys take their members in two launches: split and
+// select.  The encode has counted the candidates in fine digits, so split, grid
+// (kSplitBlocks, G) x 256, knows the digit of tau: the candidates above it are
+// members, whose bits it sets, and the few in it (0.4% of the budget where
+// activations are normal) go to a list of their own.  select, grid G x 1024, finds
+// tau and the cut of its ties among those, in LDS, and sets the rest of the bits.
+// (One workgroup that read the whole list twice and an emit launch: 18.5 us at
+// 1024 keys, 41.5 at 4096, bound by its one CU; now 12.5 and 22.  64 or
+// 128 split workgroups per group were no faster: 8 and 9 us for 7, 16 and 18 for 16.)
+// A digit that does not fit (ties by the thousand) or that the counts do not
+// reach, or a list that cannot be used: select takes all of it, by passes over
+// the list or the activations.  Beyond kSelectMax those passes would be too long
+// for one workgroup, and hist0 / digit / refine and the tie kernels, over 256
+// workgroups per group, are the better ones.
 // ---------------------------------------------------------------------------
 constexpr int kST = 1024;
 constexpr int kSelBuf = 8192;
+constexpr int kSplitBlocks = 32;
+
+// The fine digit of the budget-th largest candidate; false if split and select
+// cannot work with it.
+template <int NT>
+__device__ __forceinline__ bool find_fine(const UpdateArgs& a, int g, unsigned* wsum, Found* out, Found& f) {
+  if (threadIdx.x == 0) *out = Found{(unsigned)kBins - 1u, 0u, ~0u};
+  f = find_digit<NT>(hist_of(a, g, 0), kBins, budget_of(a), wsum, out);
+  return list_ok(a, g) && f.digit < (unsigned)kBins - 1u && f.ties <= (unsigned)kSelBuf;
+}
+
+__global__ __launch_bounds__(kUT) void split_kernel(UpdateArgs a) {
+  const int g = blockIdx.y;
+  __shared__ unsigned wsum[kUT / 64];
+  __shared__ Found found;
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  Found f;
+  if (!find_fine<kUT>(a, g, wsum, &found, f)) return;  // uniform
+  const unsigned floor = ctl[kFloor];
+  uint2* ties = reinterpret_cast<uint2*>(a.ties + (size_t)g * a.list_cap);
+  each_value<kUT>(a, g, true, blockIdx.x, gridDim.x, [&](unsigned u, unsigned flat) {
+    const unsigned d = fine_digit(u, floor);
+    if (d > f.digit) set_member(a, g, flat);
+    if (d == f.digit) ties[atomicAdd(&ctl[kTieLen], 1u)] = make_uint2(flat, u);
+  });
+}
 
 __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
   const int g = blockIdx.x, tid = threadIdx.x;
@@ -1030,81 +1089,95 @@ __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
   const unsigned count = budget_of(a);
   for (int i = tid; i < kSampleBins; i += kST) a.sample[(size_t)g * kSampleBins + i] = 0u;  // for the next call
   if (tid == 0) nbin = 0u;
-  // The listed values lie within a few octaves above the floor, 32 digits each,
-  // so they are counted in kRel digits from the floor's on, 8 replicas of each
-  // (64 lanes meet in some 25 digits: one replica took 15 us of atomics for the
-  // list of 4096 keys); a value beyond them, or an unlisted call, in all 8192.
-  constexpr unsigned kRel = kSampleBins / 8;
   Found f;
-  unsigned npos = 0u;
-  for (bool rel = listed;; rel = false) {  // uniform
-    const unsigned base = rel ? ctl[kFloor] >> kSampleShift : 0u;
+  const bool split = find_fine<kST>(a, g, wsum, &found, f);
+  for (int i = tid; i < kBins; i += kST) hist_of(a, g, 0)[i] = 0u;  // for the next call
+  unsigned prefix;
+  bool gathered = true;
+  if (split) {
+    const uint2* ties = reinterpret_cast<const uint2*>(a.ties + (size_t)g * a.list_cap);
+    for (unsigned i = tid; i < f.ties; i += kST) bin[i] = ties[i];
+    if (tid == 0) nbin = f.ties;
+    for (int i = tid; i < (1 << kFineShift); i += kST) hist[i] = 0u;
     __syncthreads();
-    for (int i = tid; i < kSampleBins; i += kST) hist[i] = 0u;
+    const unsigned base = ctl[kFloor] + (f.digit << kFineShift);
+    for (unsigned i = tid; i < nbin; i += kST) atomicAdd(&hist[bin[i].y - base], 1u);
     __syncthreads();
-    each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned) {
-      const unsigned d = (u >> kSampleShift) - base;
-      atomicAdd(&hist[rel ? 8u * min(d, kRel - 1u) + (tid & 7) : d], 1u);
-    });
-    __syncthreads();
-    if (rel) {
-      unsigned c = 0u;
-      if (tid < (int)kRel)
-#pragma unroll
-        for (int r = 0; r < 8; ++r) c += hist[8 * tid + r];
+    f = find_digit<kST>(hist, 1 << kFineShift, f.rem, wsum, &found);
+    prefix = base + f.digit;
+  } else {
+    // The listed values lie within a few octaves above the floor, 32 digits each,
+    // so they are counted in kRel digits from the floor's on, 8 replicas of each
+    // (64 lanes meet in some 25 digits: one replica took 15 us of atomics for the
+    // list of 4096 keys); a value beyond them, or an unlisted call, in all 8192.
+    constexpr unsigned kRel = kSampleBins / 8;
+    unsigned npos = 0u;
+    for (bool rel = listed;; rel = false) {  // uniform
+      const unsigned base = rel ? ctl[kFloor] >> kSampleShift : 0u;
       __syncthreads();
-      if (tid < (int)kRel) hist[tid] = c;
+      for (int i = tid; i < kSampleBins; i += kST) hist[i] = 0u;
       __syncthreads();
-    }
-    const int bins = rel ? (int)kRel : kSampleBins;
-    npos = 0u;
-    for (int i = tid; i < bins; i += kST) npos += hist[i];
-    block_incl_scan<kST>(npos, wsum);
-    npos = 0u;
-    for (int i = 0; i < kST / 64; ++i) npos += wsum[i];
-    __syncthreads();
-    if (npos < count) {  // fewer positives than the budget: every one is kept (core.py:22-26)
-      if (tid == 0) {
-        ctl[kTau] = 0u;
-        ctl[kCut] = 0u;
-      }
-      return;
-    }
-    f = find_digit<kST>(hist, bins, count, wsum, &found);
-    if (!rel) break;
-    if (f.digit < kRel - 1u) {
-      f.digit += base;
-      break;
-    }
-  }
-  const unsigned top = f.digit;
-  const bool gathered = f.ties <= (unsigned)kSelBuf;
-  if (gathered) {
-    each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
-      if ((u >> kSampleShift) == top) bin[atomicAdd(&nbin, 1u)] = make_uint2(flat, u);
-    });
-    __syncthreads();
-  }
-  // counts the digit (key >> shift) & mask of the values of tau's bin for which in(u, flat)
-  auto count_digits = [&](int bins, auto in, auto digit) {
-    for (int i = tid; i < bins; i += kST) hist[i] = 0u;
-    __syncthreads();
-    if (gathered) {
-      for (unsigned i = tid; i < nbin; i += kST)
-        if (in(bin[i].y)) atomicAdd(&hist[digit(bin[i].y, bin[i].x)], 1u);
-    } else {
-      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
-        if (in(u)) atomicAdd(&hist[digit(u, flat)], 1u);
+      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned) {
+        const unsigned d = (u >> kSampleShift) - base;
+        atomicAdd(&hist[rel ? 8u * min(d, kRel - 1u) + (tid & 7) : d], 1u);
       });
+      __syncthreads();
+      if (rel) {
+        unsigned c = 0u;
+        if (tid < (int)kRel)
+#pragma unroll
+          for (int r = 0; r < 8; ++r) c += hist[8 * tid + r];
+        __syncthreads();
+        if (tid < (int)kRel) hist[tid] = c;
+        __syncthreads();
+      }
+      const int bins = rel ? (int)kRel : kSampleBins;
+      npos = 0u;
+      for (int i = tid; i < bins; i += kST) npos += hist[i];
+      block_incl_scan<kST>(npos, wsum);
+      npos = 0u;
+      for (int i = 0; i < kST / 64; ++i) npos += wsum[i];
+      __syncthreads();
+      if (npos < count) {  // fewer positives than the budget: every one is kept (core.py:22-26)
+        each_value<kST>(a, g, listed, 0, 1, [&](unsigned, unsigned flat) { set_member(a, g, flat); });
+        return;
+      }
+      f = find_digit<kST>(hist, bins, count, wsum, &found);
+      if (!rel) break;
+      if (f.digit < kRel - 1u) {
+        f.digit += base;
+        break;
+      }
     }
-    __syncthreads();
-  };
-  unsigned prefix = top;
-  for (int shift = 9; shift >= 0; shift -= 9) {
-    count_digits(512, [&](unsigned u) { return (u >> (shift + 9)) == prefix; },
-                 [&](unsigned u, unsigned) { return (u >> shift) & 511u; });
-    f = find_digit<kST>(hist, 512, f.rem, wsum, &found);
-    prefix = (prefix << 9) | f.digit;
+    const unsigned top = f.digit;
+    gathered = f.ties <= (unsigned)kSelBuf;
+    if (gathered) {
+      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
+        if ((u >> kSampleShift) == top) bin[atomicAdd(&nbin, 1u)] = make_uint2(flat, u);
+      });
+      __syncthreads();
+    }
+    // counts the digit (key >> shift) & mask of the values of tau's bin for which in(u, flat)
+    auto count_digits = [&](int bins, auto in, auto digit) {
+      for (int i = tid; i < bins; i += kST) hist[i] = 0u;
+      __syncthreads();
+      if (gathered) {
+        for (unsigned i = tid; i < nbin; i += kST)
+          if (in(bin[i].y)) atomicAdd(&hist[digit(bin[i].y, bin[i].x)], 1u);
+      } else {
+        each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
+          if (in(u)) atomicAdd(&hist[digit(u, flat)], 1u);
+        });
+      }
+      __syncthreads();
+    };
+    prefix = top;
+    for (int shift = 9; shift >= 0; shift -= 9) {
+      count_digits(512, [&](unsigned u) { return (u >> (shift + 9)) == prefix; },
+                   [&](unsigned u, unsigned) { return (u >> shift) & 511u; });
+      f = find_digit<kST>(hist, 512, f.rem, wsum, &found);
+      prefix = (prefix << 9) | f.digit;
+    }
   }
   unsigned cut = ~0u;
   if (f.ties > f.rem) {  // the rem-th smallest flat index of the ties = the rem-th largest complement
@@ -1131,16 +1204,13 @@ __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
     }
     cut = ~key;
   }
-  if (tid == 0) {
-    ctl[kTau] = prefix;
-    ctl[kCut] = cut;
-  }
-}
-
-__device__ __forceinline__ void set_member(const UpdateArgs& a, int g, unsigned flat) {
-  const int tok = (int)(flat / kF), f = (int)(flat % kF);
-  const int t = a.H + tok;
-  atomicOr(a.bits + ((size_t)g * kF + f) * a.row_words + (t >> 5), 1u << (t & 31));
+  auto emit = [&](unsigned u, unsigned flat) {
+    if (u > prefix || (u == prefix && flat <= cut)) set_member(a, g, flat);
+  };
+  if (split)
+    for (unsigned i = tid; i < nbin; i += kST) emit(bin[i].y, bin[i].x);
+  else
+    each_value<kST>(a, g, listed, 0, 1, emit);
 }
 
 // ---------------------------------------------------------------------------
@@ -1844,6 +1914,7 @@ static UpdateArgs make_args(uint64_t k, uint64_t W, uint64_t b, uint64_t center,
   a.sample = reinterpret_cast<unsigned*>(w + L.sample);
   a.ties = reinterpret_cast<unsigned*>(w + L.ties);
   a.listed = 0;
+  a.fine = 0;
   a.target = 0;
   a.H = H;
   a.N = N;
@@ -1894,6 +1965,7 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
   a.listed = 3 * a.budget <= (long long)a.list_cap;
   const int S = a.listed ? sample_tokens(a.N) : 0;
   const bool one = a.listed && a.N <= kSelectMax;
+  a.fine = one;
   a.target = (unsigned)((one ? 4 : 3) * ((long long)S * (a.budget / a.N)) / 2);
   const dim3 grid(groups, kEParts, encode_ranges(a.N, groups));
   // 16 tokens per wave while that is one workgroup per tile: all 8 waves share the
@@ -1911,6 +1983,7 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
     hipLaunchKernelGGL((encode_kernel<KT, true, false>), grid, dim3(kET), 0, s, a);
   }
   if (one) {
+    hipLaunchKernelGGL(split_kernel, dim3(kSplitBlocks, groups), dim3(kUT), 0, s, a);
     hipLaunchKernelGGL(select_kernel, dim3(groups), dim3(kST), 0, s, a);
   } else {
     hipLaunchKernelGGL(hist0_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
@@ -1921,8 +1994,8 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
     }
     hipLaunchKernelGGL(tie_count_kernel, dim3(kTieGrid, groups), dim3(kUT), 0, s, a);
     hipLaunchKernelGGL(tie_cut_kernel, dim3(groups), dim3(kST), 0, s, a);
+    hipLaunchKernelGGL(emit_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
   }
-  hipLaunchKernelGGL(emit_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
 }
 
 template <typename KT>

@@ -132,3 +132,31 @@ def test_summarize_reads_rows_of_any_alignment():
     v = (on @ (x * x)) / c.clamp_min(1)[:, None] - m * m
     tiles = tile_moments(m[None].float(), v[None].float())
     assert torch.allclose(moments, tiles, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("first,second", [("ties", "plain"), ("wide", "plain"), ("plain", "wide")])
+def test_append_after_append(first, second):
+    # each call leaves the counts of its candidates' digits cleared for the next, whichever
+    # way it took: thousands of ties in one digit, or values beyond the digits' octave
+    from prismkv_amd import Native8B
+    block = 1100
+    k, W, b, center, scale = inputs(2 * block, 3)
+    for i, kind in enumerate((first, second)):
+        rows = slice(H + i * block, H + (i + 1) * block)
+        if kind == "ties":
+            k[:, rows] = k[:, H:H + 1]
+        if kind == "wide":  # half the tokens scaled by 2^0 .. 2^12
+            k[:, H + i * block:H + (i + 1) * block:2] *= 2.0 ** torch.randint(0, 13, (block // 2, 1), device="cuda")
+    zeros = torch.zeros(G, F, dtype=torch.int64, device="cuda")
+    op = Native8B.from_tables(H, zeros, torch.zeros(G, F, D, device="cuda"), torch.zeros(G, F, D, device="cuda"),
+                              torch.zeros(G, 1, dtype=torch.int32, device="cuda"),
+                              torch.zeros(G, F + 1, dtype=torch.int32, device="cuda"), center=center,
+                              capacity=H + 2 * block)
+    op.set_encoder_tables(W, b, scale, 8)
+    for i in range(2):
+        op.append(k[:, :H + (i + 1) * block], block)
+        act = op.update_activations(block)
+        got = membership(op, H + i * block, block)
+        for g in range(G):
+            want = oracle.positive_global_topk(act[g].cpu().numpy(), 8 * block)
+            assert np.array_equal(np.sort(want), got[g].cpu().numpy()), (i, g)
