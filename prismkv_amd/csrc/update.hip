@@ -1566,39 +1566,47 @@ __global__ __launch_bounds__(kUT) void clear_bits_kernel(UpdateArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// build_moments: grid (F, G) x 256, one workgroup per bucket f, any member
+// build_moments: grid (F, G) x NT, one workgroup per bucket f, any member
 // count.  Members are the set bits of the bucket's bitmap row below N (a
 // build indexes K rows = bitmap columns [0, N)).  The row is compacted into an
 // LDS token list, 2048 words (64K keys) requested at once; a list of more than
 // kList tokens is rebuilt 64 words at a time in each pass.  Workgroup x takes
 // bucket 375 (x % 8) + x / 8: consecutive workgroups go to the 8 XCDs in turn,
 // so each XCD works through consecutive buckets and its L2 joins their 4-byte
-// columns of the moment tiles before they are written back.  Thread = (member slot tid >> 4 of 16, dims 8 (tid & 15)
-// ..), double accumulation, fixed order: the slots of a wave by shuffles, then
-// the 4 waves.  The first 192 members (a 64K build has 175 on average; 96 of
-// fp32) are requested together and kept packed in registers, so the second pass reads
-// no memory.  mean = sum / n rounded to fp32; var = sum (x - mean)^2 / n
+// columns of the moment tiles before they are written back.  Thread = (member
+// slot tid >> 4, dims 8 (tid & 15) ..), double accumulation, fixed order: the
+// slots of a wave by shuffles, then the waves.  The first 192 members of 256
+// threads (a 64K build has 175 on average; 96 of fp32) are requested together and
+// kept packed in registers, so the second pass reads no memory.  Up to kSmallBuild keys a workgroup is one wave (four member slots,
+// a list of 512 tokens): a bucket then has so few members that the launch is
+// bound by the chain of its 24,000 workgroups' loads, and four times as many of
+// them are in flight; longer buckets are left to build_moments_rest_kernel.  256
+// against 64 threads, 8 groups: 136 / 52 us at 6000 keys, 158 / 87 at 16384, 190
+// / 159 at 32768, 282 / 331 at 65536 (and 5 us for the other launch).
+// mean = sum / n rounded to fp32; var = sum (x - mean)^2 / n
 // with that rounded mean; empty bucket -> 0 (core.py:84-88).  Counts and
 // moments are written, not merged.
 // ---------------------------------------------------------------------------
 constexpr int kList = 2048;
-constexpr int kSlots = kUT / 16;
+constexpr int kSmallBuild = 32768;  // keys up to which a bucket is one wave's
 template <typename KT>
 constexpr int kKeep = sizeof(KT) == 2 ? 12 : 6;  // members per slot kept in registers (48 of them)
 
+template <int NT>
 struct BuildMomentsLds {
-  int toks[kList];
-  double red[kUT / 64][kD];
-  unsigned wsum[kUT / 64];
+  static constexpr int kLen = NT == 64 ? kList / 4 : kList;  // of the token list
+  int toks[kLen];
+  double red[NT / 64][kD];
+  unsigned wsum[NT / 64];
   float mean[kD];
 };
 
-// Members among words [w0, w0 + 256 W) of the row below word w1, W consecutive
+// Members among words [w0, w0 + NT W) of the row below word w1, W consecutive
 // words per thread (8: the row is 16-byte aligned, as a build's is and a
 // caller's of summarize need not be) ->
-// toks[at ..] when they all fit below kList.  Returns their count (uniform);
+// toks[at ..] when they all fit below kLen.  Returns their count (uniform);
 // the caller barriers before the list is read and before the next chunk.
-template <int W>
+template <int NT, int W>
 __device__ __forceinline__ unsigned compact_chunk(const uint32_t* row, int w0, int w1, int N, int* toks, unsigned at,
                                                   unsigned* wsum) {
   const int wd = w0 + W * (int)threadIdx.x, nw = (N + 31) >> 5;
@@ -1622,9 +1630,11 @@ __device__ __forceinline__ unsigned compact_chunk(const uint32_t* row, int w0, i
     if (wd + i == nw - 1 && (N & 31)) m[i] &= (1u << (N & 31)) - 1u;
     pc += (unsigned)__popc(m[i]);
   }
-  const unsigned incl = block_incl_scan<kUT>(pc, wsum);
-  const unsigned total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-  if (at + total <= (unsigned)kList) {
+  const unsigned incl = block_incl_scan<NT>(pc, wsum);
+  unsigned total = 0u;
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) total += wsum[i];
+  if (at + total <= (unsigned)BuildMomentsLds<NT>::kLen) {
     unsigned p = at + incl - pc;
 #pragma unroll
     for (int i = 0; i < W; ++i)
@@ -1642,8 +1652,9 @@ __device__ __forceinline__ double xor_d(double v) {
   return __longlong_as_double((long long)(((unsigned long long)y << 32) | x));
 }
 
-// One pass's order-fixed sum over the slots: of dim tid for tid < kD.
-__device__ __forceinline__ double slot_sum(BuildMomentsLds& L, double (&acc)[8]) {
+// One pass's order-fixed sum over the slots, into red[0].
+template <int NT>
+__device__ __forceinline__ void slot_sum(BuildMomentsLds<NT>& L, double (&acc)[8]) {
   const int tid = threadIdx.x, lane = tid & 63;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -1654,17 +1665,17 @@ __device__ __forceinline__ double slot_sum(BuildMomentsLds& L, double (&acc)[8])
 #pragma unroll
     for (int j = 0; j < 8; ++j) L.red[tid >> 6][8 * lane + j] = acc[j];
   __syncthreads();
-  const double t = tid < kD ? (L.red[0][tid] + L.red[1][tid]) + (L.red[2][tid] + L.red[3][tid]) : 0.0;
-  __syncthreads();  // red is free again
-  return t;
+  if constexpr (NT > 64) {
+    static_assert(NT == 256, "four waves");
+    if (tid < kD) L.red[0][tid] = (L.red[0][tid] + L.red[1][tid]) + (L.red[2][tid] + L.red[3][tid]);
+    __syncthreads();
+  }
 }
 
-template <typename KT>
-__global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
-  static_assert(kF % 8 == 0, "buckets in 8 equal runs");
-  const int f = (int)(blockIdx.x & 7u) * (kF / 8) + (int)(blockIdx.x >> 3), g = blockIdx.y;
+template <typename KT, int NT>
+__device__ __forceinline__ void bucket_moments(const UpdateArgs& a, int g, int f, BuildMomentsLds<NT>& L) {
+  constexpr int kSlots = NT / 16, kLen = BuildMomentsLds<NT>::kLen;
   const int tid = threadIdx.x, slot = tid >> 4, d0 = (tid & 15) * 8;
-  __shared__ BuildMomentsLds L;
   typedef KeyLoad<KT> KL;
   const uint32_t* row = a.bits + ((size_t)g * kF + f) * a.row_words;
   const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + d0;
@@ -1673,13 +1684,16 @@ __global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
   unsigned n = 0;
   bool listed = true;
   const bool wide = ((a.row_words & 3) | (int64_t)(reinterpret_cast<uintptr_t>(a.bits) & 15u)) == 0;
-  for (int w0 = 0; w0 < nw; w0 += wide ? 8 * kUT : kUT) {  // uniform
-    const unsigned c = wide ? compact_chunk<8>(row, w0, nw, a.N, L.toks, n, L.wsum)
-                            : compact_chunk<1>(row, w0, nw, a.N, L.toks, n, L.wsum);
-    listed = listed && n + c <= (unsigned)kList;
+  for (int w0 = 0; w0 < nw; w0 += wide ? 8 * NT : NT) {  // uniform
+    const unsigned c = wide ? compact_chunk<NT, 8>(row, w0, nw, a.N, L.toks, n, L.wsum)
+                            : compact_chunk<NT, 1>(row, w0, nw, a.N, L.toks, n, L.wsum);
+    listed = listed && n + c <= (unsigned)kLen;
     __syncthreads();
     n += c;
   }
+  if (tid == 0) a.counts[(size_t)g * kFP + f] = (int)n;
+  if constexpr (NT == 64)
+    if (!listed) return;  // uniform: build_moments_rest_kernel's
   auto key_row = [&](unsigned i) { return KL::raw8(kg + (size_t)L.toks[i] * kD); };
   typename KL::Raw8 kept[kKeep<KT>];
   if (listed)
@@ -1697,9 +1711,9 @@ __global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
 #pragma unroll 4
       for (unsigned i = slot + kSlots * kKeep<KT>; i < n; i += kSlots) add(key_row(i));
     } else {
-      for (int w0 = 0; w0 < nw; w0 += kList / 32) {
+      for (int w0 = 0; w0 < nw; w0 += kLen / 32) {
         __syncthreads();  // the previous chunk's list has been read
-        const unsigned c = compact_chunk<1>(row, w0, min(nw, w0 + kList / 32), a.N, L.toks, 0u, L.wsum);  // always fits
+        const unsigned c = compact_chunk<NT, 1>(row, w0, min(nw, w0 + kLen / 32), a.N, L.toks, 0u, L.wsum);  // always fits
         __syncthreads();
 #pragma unroll 4
         for (unsigned i = slot; i < c; i += kSlots) add(key_row(i));
@@ -1710,8 +1724,8 @@ __global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] += (double)KL::at(r, j);
   });
-  const double sum = slot_sum(L, acc);
-  if (tid < kD) L.mean[tid] = n ? (float)(sum / (double)n) : 0.f;
+  slot_sum(L, acc);
+  for (int d = tid; d < kD; d += NT) L.mean[d] = n ? (float)(L.red[0][d] / (double)n) : 0.f;
   __syncthreads();
   float m[8];
 #pragma unroll
@@ -1723,14 +1737,36 @@ __global__ __launch_bounds__(kUT, 4) void build_moments_kernel(UpdateArgs a) {
       acc[j] += t * t;
     }
   });
-  const double dev = slot_sum(L, acc);
-  if (tid < kD) {
-    float* tile = a.moments + (size_t)(g * kChunks + f / kChunk) * kRow * kChunk;
-    const int col = f % kChunk;
-    tile[tid * kChunk + col] = L.mean[tid];
-    tile[(kD + tid) * kChunk + col] = n ? (float)(dev / (double)n) : 0.f;
+  slot_sum(L, acc);
+  float* tile = a.moments + (size_t)(g * kChunks + f / kChunk) * kRow * kChunk;
+  const int col = f % kChunk;
+  for (int d = tid; d < kD; d += NT) {
+    tile[d * kChunk + col] = L.mean[d];
+    tile[(kD + d) * kChunk + col] = n ? (float)(L.red[0][d] / (double)n) : 0.f;
   }
-  if (tid == 0) a.counts[(size_t)g * kFP + f] = (int)n;
+}
+
+template <typename KT, int NT>
+__global__ __launch_bounds__(NT, 4) void build_moments_kernel(UpdateArgs a) {
+  static_assert(kF % 8 == 0, "buckets in 8 equal runs");
+  __shared__ BuildMomentsLds<NT> L;
+  bucket_moments<KT, NT>(a, blockIdx.y, (int)(blockIdx.x & 7u) * (kF / 8) + (int)(blockIdx.x >> 3), L);
+}
+
+// Grid (kRestBlocks, G) x 256: the buckets of more members than a one-wave
+// workgroup lists.
+constexpr int kRestBlocks = 64;
+template <typename KT>
+__global__ __launch_bounds__(kUT, 4) void build_moments_rest_kernel(UpdateArgs a) {
+  __shared__ BuildMomentsLds<kUT> L;
+  const int g = blockIdx.y;
+  static_assert((kF + kRestBlocks - 1) / kRestBlocks <= 64, "a lane per bucket");
+  const int mine = (int)blockIdx.x + kRestBlocks * (int)(threadIdx.x & 63);
+  unsigned long long heavy = __ballot(mine < kF && a.counts[(size_t)g * kFP + min(mine, kF - 1)] > BuildMomentsLds<64>::kLen);
+  for (; heavy; heavy &= heavy - 1ull) {  // uniform
+    bucket_moments<KT, kUT>(a, g, (int)blockIdx.x + kRestBlocks * (int)__builtin_ctzll(heavy), L);
+    __syncthreads();  // the list and the sums are free again
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1999,6 +2035,15 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
 }
 
 template <typename KT>
+static void launch_build_moments(const UpdateArgs& a, int groups, hipStream_t s) {
+  if (a.N <= kSmallBuild) {
+    hipLaunchKernelGGL((build_moments_kernel<KT, 64>), dim3(kF, groups), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(build_moments_rest_kernel<KT>, dim3(kRestBlocks, groups), dim3(kUT), 0, s, a);
+  } else
+    hipLaunchKernelGGL((build_moments_kernel<KT, kUT>), dim3(kF, groups), dim3(kUT), 0, s, a);
+}
+
+template <typename KT>
 static bool aligned16(uint64_t p, int64_t stride_elems) {
   return ((p | (uint64_t)(stride_elems * (int64_t)sizeof(KT))) & 15u) == 0;
 }
@@ -2054,7 +2099,7 @@ static int build_impl(uint64_t k, uint64_t W, uint64_t b, uint64_t center, uint6
     }
     hipLaunchKernelGGL(clear_bits_kernel, dim3(512, nb), dim3(kUT), 0, s, a);
     launch_selection<KT>(a, nb, !(flags & kBuildNoAct), s);
-    hipLaunchKernelGGL(build_moments_kernel<KT>, dim3(kF, nb), dim3(kUT), 0, s, a);
+    launch_build_moments<KT>(a, nb, s);
   }
   return (int)hipGetLastError();
 }
@@ -2077,7 +2122,7 @@ static int summarize_impl(uint64_t k, uint64_t bits, uint64_t center, uint64_t c
     hipLaunchKernelGGL(center_final_kernel, dim3(groups), dim3(kD), 0, s, a, (const double*)part,
                        reinterpret_cast<float*>(center));
   }
-  hipLaunchKernelGGL(build_moments_kernel<KT>, dim3(kF, groups), dim3(kUT), 0, s, a);
+  launch_build_moments<KT>(a, groups, s);
   return (int)hipGetLastError();
 }
 

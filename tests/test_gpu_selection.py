@@ -160,3 +160,21 @@ def test_append_after_append(first, second):
         for g in range(G):
             want = oracle.positive_global_topk(act[g].cpu().numpy(), 8 * block)
             assert np.array_equal(np.sort(want), got[g].cpu().numpy()), (i, g)
+
+
+@pytest.mark.parametrize("history,heavy", [(6000, 511), (6000, 513), (32768, 2100), (32769, 2100), (40000, 16385)])
+def test_build_heavy_buckets(history, heavy):
+    # buckets around the lengths of the token lists, beside ordinary ones: a wave's list
+    # of 512 (up to 32768 keys), a workgroup's of 2048, and none
+    from prismkv_amd import Native8B
+    gen = torch.Generator(device="cuda").manual_seed(heavy)
+    k = torch.randn(G, history, D, generator=gen, device="cuda").to(torch.bfloat16)
+    k[:, :, 0] = 0
+    k[:, :heavy, 0] = 64.0
+    W = torch.randn(G, F, D, generator=gen, device="cuda") / D ** 0.5
+    W[:, 5::1000] = 0
+    W[:, 5::1000, 0] = 8.0  # far above the others for the first `heavy` keys, 0 for the rest
+    op = Native8B.from_keys(k, history, W, torch.zeros(G, F, device="cuda"), torch.ones(G), 8)
+    torch.cuda.synchronize()
+    assert (op.n[:, 5:F:1000] >= heavy).all()
+    check_moments(op, k, membership(op, 0, history))
