@@ -273,6 +273,13 @@ __device__ __forceinline__ float divide_by(float d, float s, float r) {
   return fmaf(fmaf(-q, s, d), r, q);
 }
 
+// d / s by divide_by for any d and a finite s >= 1: where d is infinite or NaN
+// (an infinite key, squares past fp32) the division's own result, which the
+// remainder would make NaN, by one more instruction.
+__device__ __forceinline__ float quotient(float d, float s, float r) {
+  return __builtin_amdgcn_div_fixupf(divide_by(d, s, r), s, d);
+}
+
 // The split x = (k - center) / key_scale (fp32, core.py:98) of the wave's
 // tokens.  xinv: the inverse of each row's scale; returns whether a row of the
 // wave is not split.
@@ -1369,15 +1376,15 @@ constexpr int kMomCols = kChunk / (kMT / 64);  // buckets per wave (4)
 
 // The update's merge (core.py:194-199) for bucket sizes a (old) and b (block),
 // den = max(a + b, 1): every rounding of (a x + b y) / den + ..., with the
-// quotients by divide_by.
+// quotients by quotient().
 __device__ __forceinline__ float merge_mean(float a, float b, float den, float rden, float ma, float mb) {
 #pragma clang fp contract(off)
-  return divide_by(a * ma + b * mb, den, rden);
+  return quotient(a * ma + b * mb, den, rden);
 }
 __device__ __forceinline__ float merge_var(float a, float b, float den, float rden, float ab, float ma, float mb, float va,
                                            float vb) {
 #pragma clang fp contract(off)
-  const float v = divide_by(a * va + b * vb, den, rden);
+  const float v = quotient(a * va + b * vb, den, rden);
   const float d = ma - mb;
   return v + ab * (d * d);
 }
@@ -1464,14 +1471,14 @@ __global__ __launch_bounds__(kMT, 6) void moments_kernel(UpdateArgs a) {
         for (int u = 0; u < kMomRound; ++u)
           if (u < b) sum(kept[u]);
         pass(kMomRound, b, sum);
-        m0 = divide_by(m0, n, rn);
-        m1 = divide_by(m1, n, rn);
+        m0 = quotient(m0, n, rn);
+        m1 = quotient(m1, n, rn);
 #pragma unroll
         for (int u = 0; u < kMomRound; ++u)
           if (u < b) dev(kept[u]);
         pass(kMomRound, b, dev);
-        v0 = divide_by(v0, n, rn);
-        v1 = divide_by(v1, n, rn);
+        v0 = quotient(v0, n, rn);
+        v1 = quotient(v1, n, rn);
       }
     } else {  // 16 words (at most 512 members) at a time, once for each pass
       b = 0;
@@ -1482,12 +1489,12 @@ __global__ __launch_bounds__(kMT, 6) void moments_kernel(UpdateArgs a) {
       }
       if (b > 0) {
         const float n = (float)b, rn = 1.0f / n;
-        m0 = divide_by(m0, n, rn);
-        m1 = divide_by(m1, n, rn);
+        m0 = quotient(m0, n, rn);
+        m1 = quotient(m1, n, rn);
         for (int w0 = w_lo; w0 <= w_hi; w0 += 16) 
           pass(0, list_words(lane < 16 ? word(j, w0 + lane) : 0u, w0, 0), dev);
-        v0 = divide_by(v0, n, rn);
-        v1 = divide_by(v1, n, rn);
+        v0 = quotient(v0, n, rn);
+        v1 = quotient(v1, n, rn);
       }
     }
     const int o = w * kMomCols + j;
