@@ -86,6 +86,15 @@ constexpr int kBuildNoAct = 4;       // prismkv_build flag: the activations need
 enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kFloor, kListLen, kCut, kTieLen, kCtl = 16 };
 enum { kModeTopK = 0, kModeAllPositive = 1 };
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ f32x2 load_f2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int base) {
+  const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, base, 0);
+  return f32x2{__uint_as_float(v[0]), __uint_as_float(v[1])};
+}
+
 // Key loads of the two key element types: 2 or 8 consecutive dims as the
 // raw loaded bits (kept packed while in flight) and their fp32 values.
 template <typename KT>
@@ -94,8 +103,8 @@ struct KeyLoad;
 template <>
 struct KeyLoad<uint16_t> {  // bf16
   typedef uint32_t Raw2;
-  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, 0, 0);
+  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int base = 0) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, byte_offset, base, 0);
   }
   static __device__ __forceinline__ float lo(Raw2 r) { return bf16_lo(r); }
   static __device__ __forceinline__ float hi(Raw2 r) { return bf16_hi(r); }
@@ -112,8 +121,8 @@ struct KeyLoad<uint16_t> {  // bf16
 template <>
 struct KeyLoad<float> {
   typedef unsigned Raw2 __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset) {
-    return __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, 0, 0);
+  static __device__ __forceinline__ Raw2 load2(__amdgpu_buffer_rsrc_t r, unsigned byte_offset, int base = 0) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, byte_offset, base, 0);
   }
   static __device__ __forceinline__ float lo(Raw2 r) { return __uint_as_float(r[0]); }
   static __device__ __forceinline__ float hi(Raw2 r) { return __uint_as_float(r[1]); }
@@ -196,7 +205,7 @@ __device__ __forceinline__ unsigned fine_digit(unsigned u, unsigned floor) {
 // to [2^14, 2^15), so nothing overflows f16 and what underflows is below 2^-39
 // of that largest one.  A row or bucket that is not finite, or whose largest
 // magnitude lies outside 2^+-60 (the scales' products would leave fp32), is
-// not split: its values are computed by plain fp32 chains (exact_value).
+// not split: its values are computed by fp32 MFMA (fp32_products).
 //
 // The split W of tile ft (64 buckets) is 32 fragments of 1 KB,
 // [kb (4)][hi, lo][j (4)], lane (i, q) = (l % 16, l / 16) of a fragment holding
@@ -205,7 +214,6 @@ __device__ __forceinline__ unsigned fine_digit(unsigned u, unsigned floor) {
 // sample kernel, and not in each encode workgroup: that takes it off the
 // encode's VALU, which its epilogue already fills.
 // ---------------------------------------------------------------------------
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int kScaleExp = 14;   // scaled rows have their largest magnitude in [2^14, 2^15)
 constexpr int kMaxScale = 60;   // |exponent| of a row's or bucket's largest magnitude, at most
@@ -350,56 +358,73 @@ __device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)
   }
 }
 
-// relu(x . w + b) of key row `tok` of the block and bucket f by one fp32 chain:
-// rows and buckets that the split does not serve.
+// The products of 16 tokens (`tok`, the lane's) with the buckets f0 .. f0 + 63 in
+// fp32, for rows and buckets that the split does not serve: v_mfma_f32_16x16x4f32
+// (lane (i, q) feeding A[i][q] and B[q][i], and holding D[4 q + r][i]), four dims
+// 16 kb + 4 q .. of its row per block.  Straight from memory: W comes from L2 for
+// each 16 tokens, 32 KB per wave against 128 MFMAs of 32 cycles, which the MFMAs
+// still bound.  (One fp32 chain per lane and value: a 64-token append whose tile
+// held one infinite key took 822 us, and 63 without it.)
 template <typename KT>
-__device__ float exact_value(const UpdateArgs& a, int g, int tok, int f) {
-  const KT* k = static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)(a.H + tok) * kD;
-  const float* w = a.W + ((size_t)g * kF + f) * kD;
-  const float* c = a.center + (size_t)g * kD;
-  const float sc = a.scale[g];
-  float s = 0.f;
+__device__ __forceinline__ void fp32_products(const UpdateArgs& a, int g, int tok, int f0, f32x4 (&acc)[kJ]) {
+  const int li = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
+  // (as buffers: one offset register each, and zeros for buckets past F)
+  const __amdgpu_buffer_rsrc_t kr = raw_buffer(static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)a.H * kD,
+                                               a.N * kD * (int)sizeof(KT));
+  const __amdgpu_buffer_rsrc_t cr = raw_buffer(a.center + (size_t)g * kD, kD * (int)sizeof(float));
+  const __amdgpu_buffer_rsrc_t wr = raw_buffer(a.W + (size_t)g * kF * kD, kF * kD * (int)sizeof(float));
+  const unsigned ko = ((unsigned)tok * kD + 4 * lq) * (unsigned)sizeof(KT);
+  const unsigned co = 4 * lq * (unsigned)sizeof(float), wo = ((unsigned)(f0 + li) * kD + 4 * lq) * (unsigned)sizeof(float);
+  const float s = a.scale[g];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-  for (int d = 0; d < kD; ++d) s = fmaf((to_f32(k[d]) - c[d]) / sc, w[d], s);
-  return s + a.b[(size_t)g * kF + f];
+  for (int e = 0; e < kD / 8; ++e) {  // two of the block's four dims at a time
+    const int d = 16 * (e >> 1) + 2 * (e & 1);
+    f32x2 wv[kJ];
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) wv[j] = load_f2(wr, wo, (16 * j * kD + d) * (int)sizeof(float));
+    const f32x2 m = load_f2(cr, co, d * (int)sizeof(float));
+    const typename KeyLoad<KT>::Raw2 r = KeyLoad<KT>::load2(kr, ko, d * (int)sizeof(KT));
+    const float x[2] = {(KeyLoad<KT>::lo(r) - m[0]) / s, (KeyLoad<KT>::hi(r) - m[1]) / s};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][t], x[t], acc[j], 0, 0, 0);
+  }
 }
 
-// The values of one bucket tile for the wave's tokens, after the products:
-// four(tb, j, v) gets lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3,
-// in rolled form one(tb, j, r, v) where a row or bucket is not split.  `tok` is
-// the lane's two tokens; sg the tile's biases, then its inverse bucket scales.
-template <typename KT, int kTB, typename Four, typename One>
+// The values of one bucket tile for the wave's 16 kTB tokens, after the products
+// (made again in fp32 where a row or bucket is not split): four(tb, j, v) gets
+// lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3.  `tok` is the lane's
+// kTB tokens; sg the tile's biases, then its inverse bucket scales.
+template <typename KT, int kTB, typename Four>
 __device__ __forceinline__ void tile_values(const UpdateArgs& a, int g, int f0, const int (&tok)[kTB],
                                             const float (&xinv)[kTB], bool bad_rows, const float* sg,
-                                            const f32x4 (&acc)[kTB][kJ], Four four, One one) {
+                                            f32x4 (&acc)[kTB][kJ], Four four) {
   const int lq = (threadIdx.x >> 4) & 3;
   float4 bias[kJ], winv[kJ];
-  bool bad_w = false;
+  bool bad = bad_rows;
 #pragma unroll
   for (int j = 0; j < kJ; ++j) {
     const int o = 16 * j + 4 * lq;
     bias[j] = *reinterpret_cast<const float4*>(sg + o);
     winv[j] = *reinterpret_cast<const float4*>(sg + kFT + o);
-    bad_w |= winv[j].x == 0.f || winv[j].y == 0.f || winv[j].z == 0.f || winv[j].w == 0.f;
+    bad |= winv[j].x == 0.f || winv[j].y == 0.f || winv[j].z == 0.f || winv[j].w == 0.f;
   }
-  if (!bad_rows && !__any(bad_w)) {
+  bad = __any(bad);
 #pragma unroll
-    for (int tb = 0; tb < kTB; ++tb)
+  for (int tb = 0; tb < kTB; ++tb) {
+    if (bad) fp32_products<KT>(a, g, tok[tb], f0, acc[tb]);  // uniform
 #pragma unroll
-      for (int j = 0; j < kJ; ++j) {
-        const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
-        const float s4[4] = {winv[j].x, winv[j].y, winv[j].z, winv[j].w};
-        float v[4];
-        // the scales are powers of two: one rounding, that of the sum with the bias
+    for (int j = 0; j < kJ; ++j) {
+      const float b4[4] = {bias[j].x, bias[j].y, bias[j].z, bias[j].w};
+      const float s4[4] = {winv[j].x, winv[j].y, winv[j].z, winv[j].w};
+      float v[4];
+      // the scales are powers of two: one rounding, that of the sum with the bias
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = fmaf(acc[tb][j][r] * xinv[tb], s4[r], b4[r]);
-        four(tb, j, v);
-      }
-  } else {
-#pragma unroll 1
-    for (int e = 0; e < kTB * kJ * 4; ++e) {
-      const int tb = e >> 4, j = (e >> 2) & 3, f = f0 + 16 * j + 4 * lq + (e & 3);
-      one(tb, j, e & 3, f < kF ? exact_value<KT>(a, g, tb ? tok[kTB - 1] : tok[0], f) : 0.f);
+      for (int r = 0; r < 4; ++r) v[r] = bad ? acc[tb][j][r] + b4[r] : fmaf(acc[tb][j][r] * xinv[tb], s4[r], b4[r]);
+      four(tb, j, v);
     }
   }
 }
@@ -506,8 +531,6 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
     tile_values<KT, kTB>(a, g, ft * kFT, tok, xinv, bad_rows, reinterpret_cast<const float*>(ws + kET * kWLoads), acc,
                     [&](int tb, int j, const float (&v)[4]) {
       most[tb] = fmaxf(most[tb], fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
-    }, [&](int tb, int j, int r, float v) {
-      if (tb) most[kTB - 1] = fmaxf(most[kTB - 1], v); else most[0] = fmaxf(most[0], v);
     });
 #pragma unroll
     for (int tb = 0; tb < kTB; ++tb)
@@ -771,22 +794,17 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
           xl = yl;
         }
         const unsigned flat = flat0 + (unsigned)(t + 16 * s) * kF;
-        if (bad_w || __any(inv == 0.f)) {  // uniform
-#pragma unroll 1
-          for (int e = 0; e < kJ * 4; ++e) {
-            const int f = 16 * (e >> 2) + (e & 3);
-            const bool in = tok < t1 && f0 + f < kF;
-            const float v = in ? exact_value<KT>(a, g, tok, f0 + f) : 0.f;
-            if constexpr (kStore)
-              if (in) a.act[(size_t)g * a.N * kF + flat + f] = v > 0.f ? v : 0.f;
-            if constexpr (kCollect) {
-              gather(in && v >= least, flat + (unsigned)f, v);
-              flush();
-            }
-          }
-          continue;
+        if (__builtin_expect(bad_w || __any(inv == 0.f), 0)) {  // uniform
+          fp32_products<KT>(a, g, min(tok, a.N - 1), ft * kFT, acc);
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[j] += bias[j];
+        } else {
+          // the scales are powers of two: one rounding, that of the sum with the bias
+#pragma unroll
+          for (int j = 0; j < kJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
         }
-        // the scales are powers of two: one rounding, that of the sum with the bias
         float most = -INFINITY;
         unsigned hits = 0u;
         // NaN (nothing is collected) for rows past the range; a bucket past F has a
@@ -797,8 +815,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
           u32x4 p;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float v = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
-            acc[j][r] = v;
+            const float v = acc[j][r];
             p[r] = __float_as_uint(v > 0.f ? v : 0.f);  // relu; NaN is not positive
             // hits = 2 hits + (v >= from), in two instructions
             if constexpr (kCollect)
