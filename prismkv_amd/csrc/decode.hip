@@ -1031,9 +1031,9 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
     // ---- 1-4. the rows of the q_activation router's selection: wave h takes
     // head h's 16 buckets of positive weight (a bucket that two heads chose
     // counts once in an OR, and an empty one has no bit set, so the union needs
-    // neither the scores nor their order: the group's last workgroup ranks them
-    // for the caller after its attention), and wave w ORs rows w, w + 8, ...
-    // over the tile's first 128 words
+    // neither the scores nor their order, NaN ones below apart: the group's last
+    // workgroup ranks them for the caller after its attention), and wave w ORs
+    // rows w, w + 8, ... over the tile's first 128 words
     int* sel64 = reinterpret_cast<int*>(lds.sel.best);  // -1: none
     static_assert(kQaSel * sizeof(int) <= sizeof(lds.sel.best) && kQaSel * sizeof(unsigned long long) <= sizeof(lds.tl),
                   "the heads' buckets, and their keys kept for the ranking");
@@ -1046,6 +1046,22 @@ __global__ __launch_bounds__(kDT) void decode_kernel(DecodeArgs a) {
       }
     }
     __syncthreads();
+    // An infinite activation's weight is NaN (inf / inf), and with it its bucket's
+    // score, whatever the other heads give that bucket: their entries of it go too.
+    // A head's largest activation is its first key.
+    const unsigned long long* top = reinterpret_cast<const unsigned long long*>(lds.tl);
+    bool infinite = false;
+#pragma unroll
+    for (int h = 0; h < kHq; ++h) infinite |= qact_infinite(top[kTop * h]);
+    if (__builtin_expect(infinite, 0)) {  // uniform
+      if (w == 0) {
+        const int row = row_of(top[lane]);
+        bool drop = false;
+        for (int e = 0; e < kQaSel; ++e) drop |= qact_infinite(top[e]) && row_of(top[e]) == row;
+        if (drop) sel64[lane] = -1;
+      }
+      __syncthreads();
+    }
     if (a.tw <= 2 * kTileWords) {
       constexpr int kRows = kQaSel / (kDT / 64);
       const int words = (a.H + 31) / 32, wd = p * a.tw + lane;

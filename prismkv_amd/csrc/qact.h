@@ -27,6 +27,8 @@ __device__ __forceinline__ unsigned long long qact_head_top(const unsigned long 
   return sorted_rows_top16<kSets>(v);  // each 16-lane row is one part's ranked list
 }
 
+__device__ __forceinline__ bool qact_infinite(unsigned long long key) { return (unsigned)(key >> 12) == 0x7f800000u; }
+
 // A head's weights: val / max(sum of the 16 in rank order, 1e-20) / 4, for the
 // wave that holds its list (lane r, rank r).
 __device__ __forceinline__ float qact_weight(unsigned long long key) {
