@@ -56,6 +56,7 @@
 // workgroup per bucket, any member count).  Unless the caller keeps them, a
 // build never writes its activations (12 KB per key) at all.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -198,14 +199,21 @@ __device__ __forceinline__ unsigned fine_digit(unsigned u, unsigned floor) {
 //   x . w = x_hi . w_hi + x_hi . w_lo + x_lo . w_hi
 // in fp32 accumulators (three f16 MFMAs of 32 dims instead of eight fp32 ones
 // of 4).  hi + lo is within 2^-22 of v at most and 2^-24.8 rms, x_lo . w_lo
-// (left out) 2^-24.7 rms of its product, so the split costs less than the
-// roundings of a 128-step fp32 chain: against 64 bits the activations are
-// within 1.4e-7 (2-norm over a block) where the fp32 MFMA chain had 2.1e-7.
+// (left out) 2^-24.7 rms of its product: not v itself, but over many dims less
+// than the roundings of an fp32 chain.  Against 64 bits the activations of dense
+// rows are within 1.4e-7 (2-norm over a block) where the fp32 MFMA chain has
+// 2.1e-7; the fewer products of a sum are not 0, the shorter the chain's error
+// (1.0e-7 at 32 of them, 2.5e-8 at one), while the split's stays (0.8 to 1.0e-7).
 // The power of two, per key row and per bucket, brings the largest magnitude
 // to [2^14, 2^15), so nothing overflows f16 and what underflows is below 2^-39
-// of that largest one.  A row or bucket that is not finite, or whose largest
-// magnitude lies outside 2^+-60 (the scales' products would leave fp32), is
-// not split: its values are computed by fp32 MFMA (fp32_products).
+// of that largest one.  A row or bucket is not split, its values being computed
+// by fp32 MFMA (fp32_products), if
+//   - it is not finite, or its largest magnitude lies outside 2^+-60 (the
+//     scales' products would leave fp32);
+//   - fewer than kMinDims of its dims are at least 2^-16 of the largest one (a
+//     key dim 2^18 above the others under a zero weight: 2.4e-7 split, 2.0e-7
+//     by the chain).  A split row and a split bucket then share 32 such dims at
+//     least, where the split is the closer one.  An all-zero one is split.
 //
 // The split W of tile ft (64 buckets) is 32 fragments of 1 KB,
 // [kb (4)][hi, lo][j (4)], lane (i, q) = (l % 16, l / 16) of a fragment holding
@@ -217,6 +225,8 @@ __device__ __forceinline__ unsigned fine_digit(unsigned u, unsigned floor) {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int kScaleExp = 14;   // scaled rows have their largest magnitude in [2^14, 2^15)
 constexpr int kMaxScale = 60;   // |exponent| of a row's or bucket's largest magnitude, at most
+constexpr int kMinDims = 80;    // significant dims of a row or bucket that is split, at least
+constexpr float kSignificant = 0x1p-16f;  // of the largest magnitude, at least
 constexpr int kWTile = kFT * kD * 2 + kFT * 4;  // f16 words of a split W tile: the fragments, 64 biases, 64 inverse scales (fp32)
 constexpr int kKB = kD / 32;          // MFMA dim blocks
 
@@ -228,6 +238,25 @@ __device__ __forceinline__ float2 row_scale(float m) {
   if (!(e >= -kMaxScale && e <= kMaxScale)) return make_float2(0.f, 0.f);
   const int k = kScaleExp - e;
   return make_float2(__uint_as_float((unsigned)(127 + k) << 23), __uint_as_float((unsigned)(127 - k) << 23));
+}
+
+// Whether at least kMinDims of a row's 128 magnitudes are significant.  The
+// calling lane holds N of them, the row's lanes are M apart (M, 2 M, .. < 64); m
+// is the row's largest.  Every row of the wave answers at once: nearly always by
+// the lanes' minima alone (a N(0, 1) row has a smaller value once in 250).
+template <int M, int N>
+__device__ __forceinline__ bool enough_dims(const float (&x)[N], float m) {
+  const float least = m * kSignificant;
+  float lo = fabsf(x[0]);
+#pragma unroll
+  for (int i = 1; i < N; ++i) lo = fminf(lo, fabsf(x[i]));
+  if (!__any(lo < least)) return true;  // uniform
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) n += fabsf(x[i]) >= least ? 1 : 0;
+#pragma unroll
+  for (int o = M; o < 64; o *= 2) n += __shfl_xor(n, o);
+  return n >= kMinDims;
 }
 
 template <typename Fn>
@@ -394,6 +423,37 @@ __device__ __forceinline__ void fp32_products(const UpdateArgs& a, int g, int to
   }
 }
 
+// fp32_products with the tile's W in the wave's registers, as f32x4 words: w[e][j]
+// is lane (i, q)'s dims 16 e + 4 q .. + 3 of bucket 16 j + i.  The same products in
+// the same order.
+template <typename KT>
+__device__ __forceinline__ void fp32_products(const UpdateArgs& a, int g, int tok, const half8 (&w)[kD / 16][kJ],
+                                              f32x4 (&acc)[kJ]) {
+  const int lq = (threadIdx.x >> 4) & 3;
+  const __amdgpu_buffer_rsrc_t kr = raw_buffer(static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)a.H * kD,
+                                               a.N * kD * (int)sizeof(KT));
+  const __amdgpu_buffer_rsrc_t cr = raw_buffer(a.center + (size_t)g * kD, kD * (int)sizeof(float));
+  const unsigned ko = ((unsigned)tok * kD + 4 * lq) * (unsigned)sizeof(KT), co = 4 * lq * (unsigned)sizeof(float);
+  const float s = a.scale[g];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < kD / 8; ++e) {  // two of the block's four dims at a time
+    const int d = 16 * (e >> 1) + 2 * (e & 1);
+    const f32x2 m = load_f2(cr, co, d * (int)sizeof(float));
+    const typename KeyLoad<KT>::Raw2 r = KeyLoad<KT>::load2(kr, ko, d * (int)sizeof(KT));
+    const float x[2] = {(KeyLoad<KT>::lo(r) - m[0]) / s, (KeyLoad<KT>::hi(r) - m[1]) / s};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const f32x4 wv = __builtin_bit_cast(f32x4, w[e >> 1][j]);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[2 * (e & 1) + t], x[t], acc[j], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // The values of one bucket tile for the wave's 16 kTB tokens, after the products
 // (made again in fp32 where a row or bucket is not split): four(tb, j, v) gets
 // lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3.  `tok` is the lane's
@@ -487,6 +547,8 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
     m = fmaxf(m, __shfl_xor(m, 16));
     m = fmaxf(m, __shfl_xor(m, 32));
     const float2 sc = row_scale(m);
+    // (the sample itself, which only places the floor, uses any split there is)
+    const bool enough = enough_dims<16>(reinterpret_cast<const float (&)[kKB * 8]>(x), m);
     half8* lds = reinterpret_cast<half8*>(ws) + lane;
     half8* out = reinterpret_cast<half8*>(a.wsplit + ((size_t)g * kFTiles + ft) * kWTile) + lane;
 #pragma unroll
@@ -507,7 +569,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
       if (y == 0) {
         float* t = reinterpret_cast<float*>(a.wsplit + ((size_t)g * kFTiles + ft) * kWTile + kFT * kD * 2) + 16 * w + lane;
         t[0] = tail[0];
-        t[kFT] = tail[kFT];
+        t[kFT] = enough ? sc.y : 0.f;
       }
     }
   }
@@ -632,6 +694,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     m = fmaxf(m, __shfl_xor(m, 16));
     m = fmaxf(m, __shfl_xor(m, 32));
     const float2 s2 = row_scale(fabsf(divide_by(m, scale, rscale)));  // the largest |x|; NaN for an infinite m
+    const bool enough = enough_dims<8>(reinterpret_cast<const float (&)[16]>(x), m);
     // (d / s) times the row's power of two: the quotient and its remainder scale exactly
     const float rs = rscale * s2.x, ss = scale * s2.y;
     half8* out = &xs[buf][((sr >> 4) * kKB + (sp >> 1)) * 2 * 64 + (2 * (sp & 1)) * 16 + (sr & 15)];
@@ -643,18 +706,23 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       out[64 + 16 * h] = lo;
     }
     // (a quotient's remainder stays in the normal range)
-    if (sp == 0) xinv[buf][sr] = scaled && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
+    // (its place is found again for each stage: kept, it would be spilled, and its
+    // reload awaits the stage's stores)
+    int zero = 0;
+    asm volatile("" : "+s"(zero));
+    const int l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, (unsigned)zero));
+    if (l < 8) xinv[buf][8 * w + l] = scaled && enough && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
   };
   load_rows(t0);
   if (tid < kD) center[tid] = a.center[(size_t)g * kD + tid];
   const _Float16* wt = a.wsplit + ((size_t)g * kFTiles + min(ft, kFTiles - 1)) * kWTile;
-  half8 wf[kKB][2][kJ];
+  // The tile's W, split ([2 kb + hi, lo][column]), or in fp32 (fp32_products).
+  static_assert(2 * kKB == kD / 16, "both forms take 128 registers");
+  half8 wf[2 * kKB][kJ];
 #pragma unroll
-  for (int kb = 0; kb < kKB; ++kb)
+  for (int e = 0; e < 2 * kKB; ++e)
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int j = 0; j < kJ; ++j) wf[kb][p][j] = reinterpret_cast<const half8*>(wt)[((kb * 2 + p) * kJ + j) * 64 + lane];
+    for (int j = 0; j < kJ; ++j) wf[e][j] = reinterpret_cast<const half8*>(wt)[(e * kJ + j) * 64 + lane];
   f32x4 bias[kJ], winv[kJ];
   bool bad_w = false;
 #pragma unroll
@@ -714,17 +782,33 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     __syncthreads();
   }
   split_rows(0);
+  __syncthreads();
+  // fp32 products throughout, W in registers, for a tile with a bucket that is not
+  // split, and where half of the first stage's steps have a row that is not; a lone
+  // such step takes its W from L2 (the build of 65536 keys with an encoder of 6 of 128
+  // weights: 15.4 ms with every step's W from there, 6.4 from registers)
+  const unsigned long long odd = __ballot(xinv[0][lane] == 0.f);
+  const int odd_steps = (int)((odd & 0xffffull) != 0) + (int)((odd >> 16 & 0xffffull) != 0) +
+                        (int)((odd >> 32 & 0xffffull) != 0) + (int)(odd >> 48 != 0);
+  const bool whole = bad_w || odd_steps >= 2;  // uniform
+  if (__builtin_expect(whole, 0)) {
+    const __amdgpu_buffer_rsrc_t wr = raw_buffer(a.W + (size_t)g * kF * kD, kF * kD * (int)sizeof(float));  // 0 past F
+    const unsigned o = ((unsigned)(ft * kFT + li) * kD + 4 * lq) * (unsigned)sizeof(float);
+#pragma unroll
+    for (int e = 0; e < kD / 16; ++e)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+        wf[e][j] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(
+            wr, o, (16 * j * kD + 16 * e) * (int)sizeof(float), 0));
+  }
   // W is awaited here: left pending into the loop, its first use there waited in every
   // step for the stores of the step before
 #pragma unroll
-  for (int kb = 0; kb < kKB; ++kb)
+  for (int e = 0; e < 2 * kKB; ++e)
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int j = 0; j < kJ; ++j) asm volatile("" ::"v"(wf[kb][p][j]));
+    for (int j = 0; j < kJ; ++j) asm volatile("" ::"v"(wf[e][j]));
 #pragma unroll
   for (int j = 0; j < kJ; ++j) asm volatile("" ::"v"(bias[j]), "v"(winv[j]));
-  __syncthreads();
   uint2* list = a.list + (size_t)g * a.list_cap;
   unsigned n = 0u;  // the wave's gathered candidates (uniform)
   auto put = [&](unsigned at, unsigned i) {
@@ -761,97 +845,109 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
 #pragma unroll
   for (int j = 0; j < kJ; ++j) column[j] = f0 + 16 * j < kF ? (flat0 + 16u * j) * (unsigned)sizeof(float) : 1u << 31;
   int buf = 0;
-  for (int t = t0; t < t1; t += kStage) {  // uniform
-    const bool more = t + kStage < t1;
-    if (more) load_rows(t + kStage);  // in flight while this stage is multiplied
-    // the stage's activation rows; stores past them (rows past the block, buckets
-    // past F) carry an offset outside the resource and are dropped
-    const __amdgpu_buffer_rsrc_t ar = raw_buffer(a.act + ((size_t)g * a.N + t) * kF,
-                                                 kStore ? min(kStage, t1 - t) * kF * (int)sizeof(float) : 0);
-    if (live) {
+  auto tokens = [&](auto in_fp32) {
+    constexpr bool kWhole = decltype(in_fp32)::value;
+    for (int t = t0; t < t1; t += kStage) {  // uniform
+      const bool more = t + kStage < t1;
+      if (more) load_rows(t + kStage);  // in flight while this stage is multiplied
+      // the stage's activation rows; stores past them (rows past the block, buckets
+      // past F) carry an offset outside the resource and are dropped
+      const __amdgpu_buffer_rsrc_t ar = raw_buffer(a.act + ((size_t)g * a.N + t) * kF,
+                                                   kStore ? min(kStage, t1 - t) * kF * (int)sizeof(float) : 0);
+      if (live) {
 #pragma unroll 1
-      for (int s = 0; s < kSteps && t + 16 * s < t1; ++s) {  // uniform
-        const int tok = t + 16 * s + li;
-        const half8* x = &xs[buf][s * kKB * 2 * 64 + lane];
-        half8 xh = x[0], xl = x[64];
-        const float inv = xinv[buf][16 * s + li];
-        f32x4 acc[kJ];
+        for (int s = 0; s < kSteps && t + 16 * s < t1; ++s) {  // uniform
+          const int tok = t + 16 * s + li;
+          const half8* x = &xs[buf][s * kKB * 2 * 64 + lane];
+          half8 xh = x[0], xl = x[64];
+          const float inv = xinv[buf][16 * s + li];
+          f32x4 acc[kJ];
+          if constexpr (!kWhole) {
 #pragma unroll
-        for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kb = 0; kb < kKB; ++kb) {
-          // the next dim block's rows are requested before this one's products
-          const half8 yh = x[(kb + 1) % kKB * 2 * 64], yl = x[((kb + 1) % kKB * 2 + 1) * 64];
-          __builtin_amdgcn_sched_barrier(0);
+            for (int kb = 0; kb < kKB; ++kb) {
+              // the next dim block's rows are requested before this one's products
+              const half8 yh = x[(kb + 1) % kKB * 2 * 64], yl = x[((kb + 1) % kKB * 2 + 1) * 64];
+              __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][1][j], xh, acc[j], 0, 0, 0);
+              for (int j = 0; j < kJ; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[2 * kb + 1][j], xh, acc[j], 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][0][j], xl, acc[j], 0, 0, 0);
+              for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[2 * kb][j], xl, acc[j], 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[kb][0][j], xh, acc[j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          xh = yh;
-          xl = yl;
-        }
-        const unsigned flat = flat0 + (unsigned)(t + 16 * s) * kF;
-        if (__builtin_expect(bad_w || __any(inv == 0.f), 0)) {  // uniform
-          fp32_products<KT>(a, g, min(tok, a.N - 1), ft * kFT, acc);
-#pragma unroll
-          for (int j = 0; j < kJ; ++j) acc[j] += bias[j];
-        } else {
-          // the scales are powers of two: one rounding, that of the sum with the bias
-#pragma unroll
-          for (int j = 0; j < kJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
-        }
-        float most = -INFINITY;
-        unsigned hits = 0u;
-        // NaN (nothing is collected) for rows past the range; a bucket past F has a
-        // zero row and bias: its 0 is below every floor
-        const float from = tok < t1 ? least : __builtin_nanf("");
-#pragma unroll
-        for (int j = 0; j < kJ; ++j) {
-          u32x4 p;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float v = acc[j][r];
-            p[r] = __float_as_uint(v > 0.f ? v : 0.f);  // relu; NaN is not positive
-            // hits = 2 hits + (v >= from), in two instructions
-            if constexpr (kCollect)
-              asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(hits) : "v"(v), "v"(from) : "vcc");
-            most = fmaxf(most, v);
-          }
-          if constexpr (kStore)
-            __builtin_amdgcn_raw_buffer_store_b128(p, ar, column[j] + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
-        }
-        if constexpr (kCollect) {
-          // a lane's one candidate is its largest value
-          const bool one = hits != 0u && (hits & (hits - 1u)) == 0u;
-          const unsigned long long m = __ballot(one);
-          const unsigned e = (unsigned)__clz((int)hits) & 15u;  // bit 15 is the first value
-          cand[w][one ? place(m) : kWaveBuf + lane] = make_uint2(flat + 4u * (e & 12u) + (e & 3u), __float_as_uint(most));
-          n += (unsigned)__popcll(m);
-          const bool several = hits != 0u && !one;
-          if (__any(several)) {  // uniform
-#pragma unroll
-            for (int j = 0; j < kJ; ++j) {
-              flush();
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                gather(several && (hits >> (15 - 4 * j - r) & 1u), flat + (unsigned)(16 * j + r), acc[j][r]);
+              for (int j = 0; j < kJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[2 * kb][j], xh, acc[j], 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+              xh = yh;
+              xl = yl;
             }
+          } else {
+            fp32_products<KT>(a, g, min(tok, a.N - 1), wf, acc);
           }
-          flush();
+          const unsigned flat = flat0 + (unsigned)(t + 16 * s) * kF;
+          if (kWhole || __builtin_expect(__any(inv == 0.f), 0)) {  // uniform
+            if constexpr (!kWhole) fp32_products<KT>(a, g, min(tok, a.N - 1), ft * kFT, acc);
+#pragma unroll
+            for (int j = 0; j < kJ; ++j) acc[j] += bias[j];
+          } else {
+            // the scales are powers of two: one rounding, that of the sum with the bias
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
+          }
+          float most = -INFINITY;
+          unsigned hits = 0u;
+          // NaN (nothing is collected) for rows past the range; a bucket past F has a
+          // zero row and bias: its 0 is below every floor
+          const float from = tok < t1 ? least : __builtin_nanf("");
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) {
+            u32x4 p;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float v = acc[j][r];
+              p[r] = __float_as_uint(v > 0.f ? v : 0.f);  // relu; NaN is not positive
+              // hits = 2 hits + (v >= from), in two instructions
+              if constexpr (kCollect)
+                asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(hits) : "v"(v), "v"(from) : "vcc");
+              most = fmaxf(most, v);
+            }
+            if constexpr (kStore)
+              __builtin_amdgcn_raw_buffer_store_b128(p, ar, column[j] + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
+          }
+          if constexpr (kCollect) {
+            // a lane's one candidate is its largest value
+            const bool one = hits != 0u && (hits & (hits - 1u)) == 0u;
+            const unsigned long long m = __ballot(one);
+            const unsigned e = (unsigned)__clz((int)hits) & 15u;  // bit 15 is the first value
+            cand[w][one ? place(m) : kWaveBuf + lane] = make_uint2(flat + 4u * (e & 12u) + (e & 3u), __float_as_uint(most));
+            n += (unsigned)__popcll(m);
+            const bool several = hits != 0u && !one;
+            if (__any(several)) {  // uniform
+#pragma unroll
+              for (int j = 0; j < kJ; ++j) {
+                flush();
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  gather(several && (hits >> (15 - 4 * j - r) & 1u), flat + (unsigned)(16 * j + r), acc[j][r]);
+              }
+            }
+            flush();
+          }
         }
       }
+      if (more) {
+        split_rows(buf ^ 1);  // last read before the previous barrier
+        __syncthreads();
+        buf ^= 1;
+      }
     }
-    if (more) {
-      split_rows(buf ^ 1);  // last read before the previous barrier
-      __syncthreads();
-      buf ^= 1;
-    }
-  }
+  };
+  if (__builtin_expect(whole, 0))
+    tokens(std::true_type{});
+  else
+    tokens(std::false_type{});
   if constexpr (kCollect) {  // the rest of the 8 waves, one reservation
     __syncthreads();
     if (lane == 0) wsum[w] = n;

@@ -125,3 +125,40 @@ def test_encode_key_scales(exponent):
     scale = scale * 2.0 ** exponent
     _, act = run_append(k, W, b, center, scale, 100)
     check(k, W, b, center, scale, act)
+
+
+@pytest.mark.parametrize("where", ["buckets", "keys"])
+@pytest.mark.parametrize("dims,norm", [(1, 3.2e-8), (4, 4.9e-8), (16, 8.5e-8), (79, 1.8e-7)])
+def test_encode_of_few_dims(where, dims, norm):
+    # a sum of few products has few roundings in fp32, fewer than the split's operands
+    # cost it: fp32 chains measure 2.5e-8, 3.9e-8, 7.5e-8 and 1.6e-7 (2-norm), the split
+    # 0.8 to 1.0e-7.  Every third row or bucket is such a one, the others are dense
+    k, W, b, center, scale = inputs(200, 81)
+    center.zero_()
+    b.zero_()
+    if where == "buckets":
+        W[:, ::3, dims:] = 0
+        pick = (slice(None), slice(0, F, 3))
+    else:
+        k[:, H::3, dims:] = 0
+        pick = (slice(0, None, 3), slice(None))
+    _, act = run_append(k, W, b, center, scale, 200)
+    x = (k[:, H:].float() / scale[:, None, None])[:, pick[0]]
+    want = torch.stack([torch.relu(x[g].double() @ W[g, pick[1]].double().T) for g in range(G)])
+    got = act[:, pick[0], pick[1]].double()
+    assert float((got - want).norm() / want.norm()) < norm
+    if dims == 1:  # one product, one rounding
+        assert bool(((got - want).abs() <= 2.0 ** -24 * want).all())
+
+
+def test_encode_of_a_key_with_one_large_dim():
+    # the other dims fall toward f16's subnormals once the largest one is at 2^15: 2.0e-7 by
+    # fp32 chains, 2.4e-7 split
+    k, W, b, center, scale = inputs(200, 82)
+    b.zero_()
+    k[:, :, 7] = (k[:, :, 7].float() * 2.0 ** 18).to(torch.bfloat16)
+    W[:, :, 7] = 0
+    _, act = run_append(k, W, b, center, scale, 200)
+    x = (k[:, H:].float() - center[:, None]) / scale[:, None, None]
+    want = torch.stack([torch.relu(x[g].double() @ W[g].double().T) for g in range(G)])
+    assert float((act.double() - want).norm() / want.norm()) < 2.15e-7
