@@ -1702,7 +1702,7 @@ __global__ __launch_bounds__(kUT) void clear_bits_kernel(UpdateArgs a) {
 // bound by the chain of its 24,000 workgroups' loads, and four times as many of
 // them are in flight; longer buckets are left to build_moments_rest_kernel.  256
 // against 64 threads, 8 groups: 136 / 52 us at 6000 keys, 158 / 87 at 16384, 190
-// / 159 at 32768, 282 / 331 at 65536 (and 5 us for the other launch).
+// / 159 at 32768, 282 / 331 at 65536 (and the other launch).
 // mean = sum / n rounded to fp32; var = sum (x - mean)^2 / n
 // with that rounded mean; empty bucket -> 0 (core.py:84-88).  Counts and
 // moments are written, not merged.
@@ -1866,27 +1866,27 @@ __device__ __forceinline__ void bucket_moments(const UpdateArgs& a, int g, int f
   }
 }
 
-template <typename KT, int NT>
-__global__ __launch_bounds__(NT, 4) void build_moments_kernel(UpdateArgs a) {
+__device__ __forceinline__ int moment_bucket(unsigned x) {
   static_assert(kF % 8 == 0, "buckets in 8 equal runs");
-  __shared__ BuildMomentsLds<NT> L;
-  bucket_moments<KT, NT>(a, blockIdx.y, (int)(blockIdx.x & 7u) * (kF / 8) + (int)(blockIdx.x >> 3), L);
+  return (int)(x & 7u) * (kF / 8) + (int)(x >> 3);
 }
 
-// Grid (kRestBlocks, G) x 256: the buckets of more members than a one-wave
-// workgroup lists.
-constexpr int kRestBlocks = 64;
+template <typename KT, int NT>
+__global__ __launch_bounds__(NT, 4) void build_moments_kernel(UpdateArgs a) {
+  __shared__ BuildMomentsLds<NT> L;
+  bucket_moments<KT, NT>(a, blockIdx.y, moment_bucket(blockIdx.x), L);
+}
+
+// After it, grid (F, G) x 256: the buckets of more members than a one-wave
+// workgroup lists.  A workgroup each, as any number of them may be (a dense bitmap,
+// a budget of many per key): 64 workgroups for all took 22.9 ms for one group of
+// 32768 keys with half of them in every bucket, 1000 took 2.1, now 1.9 (one launch
+// of 256 threads: 1.7); where there is none, 8 groups' launch takes 10 us.
 template <typename KT>
 __global__ __launch_bounds__(kUT, 4) void build_moments_rest_kernel(UpdateArgs a) {
   __shared__ BuildMomentsLds<kUT> L;
-  const int g = blockIdx.y;
-  static_assert((kF + kRestBlocks - 1) / kRestBlocks <= 64, "a lane per bucket");
-  const int mine = (int)blockIdx.x + kRestBlocks * (int)(threadIdx.x & 63);
-  unsigned long long heavy = __ballot(mine < kF && a.counts[(size_t)g * kFP + min(mine, kF - 1)] > BuildMomentsLds<64>::kLen);
-  for (; heavy; heavy &= heavy - 1ull) {  // uniform
-    bucket_moments<KT, kUT>(a, g, (int)blockIdx.x + kRestBlocks * (int)__builtin_ctzll(heavy), L);
-    __syncthreads();  // the list and the sums are free again
-  }
+  const int g = blockIdx.y, f = moment_bucket(blockIdx.x);
+  if (a.counts[(size_t)g * kFP + f] > BuildMomentsLds<64>::kLen) bucket_moments<KT, kUT>(a, g, f, L);  // uniform
 }
 
 // ---------------------------------------------------------------------------
@@ -2156,9 +2156,11 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
 
 template <typename KT>
 static void launch_build_moments(const UpdateArgs& a, int groups, hipStream_t s) {
-  if (a.N <= kSmallBuild) {
+  // a budget that fills most buckets past a wave's list goes to whole workgroups at once
+  // (64 per key of 32768: 4.34 ms, 4.59 by way of the other two launches)
+  if (a.N <= kSmallBuild && a.budget <= (long long)kF * BuildMomentsLds<64>::kLen) {
     hipLaunchKernelGGL((build_moments_kernel<KT, 64>), dim3(kF, groups), dim3(64), 0, s, a);
-    hipLaunchKernelGGL(build_moments_rest_kernel<KT>, dim3(kRestBlocks, groups), dim3(kUT), 0, s, a);
+    hipLaunchKernelGGL(build_moments_rest_kernel<KT>, dim3(kF, groups), dim3(kUT), 0, s, a);
   } else
     hipLaunchKernelGGL((build_moments_kernel<KT, kUT>), dim3(kF, groups), dim3(kUT), 0, s, a);
 }

@@ -61,3 +61,30 @@ def test_append_of_few_dims(where):
     else:
         k[:, :, 70:] = 0
     assert append_us(k, W, b, center, scale, 4096) < 4 * plain
+
+
+@pytest.mark.parametrize("density", [0.5, 0.02])
+def test_summarize_of_full_buckets(density):
+    # up to 32768 keys a bucket is one wave's unless its list is full, which any number of
+    # buckets may find: 1.1 times the call of one key more, whose buckets are a workgroup's
+    # each (1.5 where half of the lists are; 13.8 and 5.6 with 64 workgroups for all of them)
+    from prismkv_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    n, rw = 32769, 1028
+    k = torch.randn(1, n, D, generator=gen, device="cuda").to(torch.bfloat16)
+    on = torch.rand(F, rw, 32, generator=gen, device="cuda") < density
+    bits = (on << torch.arange(32, device="cuda")).sum(-1).to(torch.int32)
+    center = torch.zeros(1, D, device="cuda")
+    work = torch.zeros(lib.query("prismkv_summarize_work_bytes", 1), dtype=torch.uint8, device="cuda")
+    counts = torch.zeros(1, 3008, dtype=torch.int32, device="cuda")
+    moments = torch.zeros(1, 94, 256, 32, device="cuda")
+
+    def once(keys):
+        lib.call("prismkv_summarize", k.data_ptr(), bits.data_ptr(), center.data_ptr(), counts.data_ptr(),
+                 moments.data_ptr(), work.data_ptr(), 1, keys, 0, n * D, rw, _lib.nbytes(work),
+                 stream=torch.cuda.current_stream().cuda_stream)
+
+    whole = shortest(lambda: once(n))
+    assert shortest(lambda: once(n - 1)) < 2.5 * whole
+    assert torch.equal(counts[0, :F], on.reshape(F, -1)[:, :n - 1].sum(1).int())
