@@ -88,3 +88,11 @@ def test_summarize_of_full_buckets(density):
     whole = shortest(lambda: once(n))
     assert shortest(lambda: once(n - 1)) < 2.5 * whole
     assert torch.equal(counts[0, :F], on.reshape(F, -1)[:, :n - 1].sum(1).int())
+
+
+def test_append_of_many_per_key():
+    # 100 memberships per key are more than the sample can count, so no list is made: 2.1 times
+    # the plain call (20 with a list that overflows)
+    k, W, b, center, scale = inputs(1024, 3)
+    plain = append_us(k, W, b, center, scale, 1024)
+    assert append_us(k, W, b, center, scale, 1024, 100) < 5 * plain

@@ -178,3 +178,15 @@ def test_build_heavy_buckets(history, heavy):
     torch.cuda.synchronize()
     assert (op.n[:, 5:F:1000] >= heavy).all()
     check_moments(op, k, membership(op, 0, history))
+
+
+@pytest.mark.parametrize("block,key_mean", [(1024, 60), (1024, 74), (1024, 76), (1024, 100), (4096, 42), (300, 300)])
+def test_append_of_many_per_key(block, key_mean):
+    # memberships per key around those that the sample can count
+    k, W, b, center, scale = inputs(block, key_mean)
+    op, act = run_append(k, W, b, center, scale, block, key_mean)
+    got = membership(op, H, block)
+    for g in (0, 5):
+        want = oracle.positive_global_topk(act[g].cpu().numpy(), key_mean * block)
+        assert np.array_equal(np.sort(want), got[g].cpu().numpy())
+    check_moments(op, k[:, H:], got)
