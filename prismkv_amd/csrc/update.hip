@@ -85,7 +85,7 @@ constexpr int kBuildCenter = 1;      // prismkv_build flag: compute the center (
 constexpr int kBuildNoAct = 4;       // prismkv_build flag: the activations need not be left in the workspace
 
 // ctl words per group
-enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kFloor, kListLen, kCut, kTieLen, kCtl = 16 };
+enum { kMode = 0, kPrefix, kRem, kTau, kNeed, kTies, kOrdered, kCount, kFloor, kListLen, kCut, kTieLen, kArrived, kCtl = 16 };
 enum { kModeTopK = 0, kModeAllPositive = 1 };
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -388,6 +388,15 @@ __device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)
   }
 }
 
+// The lane's number, found again where it is rarely needed: what the compiler derives
+// from it is then not kept in registers of a loop that has none to spare (a spilled
+// word's reload awaits the activations' stores).
+__device__ __forceinline__ int lane_again() {
+  unsigned zero = 0u;
+  asm volatile("" : "+s"(zero));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 // The products of 16 tokens (`tok`, the lane's) with the buckets f0 .. f0 + 63 in
 // fp32, for rows and buckets that the split does not serve: v_mfma_f32_16x16x4f32
 // (lane (i, q) feeding A[i][q] and B[q][i], and holding D[4 q + r][i]), four dims
@@ -397,7 +406,7 @@ __device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)
 // held one infinite key took 822 us, and 63 without it.)
 template <typename KT>
 __device__ __forceinline__ void fp32_products(const UpdateArgs& a, int g, int tok, int f0, f32x4 (&acc)[kJ]) {
-  const int li = threadIdx.x & 15, lq = (threadIdx.x >> 4) & 3;
+  const int l = lane_again(), li = l & 15, lq = l >> 4;
   // (as buffers: one offset register each, and zeros for buckets past F)
   const __amdgpu_buffer_rsrc_t kr = raw_buffer(static_cast<const KT*>(a.k) + (size_t)g * a.ks + (size_t)a.H * kD,
                                                a.N * kD * (int)sizeof(KT));
@@ -577,6 +586,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
   if (y == 0 && ft == 0 && tid == 0) {
     a.ctl[(size_t)g * kCtl + kListLen] = 0u;
     a.ctl[(size_t)g * kCtl + kTieLen] = 0u;
+    a.ctl[(size_t)g * kCtl + kArrived] = 0u;
   }
   if (S == 0) return;  // uniform
   for (int i = tid; i < kSampleBins; i += kET) hist[i] = 0u;
@@ -707,11 +717,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       out[64 + 16 * h] = lo;
     }
     // (a quotient's remainder stays in the normal range)
-    // (its place is found again for each stage: kept, it would be spilled, and its
-    // reload awaits the stage's stores)
-    int zero = 0;
-    asm volatile("" : "+s"(zero));
-    const int l = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, (unsigned)zero));
+    const int l = lane_again();
     if (l < 8) xinv[buf][8 * w + l] = scaled && enough && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
   };
   load_rows(t0);
@@ -827,12 +833,14 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       n += (unsigned)__popcll(m);
     }
   };
+  bool full = false;  // the list overflowed and is of no use: no more of it (uniform)
   auto flush = [&]() {
     if (n <= kWaveBuf - 256) return;  // uniform
     __builtin_amdgcn_wave_barrier();
     unsigned at = 0u;
     if (lane == 0) at = atomicAdd(&ctl[kListLen], n);
     at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
+    full |= at >= a.list_cap;
     for (unsigned i = lane; i < n; i += 64) put(at, i);
     __builtin_amdgcn_wave_barrier();
     n = 0u;
@@ -842,9 +850,9 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   // added to them and not given as the instruction's scalar offset: four-word
   // stores with one lost their last word to the vector instruction that
   // followed, which the compiler takes to need no wait.)
-  unsigned column[kJ];
-#pragma unroll
-  for (int j = 0; j < kJ; ++j) column[j] = f0 + 16 * j < kF ? (flat0 + 16u * j) * (unsigned)sizeof(float) : 1u << 31;
+  static_assert(kF - (kFTiles - 1) * kFT > 16 * (kJ - 1) && kF % 4 == 0, "of the last tile only the last column ends early");
+  const unsigned column = flat0 * (unsigned)sizeof(float);
+  const unsigned last_column = f0 + 16 * (kJ - 1) < kF ? column + 64u * (kJ - 1) : 1u << 31;
   int buf = 0;
   auto tokens = [&](auto in_fp32) {
     constexpr bool kWhole = decltype(in_fp32)::value;
@@ -915,9 +923,10 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
               most = fmaxf(most, v);
             }
             if constexpr (kStore)
-              __builtin_amdgcn_raw_buffer_store_b128(p, ar, column[j] + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b128(
+                  p, ar, (j < kJ - 1 ? column + 64u * j : last_column) + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
           }
-          if constexpr (kCollect) {
+          if (kCollect && !full) {
             // a lane's one candidate is its largest value
             const bool one = hits != 0u && (hits & (hits - 1u)) == 0u;
             const unsigned long long m = __ballot(one);
@@ -1082,12 +1091,19 @@ __device__ __forceinline__ void each_value(const UpdateArgs& a, int g, bool list
   } else {
     const size_t n4 = (size_t)a.N * kF / 4, step = (size_t)NT * blocks;
     const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * a.N * kF);
-    for (size_t i = (size_t)block * NT + threadIdx.x; i < n4; i += step) {
-      const float4 v = ag[i];
-      const float vv[4] = {v.x, v.y, v.z, v.w};
+    for (size_t i0 = (size_t)block * NT + threadIdx.x; i0 < n4; i0 += kU * step) {
+      float4 v[kU];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (vv[j] > 0.f) fn(__float_as_uint(vv[j]), (unsigned)(4 * i + j));
+      for (int u = 0; u < kU; ++u) v[u] = ag[i0 + u * step < n4 ? i0 + u * step : i0];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const size_t i = i0 + u * step;
+        if (i >= n4) break;
+        const float vv[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (vv[j] > 0.f) fn(__float_as_uint(vv[j]), (unsigned)(4 * i + j));
+      }
     }
   }
 }
@@ -1165,14 +1181,24 @@ __device__ __forceinline__ void set_member(const UpdateArgs& a, int g, unsigned 
 // 1024 keys, 41.5 at 4096, bound by its one CU; now 12.5 and 22.  64 or
 // 128 split workgroups per group were no faster: 8 and 9 us for 7, 16 and 18 for 16.)
 // A digit that does not fit (ties by the thousand) or that the counts do not
-// reach, or a list that cannot be used: select takes all of it, by passes over
-// the list or the activations.  Beyond kSelectMax those passes would be too long
-// for one workgroup, and hist0 / digit / refine and the tie kernels, over 256
-// workgroups per group, are the better ones.
+// reach: select takes all of it, by passes over the list.  Beyond kSelectMax those
+// would be too long for one workgroup, and hist0 / digit / refine and the tie
+// kernels, over 256 workgroups per group, are the better ones.
+//
+// A list that cannot be used (the sample misjudged): both launches read the dense
+// activations, over all their workgroups.  split counts the positive values in
+// 13-bit digits; select's workgroups, which otherwise leave at once, set the bits of
+// the values above tau's digit and list those in it, and the last of them to end
+// finds tau and the cut among these.  Where even they are more than the list holds
+// (one value millions of times) they are counted by their other 18 bits, and the
+// last workgroup takes the ties in one ordered pass.  (Appends of 600 / 4096 keys with
+// every value tied: 0.23 / 0.56 ms; 8.1 / 49 with all of it in one workgroup per group.)
 // ---------------------------------------------------------------------------
 constexpr int kST = 1024;
 constexpr int kSelBuf = 8192;
 constexpr int kSplitBlocks = 32;
+constexpr int kSelectBlocks = 32;
+constexpr int kLowBins = 1 << kSampleShift;  // the values of one 13-bit digit
 
 // The fine digit of the budget-th largest candidate; false if split and select
 // cannot work with it.
@@ -1183,11 +1209,59 @@ __device__ __forceinline__ bool find_fine(const UpdateArgs& a, int g, unsigned* 
   return list_ok(a, g) && f.digit < (unsigned)kBins - 1u && f.ties <= (unsigned)kSelBuf;
 }
 
+// Adds to a histogram, a thread's run of equal bins at once: where one value comes
+// by the million its counter would take an atomic for each.
+struct RunCount {
+  unsigned bin = 0u, n = 0u;
+  __device__ __forceinline__ void add(unsigned* hist, unsigned d) {
+    if (d != bin) flush(hist);
+    bin = d;
+    ++n;
+  }
+  __device__ __forceinline__ void flush(unsigned* hist) {
+    if (n) atomicAdd(&hist[bin], n);
+    n = 0u;
+  }
+  // The whole wave's runs, equal bins joined (a counter in memory takes 10 ns for each).
+  __device__ __forceinline__ void flush_wave(unsigned* hist) {
+    for (unsigned long long left = __ballot(n != 0u); left; left = __ballot(n != 0u)) {  // uniform
+      const int lead = (int)__builtin_ctzll(left);
+      const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)bin, lead);
+      const bool same = n != 0u && bin == b;
+      const int total = wave_sum_i(same ? (int)n : 0);
+      if ((int)(threadIdx.x & 63) == lead) atomicAdd(&hist[b], (unsigned)total);
+      if (same) n = 0u;
+    }
+  }
+};
+
+// The 13-bit counts of a group whose list cannot be used: in the levels of the
+// histogram that calls of up to kSelectMax keys have no other use for.
+__device__ __forceinline__ unsigned* dense_hist(const UpdateArgs& a, int g) {
+  static_assert(2 * kRep * kBins >= kSampleBins, "room in levels 1 and 2");
+  return hist_of(a, g, 1);
+}
+
 __global__ __launch_bounds__(kUT) void split_kernel(UpdateArgs a) {
-  const int g = blockIdx.y;
+  const int g = blockIdx.y, tid = threadIdx.x;
   __shared__ unsigned wsum[kUT / 64];
+  __shared__ unsigned dense[kSampleBins];
   __shared__ Found found;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  if (__builtin_expect(!list_ok(a, g), 0)) {  // uniform
+    for (int i = tid; i < kSampleBins; i += kUT) dense[i] = 0u;
+    unsigned* low = a.ties + (size_t)g * a.list_cap;
+    for (int i = (int)blockIdx.x * kUT + tid; i < kLowBins; i += kSplitBlocks * kUT) low[i] = 0u;
+    __syncthreads();
+    RunCount run;
+    each_value<kUT>(a, g, false, blockIdx.x, gridDim.x, [&](unsigned u, unsigned) { run.add(dense, u >> kSampleShift); });
+    run.flush(dense);
+    __syncthreads();
+    unsigned* hg = dense_hist(a, g);
+    for (int i = tid; i < kSampleBins; i += kUT)
+      if (dense[i]) atomicAdd(&hg[i], dense[i]);
+    return;
+  }
   Found f;
   if (!find_fine<kUT>(a, g, wsum, &found, f)) return;  // uniform
   const unsigned floor = ctl[kFloor];
@@ -1199,139 +1273,298 @@ __global__ __launch_bounds__(kUT) void split_kernel(UpdateArgs a) {
   });
 }
 
+// The flat index of the `rem`-th of the ties at `tau` in ascending order, by a radix
+// search over the complements of what each(fn(value, flat)) goes through.
+template <typename Each>
+__device__ __forceinline__ unsigned tie_cut(unsigned tau, unsigned rem, unsigned* hist, unsigned* wsum, Found* found,
+                                            Each each) {
+  unsigned key = 0u;
+  const int width[3] = {11, 11, 10};
+  int shift = 32;
+  for (int l = 0; l < 3; ++l) {
+    shift -= width[l];
+    const unsigned mask = (1u << width[l]) - 1u;
+    const int hi = shift + width[l];
+    for (int i = threadIdx.x; i < (1 << width[l]); i += kST) hist[i] = 0u;
+    __syncthreads();
+    each([&](unsigned u, unsigned flat) {
+      const unsigned c = ~flat;
+      if (u == tau && (hi == 32 || (c >> hi) == key)) atomicAdd(&hist[(c >> shift) & mask], 1u);
+    });
+    __syncthreads();
+    const Found f = find_digit<kST>(hist, 1 << width[l], rem, wsum, found);
+    key = (key << width[l]) | f.digit;
+    rem = f.rem;
+  }
+  return ~key;
+}
+
+// tau, given its 13-bit digit and its rank f.rem among that digit's values, from
+// passes over them; f becomes that of tau's own ties.
+template <typename Each>
+__device__ __forceinline__ unsigned find_tau(unsigned top, Found& f, unsigned* hist, unsigned* wsum, Found* found,
+                                             Each each) {
+  unsigned prefix = top;
+  for (int shift = 9; shift >= 0; shift -= 9) {
+    for (int i = threadIdx.x; i < 512; i += kST) hist[i] = 0u;
+    __syncthreads();
+    each([&](unsigned u, unsigned) {
+      if ((u >> (shift + 9)) == prefix) atomicAdd(&hist[(u >> shift) & 511u], 1u);
+    });
+    __syncthreads();
+    f = find_digit<kST>(hist, 512, f.rem, wsum, found);
+    prefix = (prefix << 9) | f.digit;
+  }
+  return prefix;
+}
+
+struct SelectLds {
+  unsigned hist[kSampleBins];
+  uint2 bin[kSelBuf];
+  unsigned wsum[kST / 64], nbin, base;
+  Found found;
+};
+
+// select of a group whose list cannot be used, by workgroup x of kSelectBlocks.
+__device__ __forceinline__ void select_dense(const UpdateArgs& a, int g, int x, SelectLds& L) {
+  const int tid = threadIdx.x;
+  unsigned* ctl = a.ctl + (size_t)g * kCtl;
+  const unsigned count = budget_of(a);
+  unsigned npos = 0u;
+  for (int i = tid; i < kSampleBins; i += kST) {
+    L.hist[i] = dense_hist(a, g)[i];
+    npos += L.hist[i];
+  }
+  block_incl_scan<kST>(npos, L.wsum);
+  npos = 0u;
+  for (int i = 0; i < kST / 64; ++i) npos += L.wsum[i];
+  __syncthreads();
+  const bool all = npos < count;  // fewer positives than the budget: every one is kept (core.py:22-26)
+  Found f{0u, 0u, 0u};
+  if (!all) f = find_digit<kST>(L.hist, kSampleBins, count, L.wsum, &L.found);
+  const unsigned top = f.digit;
+  const bool gathered = f.ties <= a.list_cap;
+  uint2* list = a.list + (size_t)g * a.list_cap;  // (what the encode left there serves nothing)
+  unsigned* low = a.ties + (size_t)g * a.list_cap;
+  RunCount run;
+  each_value<kST>(a, g, false, x, kSelectBlocks, [&](unsigned u, unsigned flat) {
+    const unsigned d = u >> kSampleShift;
+    if (all || d > top)
+      set_member(a, g, flat);
+    else if (d == top && gathered) {
+      const unsigned i = atomicAdd(&L.nbin, 1u);
+      uint2* to = i < (unsigned)kSelBuf ? L.bin + i : list + atomicAdd(&ctl[kTieLen], 1u);
+      *to = make_uint2(flat, u);
+    } else if (d == top)
+      run.add(low, u & (kLowBins - 1u));
+  });
+  run.flush_wave(low);
+  __syncthreads();
+  const unsigned mine = min(L.nbin, (unsigned)kSelBuf);
+  if (tid == 0) L.base = mine ? atomicAdd(&ctl[kTieLen], mine) : 0u;
+  __syncthreads();
+  for (unsigned i = tid; i < mine; i += kST) list[L.base + i] = L.bin[i];
+  // the last workgroup to come here goes on
+  __threadfence();
+  __syncthreads();
+  if (tid == 0) L.base = atomicAdd(&ctl[kArrived], 1u);
+  __syncthreads();
+  if (L.base != kSelectBlocks - 1) return;  // uniform
+  __threadfence();
+  for (int i = tid; i < kSampleBins; i += kST) dense_hist(a, g)[i] = 0u;  // for the next call
+  if (all) return;
+  if (gathered) {
+    const unsigned n = f.ties;
+    const bool in_lds = n <= (unsigned)kSelBuf;
+    if (in_lds) {
+      for (unsigned i = tid; i < n; i += kST) L.bin[i] = list[i];
+      __syncthreads();
+    }
+    auto each = [&](auto fn) {
+      for (unsigned i = tid; i < n; i += kST) {
+        const uint2 e = in_lds ? L.bin[i] : list[i];
+        fn(e.y, e.x);
+      }
+    };
+    const unsigned tau = find_tau(top, f, L.hist, L.wsum, &L.found, each);
+    const unsigned cut = f.ties > f.rem ? tie_cut(tau, f.rem, L.hist, L.wsum, &L.found, each) : ~0u;
+    each([&](unsigned u, unsigned flat) {
+      if (u > tau || (u == tau && flat <= cut)) set_member(a, g, flat);
+    });
+    return;
+  }
+  // tau from the counts of the digit's 2^18 values, 256 of them (a wave's load) at first
+  constexpr int kPer = kLowBins / kST;
+  static_assert(kPer == 4 * 64, "a wave's 16-byte words");
+  const unsigned in_digit = f.rem;
+  constexpr int kLoads = 8;
+  for (int i0 = tid / 64 * 64; i0 < tid / 64 * 64 + 64; i0 += kLoads) {
+    uint4 v[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) v[i] = reinterpret_cast<const uint4*>(low + kPer * (i0 + i))[tid & 63];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int c = wave_sum_i((int)(v[i].x + v[i].y + v[i].z + v[i].w));
+      if ((tid & 63) == 0) L.hist[i0 + i] = (unsigned)c;
+    }
+  }
+  __syncthreads();
+  f = find_digit<kST>(L.hist, kST, f.rem, L.wsum, &L.found);
+  const unsigned high = f.digit;
+  if (tid < kPer) L.hist[tid] = low[kPer * high + tid];
+  __syncthreads();
+  f = find_digit<kST>(L.hist, kPer, f.rem, L.wsum, &L.found);
+  const unsigned tau = (top << kSampleShift) | (kPer * high + f.digit);
+  const unsigned above = in_digit - f.rem, need = f.rem;  // the digit's members beside tau's ties, and those
+  // the activations in flat order until both are complete
+  constexpr int kU = 8;
+  const size_t n4 = (size_t)a.N * kF / 4;
+  const float4* ag = reinterpret_cast<const float4*>(a.act + (size_t)g * a.N * kF);
+  unsigned taken = 0u, over = 0u;
+  for (size_t base = 0; base < n4 && (taken < need || over < above); base += kU * kST) {  // uniform
+    auto value = [&](int u) {
+      const size_t i = base + (size_t)u * kST + tid;
+      return i < n4 ? ag[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    auto bits = [](float x) { return x > 0.f ? __float_as_uint(x) : 0u; };
+    auto in = [&](unsigned b) { return b >= tau && (b >> kSampleShift) == top; };
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const float4 v = value(u);
+      any |= in(bits(v.x)) || in(bits(v.y)) || in(bits(v.z)) || in(bits(v.w));
+    }
+    if (!__syncthreads_or(any)) continue;
+#pragma unroll 1
+    for (int u = 0; u < kU; ++u) {
+      const unsigned flat = 4u * (unsigned)(base + (size_t)u * kST + tid);
+      const float4 v = value(u);
+      const unsigned b[4] = {bits(v.x), bits(v.y), bits(v.z), bits(v.w)};
+      unsigned k = 0u;  // ties, and in the upper half the larger ones
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        k += b[j] == tau ? 1u : 0u;
+        if (b[j] > tau && in(b[j])) {
+          set_member(a, g, flat + j);
+          k += 1u << 16;
+        }
+      }
+      unsigned rank = taken + ((block_incl_scan<kST>(k, L.wsum) - k) & 0xffffu);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (b[j] == tau && rank++ < need) set_member(a, g, flat + j);
+      unsigned total = 0u;
+      for (int i = 0; i < kST / 64; ++i) total += L.wsum[i];
+      taken += total & 0xffffu;
+      over += total >> 16;
+      __syncthreads();  // wsum is rewritten by the next scan
+    }
+  }
+}
+
+// Grid (G, kSelectBlocks) x 1024.
 __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
   const int g = blockIdx.x, tid = threadIdx.x;
-  __shared__ unsigned hist[kSampleBins];
-  __shared__ uint2 bin[kSelBuf];
-  __shared__ unsigned wsum[kST / 64], nbin;
-  __shared__ Found found;
+  const bool listed = list_ok(a, g);  // uniform
+  if (listed && blockIdx.y) return;
+  __shared__ SelectLds L;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
-  const bool listed = list_ok(a, g);
   const unsigned count = budget_of(a);
-  for (int i = tid; i < kSampleBins; i += kST) a.sample[(size_t)g * kSampleBins + i] = 0u;  // for the next call
-  if (tid == 0) nbin = 0u;
+  if (blockIdx.y == 0)
+    for (int i = tid; i < kSampleBins; i += kST) a.sample[(size_t)g * kSampleBins + i] = 0u;  // for the next call
+  if (tid == 0) L.nbin = 0u;
   Found f;
-  const bool split = find_fine<kST>(a, g, wsum, &found, f);
-  for (int i = tid; i < kBins; i += kST) hist_of(a, g, 0)[i] = 0u;  // for the next call
+  const bool split = listed && find_fine<kST>(a, g, L.wsum, &L.found, f);
+  if (blockIdx.y == 0)
+    for (int i = tid; i < kBins; i += kST) hist_of(a, g, 0)[i] = 0u;  // for the next call
+  if (!listed) {
+    select_dense(a, g, blockIdx.y, L);
+    return;
+  }
   unsigned prefix;
-  bool gathered = true;
   if (split) {
     const uint2* ties = reinterpret_cast<const uint2*>(a.ties + (size_t)g * a.list_cap);
-    for (unsigned i = tid; i < f.ties; i += kST) bin[i] = ties[i];
-    if (tid == 0) nbin = f.ties;
-    for (int i = tid; i < (1 << kFineShift); i += kST) hist[i] = 0u;
+    for (unsigned i = tid; i < f.ties; i += kST) L.bin[i] = ties[i];
+    if (tid == 0) L.nbin = f.ties;
+    for (int i = tid; i < (1 << kFineShift); i += kST) L.hist[i] = 0u;
     __syncthreads();
     const unsigned base = ctl[kFloor] + (f.digit << kFineShift);
-    for (unsigned i = tid; i < nbin; i += kST) atomicAdd(&hist[bin[i].y - base], 1u);
+    for (unsigned i = tid; i < L.nbin; i += kST) atomicAdd(&L.hist[L.bin[i].y - base], 1u);
     __syncthreads();
-    f = find_digit<kST>(hist, 1 << kFineShift, f.rem, wsum, &found);
+    f = find_digit<kST>(L.hist, 1 << kFineShift, f.rem, L.wsum, &L.found);
     prefix = base + f.digit;
-  } else {
-    // The listed values lie within a few octaves above the floor, 32 digits each,
-    // so they are counted in kRel digits from the floor's on, 8 replicas of each
-    // (64 lanes meet in some 25 digits: one replica took 15 us of atomics for the
-    // list of 4096 keys); a value beyond them, or an unlisted call, in all 8192.
-    constexpr unsigned kRel = kSampleBins / 8;
-    unsigned npos = 0u;
-    for (bool rel = listed;; rel = false) {  // uniform
-      const unsigned base = rel ? ctl[kFloor] >> kSampleShift : 0u;
-      __syncthreads();
-      for (int i = tid; i < kSampleBins; i += kST) hist[i] = 0u;
-      __syncthreads();
-      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned) {
-        const unsigned d = (u >> kSampleShift) - base;
-        atomicAdd(&hist[rel ? 8u * min(d, kRel - 1u) + (tid & 7) : d], 1u);
-      });
-      __syncthreads();
-      if (rel) {
-        unsigned c = 0u;
-        if (tid < (int)kRel)
-#pragma unroll
-          for (int r = 0; r < 8; ++r) c += hist[8 * tid + r];
-        __syncthreads();
-        if (tid < (int)kRel) hist[tid] = c;
-        __syncthreads();
-      }
-      const int bins = rel ? (int)kRel : kSampleBins;
-      npos = 0u;
-      for (int i = tid; i < bins; i += kST) npos += hist[i];
-      block_incl_scan<kST>(npos, wsum);
-      npos = 0u;
-      for (int i = 0; i < kST / 64; ++i) npos += wsum[i];
-      __syncthreads();
-      if (npos < count) {  // fewer positives than the budget: every one is kept (core.py:22-26)
-        each_value<kST>(a, g, listed, 0, 1, [&](unsigned, unsigned flat) { set_member(a, g, flat); });
-        return;
-      }
-      f = find_digit<kST>(hist, bins, count, wsum, &found);
-      if (!rel) break;
-      if (f.digit < kRel - 1u) {
-        f.digit += base;
-        break;
-      }
-    }
-    const unsigned top = f.digit;
-    gathered = f.ties <= (unsigned)kSelBuf;
-    if (gathered) {
-      each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
-        if ((u >> kSampleShift) == top) bin[atomicAdd(&nbin, 1u)] = make_uint2(flat, u);
-      });
-      __syncthreads();
-    }
-    // counts the digit (key >> shift) & mask of the values of tau's bin for which in(u, flat)
-    auto count_digits = [&](int bins, auto in, auto digit) {
-      for (int i = tid; i < bins; i += kST) hist[i] = 0u;
-      __syncthreads();
-      if (gathered) {
-        for (unsigned i = tid; i < nbin; i += kST)
-          if (in(bin[i].y)) atomicAdd(&hist[digit(bin[i].y, bin[i].x)], 1u);
-      } else {
-        each_value<kST>(a, g, listed, 0, 1, [&](unsigned u, unsigned flat) {
-          if (in(u)) atomicAdd(&hist[digit(u, flat)], 1u);
-        });
-      }
-      __syncthreads();
+    auto each = [&](auto fn) {
+      for (unsigned i = tid; i < L.nbin; i += kST) fn(L.bin[i].y, L.bin[i].x);
     };
-    prefix = top;
-    for (int shift = 9; shift >= 0; shift -= 9) {
-      count_digits(512, [&](unsigned u) { return (u >> (shift + 9)) == prefix; },
-                   [&](unsigned u, unsigned) { return (u >> shift) & 511u; });
-      f = find_digit<kST>(hist, 512, f.rem, wsum, &found);
-      prefix = (prefix << 9) | f.digit;
+    const unsigned cut = f.ties > f.rem ? tie_cut(prefix, f.rem, L.hist, L.wsum, &L.found, each) : ~0u;
+    each([&](unsigned u, unsigned flat) {
+      if (u > prefix || (u == prefix && flat <= cut)) set_member(a, g, flat);
+    });
+    return;
+  }
+  // The listed values lie within a few octaves above the floor, 32 digits each,
+  // so they are counted in kRel digits from the floor's on, 8 replicas of each
+  // (64 lanes meet in some 25 digits: one replica took 15 us of atomics for the
+  // list of 4096 keys); where tau lies beyond them, in all 8192.
+  auto listed_values = [&](auto fn) { each_value<kST>(a, g, true, 0, 1, fn); };
+  constexpr unsigned kRel = kSampleBins / 8;
+  unsigned npos = 0u;
+  for (bool rel = true;; rel = false) {  // uniform
+    const unsigned base = rel ? ctl[kFloor] >> kSampleShift : 0u;
+    __syncthreads();
+    for (int i = tid; i < kSampleBins; i += kST) L.hist[i] = 0u;
+    __syncthreads();
+    listed_values([&](unsigned u, unsigned) {
+      const unsigned d = (u >> kSampleShift) - base;
+      atomicAdd(&L.hist[rel ? 8u * min(d, kRel - 1u) + (tid & 7) : d], 1u);
+    });
+    __syncthreads();
+    if (rel) {
+      unsigned c = 0u;
+      if (tid < (int)kRel)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) c += L.hist[8 * tid + r];
+      __syncthreads();
+      if (tid < (int)kRel) L.hist[tid] = c;
+      __syncthreads();
+    }
+    const int bins = rel ? (int)kRel : kSampleBins;
+    npos = 0u;
+    for (int i = tid; i < bins; i += kST) npos += L.hist[i];
+    block_incl_scan<kST>(npos, L.wsum);
+    npos = 0u;
+    for (int i = 0; i < kST / 64; ++i) npos += L.wsum[i];
+    __syncthreads();
+    if (npos < count) {  // fewer positives than the budget: every one is kept (core.py:22-26)
+      listed_values([&](unsigned, unsigned flat) { set_member(a, g, flat); });
+      return;
+    }
+    f = find_digit<kST>(L.hist, bins, count, L.wsum, &L.found);
+    if (!rel) break;
+    if (f.digit < kRel - 1u) {
+      f.digit += base;
+      break;
     }
   }
-  unsigned cut = ~0u;
-  if (f.ties > f.rem) {  // the rem-th smallest flat index of the ties = the rem-th largest complement
-    unsigned key = 0u;
-    const int width[3] = {11, 11, 10};
-    int shift = 32;
-    for (int l = 0; l < 3; ++l) {
-      shift -= width[l];
-      const unsigned mask = (1u << width[l]) - 1u;
-      const int hi = shift + width[l];
-      for (int i = tid; i < (1 << width[l]); i += kST) hist[i] = 0u;
-      __syncthreads();
-      auto tie = [&](unsigned u, unsigned flat) {
-        const unsigned c = ~flat;
-        if (u == prefix && (hi == 32 || (c >> hi) == key)) atomicAdd(&hist[(c >> shift) & mask], 1u);
-      };
-      if (gathered)
-        for (unsigned i = tid; i < nbin; i += kST) tie(bin[i].y, bin[i].x);
-      else
-        each_value<kST>(a, g, listed, 0, 1, tie);
-      __syncthreads();
-      f = find_digit<kST>(hist, 1 << width[l], f.rem, wsum, &found);
-      key = (key << width[l]) | f.digit;
-    }
-    cut = ~key;
+  const unsigned top = f.digit;
+  const bool gathered = f.ties <= (unsigned)kSelBuf;
+  if (gathered) {
+    listed_values([&](unsigned u, unsigned flat) {
+      if ((u >> kSampleShift) == top) L.bin[atomicAdd(&L.nbin, 1u)] = make_uint2(flat, u);
+    });
+    __syncthreads();
   }
-  auto emit = [&](unsigned u, unsigned flat) {
-    if (u > prefix || (u == prefix && flat <= cut)) set_member(a, g, flat);
+  auto each = [&](auto fn) {
+    if (gathered)
+      for (unsigned i = tid; i < L.nbin; i += kST) fn(L.bin[i].y, L.bin[i].x);
+    else
+      listed_values(fn);
   };
-  if (split)
-    for (unsigned i = tid; i < nbin; i += kST) emit(bin[i].y, bin[i].x);
-  else
-    each_value<kST>(a, g, listed, 0, 1, emit);
+  prefix = find_tau(top, f, L.hist, L.wsum, &L.found, each);
+  const unsigned cut = f.ties > f.rem ? tie_cut(prefix, f.rem, L.hist, L.wsum, &L.found, each) : ~0u;
+  listed_values([&](unsigned u, unsigned flat) {
+    if (u > prefix || (u == prefix && flat <= cut)) set_member(a, g, flat);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -2146,7 +2379,7 @@ static void launch_selection(UpdateArgs a, int groups, bool keep, hipStream_t s)
   }
   if (one) {
     hipLaunchKernelGGL(split_kernel, dim3(kSplitBlocks, groups), dim3(kUT), 0, s, a);
-    hipLaunchKernelGGL(select_kernel, dim3(groups), dim3(kST), 0, s, a);
+    hipLaunchKernelGGL(select_kernel, dim3(groups, kSelectBlocks), dim3(kST), 0, s, a);
   } else {
     hipLaunchKernelGGL(hist0_kernel, dim3(kRefineBlocks, groups), dim3(kUT), 0, s, a);
     hipLaunchKernelGGL(digit_kernel, dim3(groups), dim3(kUT), 0, s, a, 0);

@@ -190,3 +190,40 @@ def test_append_of_many_per_key(block, key_mean):
         want = oracle.positive_global_topk(act[g].cpu().numpy(), key_mean * block)
         assert np.array_equal(np.sort(want), got[g].cpu().numpy())
     check_moments(op, k[:, H:], got)
+
+
+def sampled(block):
+    """The tokens whose activations place the floor (sample_token)."""
+    S = min(block, 128)
+    r = torch.arange(S)
+    return r if S == block else r * block // S + ((r * 0x9E3779B9 & 0xFFFFFFFF) >> 8) % (block // S)
+
+
+@pytest.mark.parametrize("block", [200, 600, 1024, 4096])
+@pytest.mark.parametrize("kind", ["low floor", "high floor", "few values", "two values"])
+def test_append_with_a_list_of_no_use(kind, block):
+    # the sample misjudges: the members are found from the dense activations, by many
+    # workgroups and the last of them
+    k, W, b, center, scale = inputs(block, 60 + block)
+    tok = (H + sampled(block)).cuda()
+    loud = torch.ones(H + block, device="cuda")
+    if kind == "low floor":  # the others are the loud ones: more candidates than the list holds
+        loud[H:] = 30.0
+        loud[tok] = 1.0
+    else:  # the sampled ones are: fewer candidates than the budget
+        loud[tok] = 30.0
+    k = (k.float() * loud[:, None]).to(torch.bfloat16)
+    if kind == "few values":  # and all the positive ones together are fewer
+        center.zero_()
+        k[:, H:][:, loud[H:] == 1.0] = 0
+        b.fill_(-60.0)
+    if kind == "two values":  # the larger one four times a token, the other more often than the list holds
+        W.zero_()
+        b.fill_(1.0)
+        b[:, ::750] = 1.0 + 2.0 ** -22
+    op, act = run_append(k, W, b, center, scale, block)
+    got = membership(op, H, block)
+    for g in (0, 3):
+        want = oracle.positive_global_topk(act[g].cpu().numpy(), 8 * block)
+        assert np.array_equal(np.sort(want), got[g].cpu().numpy())
+    check_moments(op, k[:, H:], got)
