@@ -361,7 +361,7 @@ int prismkv_topk(uint64_t act, uint64_t out, uint64_t out_len, uint64_t work, in
 
 /* The id checks of attend (core.py:176-179) for one group's ids i64 [n]: out
  * i32 [n] <- the ids (clamped into [0, H)), meta i32 [2] <- n, and 1 if an id lies
- * outside [0, H) | 2 if an id comes twice.  H in [1, 2^20]. */
+ * outside [0, H) | 2 if an id comes twice.  n in [0, 2^31), H in [1, 2^20]; -1 else. */
 int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int H, uint64_t stream);
 
 /* summarize (core.py:76-89) of every group from its bitmap rows: counts and

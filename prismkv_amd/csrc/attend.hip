@@ -161,7 +161,7 @@ constexpr int kIdThreads = 1024;
 constexpr int kMaxCheckedHistory = 1 << 20;
 constexpr int kIdRange = 1, kIdTwice = 2;  // meta[1]
 
-__global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __restrict__ ids, int n, int H,
+__global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __restrict__ ids, unsigned n, int H,
                                                                int32_t* __restrict__ out, int* __restrict__ meta) {
   extern __shared__ unsigned seen[];
   __shared__ int bad_s;
@@ -171,7 +171,8 @@ __global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __
   __syncthreads();
   constexpr int kU = 8;
   int bad = 0;
-  for (int i0 = tid; i0 < n; i0 += kU * kIdThreads) {
+  // (n < 2^31, so no index below passes 2^31 + 2^13: unsigned, that is)
+  for (unsigned i0 = tid; i0 < n; i0 += kU * kIdThreads) {
     int64_t v[kU];
 #pragma unroll
     for (int u = 0; u < kU; ++u) v[u] = ids[i0 + u * kIdThreads < n ? i0 + u * kIdThreads : i0];
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __
   if (bad) atomicOr(&bad_s, bad);
   __syncthreads();
   if (tid == 0) {
-    meta[0] = n;
+    meta[0] = (int)n;
     meta[1] = bad_s;
   }
 }
@@ -265,7 +266,7 @@ int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int 
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL(check_ids_kernel, dim3(1), dim3(kIdThreads), lds, (hipStream_t)stream,
-                     reinterpret_cast<const int64_t*>(ids), (int)n, H, reinterpret_cast<int32_t*>(out),
+                     reinterpret_cast<const int64_t*>(ids), (unsigned)n, H, reinterpret_cast<int32_t*>(out),
                      reinterpret_cast<int*>(meta));
   return (int)hipGetLastError();
 }
