@@ -388,6 +388,12 @@ __device__ __forceinline__ void tile_products(const u32x4* ws, const half8 (&xh)
   }
 }
 
+// A byte offset as a vector register, whatever it is the sum of.
+__device__ __forceinline__ unsigned vector_offset(unsigned o) {
+  asm("" : "+v"(o));
+  return o;
+}
+
 // The lane's number, found again where it is rarely needed: what the compiler derives
 // from it is then not kept in registers of a loop that has none to spare (a spilled
 // word's reload awaits the activations' stores).
@@ -846,10 +852,11 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
     n = 0u;
   };
   const unsigned flat0 = (unsigned)li * kF + (unsigned)f0;
-  // The lane's offsets in a step's rows; 2^31 is outside.  (The step's own part is
-  // added to them and not given as the instruction's scalar offset: four-word
-  // stores with one lost their last word to the vector instruction that
-  // followed, which the compiler takes to need no wait.)
+  // The lane's offsets in a step's rows; 2^31 is outside.  The step's own part is
+  // added to them, by vector_offset where the compiler can't take it apart again, and
+  // not given as the instruction's scalar offset: four-word stores with one lost their
+  // last word to the vector instruction that followed, which the compiler takes to
+  // need no wait.
   static_assert(kF - (kFTiles - 1) * kFT > 16 * (kJ - 1) && kF % 4 == 0, "of the last tile only the last column ends early");
   const unsigned column = flat0 * (unsigned)sizeof(float);
   const unsigned last_column = f0 + 16 * (kJ - 1) < kF ? column + 64u * (kJ - 1) : 1u << 31;
@@ -905,6 +912,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
 #pragma unroll
               for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(acc[j][r] * inv, winv[j][r], bias[j][r]);
           }
+          const unsigned at_step = 16u * s * kF * (unsigned)sizeof(float);
           float most = -INFINITY;
           unsigned hits = 0u;
           // NaN (nothing is collected) for rows past the range; a bucket past F has a
@@ -924,7 +932,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
             }
             if constexpr (kStore)
               __builtin_amdgcn_raw_buffer_store_b128(
-                  p, ar, (j < kJ - 1 ? column + 64u * j : last_column) + 16u * s * kF * (unsigned)sizeof(float), 0, 0);
+                  p, ar, j < kJ - 1 ? vector_offset(column + at_step) + 64u * j : vector_offset(last_column + at_step), 0, 0);
           }
           if (kCollect && !full) {
             // a lane's one candidate is its largest value
