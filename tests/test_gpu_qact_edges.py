@@ -1,5 +1,6 @@
 """The fused q_activation decode (core.py:131-139, :142-183) off its common
-path, against the separate launches: infinite activations, whose weights are NaN."""
+path, against the separate launches: infinite activations, whose weights are
+NaN, and group counts whose launches have 64 to 256 workgroups per group."""
 import pytest
 import torch
 
@@ -55,3 +56,72 @@ def test_infinite_activations(H, heads):
     # bf16 outputs of two exact softmaxes: at most a rounding of 2^-9 apart
     assert float((got.float() - want_out.float()).norm()) <= 4e-3 * float(want_out.float().norm())
     assert op.decode_errors() == 0
+
+
+@pytest.mark.parametrize("H,T", [(1, 2), (777, 5), (9000, 0), (65537, 33), (300001, 7)])
+@pytest.mark.parametrize("groups", [1, 2, 4])
+def test_other_group_counts_equal_the_separate_launches(groups, H, T):
+    # 256, 128 and 64 workgroups per group (Native8B's 8 groups have 32)
+    from prismkv_amd import _lib
+    op, q, k, v, W, b = operator(H, T, groups + H)
+    lib = op.lib
+    q, k, v, W, b = (x[:groups].contiguous() for x in (q, k, v, W, b))
+    scale = torch.linspace(0.5, 1.5, groups, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    cap = op.capacity
+
+    def work(name, *args):
+        return torch.zeros(max(lib.query(name, *args), 16), dtype=torch.uint8, device="cuda")
+
+    def outputs():
+        return dict(features=torch.full((groups, 64), 3, dtype=torch.int64, device="cuda"),
+                    valid=torch.full((groups, 64), 3.0, device="cuda"),
+                    raw=torch.full((groups,), 3, dtype=torch.int32, device="cuda"),
+                    ids=torch.full((groups, cap), 3, dtype=torch.int32, device="cuda"),
+                    count=torch.full((groups,), 3, dtype=torch.int32, device="cuda"),
+                    out=torch.full((groups, 4, 128), 3.0, dtype=torch.bfloat16, device="cuda"))
+
+    want, got = outputs(), outputs()
+    at = {x: t.data_ptr() for x, t in want.items()}
+    qact, union, state = (work("prismkv_route_qact_work_bytes", groups), work("prismkv_union_work_bytes", groups, H),
+                          work("prismkv_attend_work_bytes", groups, 64))
+    lib.call("prismkv_route_qact", q.data_ptr(), W.data_ptr(), b.data_ptr(), scale.data_ptr(), op.n.data_ptr(),
+             qact.data_ptr(), at["features"], at["valid"], at["raw"], 0, groups, _lib.nbytes(qact), stream=stream)
+    lib.call("prismkv_union_n", op.bits.data_ptr(), at["features"], at["valid"], union.data_ptr(), at["ids"], at["count"],
+             groups, H, op.row_words, cap, 64, _lib.nbytes(union), stream=stream)
+    lib.call("prismkv_attend", q.data_ptr(), k.data_ptr(), v.data_ptr(), at["ids"], at["count"], state.data_ptr(),
+             at["out"], groups, H, T, k.stride(0), v.stride(0), cap, 64, _lib.nbytes(state), stream=stream)
+    at = {x: t.data_ptr() for x, t in got.items()}
+    qact, decode = work("prismkv_route_qact_work_bytes", groups), work("prismkv_decode_work_bytes", groups, cap)
+    for _ in range(2):
+        lib.call("prismkv_decode_qact", q.data_ptr(), W.data_ptr(), b.data_ptr(), scale.data_ptr(), op.n.data_ptr(),
+                 op.bits.data_ptr(), k.data_ptr(), v.data_ptr(), qact.data_ptr(), decode.data_ptr(), at["features"],
+                 at["valid"], at["raw"], at["ids"], at["count"], at["out"], groups, H, T, cap, op.row_words, k.stride(0),
+                 v.stride(0), cap, _lib.nbytes(qact), _lib.nbytes(decode), stream=stream)
+        assert int(decode[:4].view(torch.int32)) == 0  # no wait gave up
+        for x in ("features", "valid", "raw", "count"):
+            assert torch.equal(got[x], want[x]), x
+        for g in range(groups):
+            assert torch.equal(got["ids"][g, :want["count"][g]], want["ids"][g, :want["count"][g]])
+        a, e = got["out"].float(), want["out"].float()
+        assert bool(e.isfinite().all()) and float((a - e).norm()) <= 4e-3 * float(e.norm()) + 1e-6
+
+
+def test_accepted_beside_the_refused():
+    # the argument set of test_fused_q_activation_refuses_what_the_decode_refuses, on real memory
+    op, q, k, v, W, b = operator(100, 4, 1)
+    op.set_query_encoders(W, b, torch.ones(8))
+    op.router = "q_activation"
+    call = getattr(op.lib.cdll, "prismkv_decode_qact")
+    need = op.lib.query("prismkv_decode_work_bytes", 8, 100), op.lib.query("prismkv_route_qact_work_bytes", 8)
+    good = [x.data_ptr() for x in (q, W, op.b_query, op.query_scale, op.n, op.bits, k, v, op.qact_work, op.decode_work,
+                                   op.features, op.valid, op.raw, op.ids, op.count, op.out)]
+    good += [8, 100, 4, 100, op.row_words, k.stride(0), v.stride(0), op.capacity, need[1], need[0],
+             torch.cuda.current_stream().cuda_stream]
+    assert op.capacity >= 100 and call(*good) == 0
+    torch.cuda.synchronize()
+    assert op.decode_errors() == 0
+    for at, value in ((24, need[1] - 1), (25, need[0] - 1), (17, 0), (18, -1), (1, 0)):
+        args = list(good)
+        args[at] = value
+        assert call(*args) == -1, (at, value)
