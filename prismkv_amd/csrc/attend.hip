@@ -156,17 +156,20 @@ __global__ __launch_bounds__(kAT) void attend_merge(const float* __restrict__ st
 // unique, each read back, they and the selection's read-backs took two thirds of
 // a 480 us call pair (core.select_buckets + core.attend at 1024 + 32 tokens, fp32;
 // 150 us with this kernel and one read-back each).  Bound by the one CU's reads:
-// 8 in flight per thread.
+// 8 in flight per thread.  An id's bit is id / words of word id % words, words a power
+// of two, so that the consecutive ids of a long list meet in no word (600,000 in 151 us;
+// 503 with 32 of them in each word).
 constexpr int kIdThreads = 1024;
 constexpr int kMaxCheckedHistory = 1 << 20;
 constexpr int kIdRange = 1, kIdTwice = 2;  // meta[1]
 
 __global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __restrict__ ids, unsigned n, int H,
-                                                               int32_t* __restrict__ out, int* __restrict__ meta) {
+                                                               int log_words, int32_t* __restrict__ out,
+                                                               int* __restrict__ meta) {
   extern __shared__ unsigned seen[];
   __shared__ int bad_s;
   const int tid = threadIdx.x;
-  for (int i = tid; i < (H + 31) / 32; i += kIdThreads) seen[i] = 0u;
+  for (int i = tid; i < 1 << log_words; i += kIdThreads) seen[i] = 0u;
   if (tid == 0) bad_s = 0;
   __syncthreads();
   constexpr int kU = 8;
@@ -183,7 +186,8 @@ __global__ __launch_bounds__(kIdThreads) void check_ids_kernel(const int64_t* __
         const int id = in ? (int)v[u] : 0;
         out[i0 + u * kIdThreads] = id;
         if (!in) bad |= kIdRange;
-        else if (atomicOr(&seen[id >> 5], 1u << (id & 31)) >> (id & 31) & 1u) bad |= kIdTwice;
+        else if (atomicOr(&seen[id & ((1 << log_words) - 1)], 1u << (id >> log_words)) >> (id >> log_words) & 1u)
+          bad |= kIdTwice;
       }
   }
   if (bad) atomicOr(&bad_s, bad);
@@ -258,7 +262,9 @@ int prismkv_attend_f32(uint64_t q, uint64_t k, uint64_t v, uint64_t ids, uint64_
 
 int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int H, uint64_t stream) {
   if (n < 0 || n > INT32_MAX || H < 1 || H > kMaxCheckedHistory || !out || !meta || (n && !ids)) return kBadSize;
-  const int lds = (H + 31) / 32 * (int)sizeof(unsigned);
+  int log_words = 0;
+  while (32ll << log_words < H) ++log_words;
+  const int lds = (int)sizeof(unsigned) << log_words;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(check_ids_kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -266,7 +272,7 @@ int prismkv_check_ids(uint64_t ids, uint64_t out, uint64_t meta, int64_t n, int 
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL(check_ids_kernel, dim3(1), dim3(kIdThreads), lds, (hipStream_t)stream,
-                     reinterpret_cast<const int64_t*>(ids), (unsigned)n, H, reinterpret_cast<int32_t*>(out),
+                     reinterpret_cast<const int64_t*>(ids), (unsigned)n, H, log_words, reinterpret_cast<int32_t*>(out),
                      reinterpret_cast<int*>(meta));
   return (int)hipGetLastError();
 }

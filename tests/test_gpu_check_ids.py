@@ -22,6 +22,35 @@ def test_the_largest_count_of_ids():
     assert bool((out[n:] == -7).all())
 
 
+def check(ids, H):
+    from prismkv_amd import _lib
+    out = torch.full((len(ids),), -7, dtype=torch.int32, device="cuda")
+    meta = torch.zeros(2, dtype=torch.int32, device="cuda")
+    _lib.load().call("prismkv_check_ids", ids.data_ptr(), out.data_ptr(), meta.data_ptr(), len(ids), H,
+                     stream=torch.cuda.current_stream().cuda_stream)
+    return out, meta
+
+
+@pytest.mark.parametrize("H", [1, 32, 33, 64, 65, 1000, 2049, 1 << 19, (1 << 19) + 1, 1 << 20])
+def test_every_id_and_one_twice(H):
+    # the bits' places around the powers of two
+    ids = torch.randperm(H, generator=torch.Generator().manual_seed(H)).cuda()
+    out, meta = check(ids, H)
+    assert meta.tolist() == [H, 0] and torch.equal(out.long(), ids)
+    assert check(torch.cat((ids, ids[H // 2:H // 2 + 1])), H)[1].tolist() == [H + 1, 2]
+    ids[H // 3] = H
+    assert check(ids, H)[1].tolist() == [H, 1]
+
+
+def test_consecutive_ids_cost_what_others_do():
+    # 151 us of either (503 of consecutive ones where 32 of them share an LDS word)
+    from tests.test_gpu_index_cost import shortest
+    H = 600000
+    ordered = torch.arange(H, device="cuda")
+    mixed = ordered[torch.randperm(H, generator=torch.Generator().manual_seed(1)).cuda()]
+    assert shortest(lambda: check(ordered, H)) < 2 * shortest(lambda: check(mixed, H))
+
+
 def test_refusals():
     from prismkv_amd import _lib
     lib = _lib.load()
