@@ -1,6 +1,7 @@
 """The fused q_activation decode (core.py:131-139, :142-183) off its common
 path, against the separate launches: infinite activations, whose weights are
-NaN, and group counts whose launches have 64 to 256 workgroups per group."""
+NaN, group counts whose launches have 64 to 256 workgroups per group, and a
+captured call."""
 import pytest
 import torch
 
@@ -125,3 +126,35 @@ def test_accepted_beside_the_refused():
         args = list(good)
         args[at] = value
         assert call(*args) == -1, (at, value)
+
+
+@pytest.mark.parametrize("H", [700, 40000])
+def test_captured_launches(H):
+    # the two launches replayed from a HIP graph on new queries, with eager calls between
+    op, q, k, v, W, b = operator(H, 9, H)
+    op.set_query_encoders(W, b, torch.ones(8))
+    op.router = "q_activation"
+    names = ("features", "valid", "raw", "count", "out")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        op(q, k, v)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op(q, k, v)
+    for i in range(4):
+        q.copy_(torch.randn(q.shape, generator=torch.Generator().manual_seed(i)))
+        op(q, k, v)
+        want = {x: getattr(op, x).clone() for x in names}
+        ids = [op.ids[g, :op.count[g]].clone() for g in range(8)]
+        for x in names + ("ids",):
+            getattr(op, x).fill_(3)
+        graph.replay()
+        torch.cuda.synchronize()
+        for x in names:
+            assert torch.equal(getattr(op, x), want[x]), (i, x)
+        for g in range(8):
+            assert torch.equal(op.ids[g, :op.count[g]], ids[g]), (i, g)
+    assert op.decode_errors() == 0
