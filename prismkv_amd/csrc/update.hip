@@ -839,14 +839,14 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       n += (unsigned)__popcll(m);
     }
   };
-  bool full = false;  // the list overflowed and is of no use: no more of it (uniform)
+  int collect_to = t1;  // the first token of which nothing is collected (uniform)
   auto flush = [&]() {
     if (n <= kWaveBuf - 256) return;  // uniform
     __builtin_amdgcn_wave_barrier();
     unsigned at = 0u;
     if (lane == 0) at = atomicAdd(&ctl[kListLen], n);
     at = (unsigned)__builtin_amdgcn_readfirstlane((int)at);
-    full |= at >= a.list_cap;
+    if (at >= a.list_cap) collect_to = 0;  // the list overflowed and is of no use: no more of it
     for (unsigned i = lane; i < n; i += 64) put(at, i);
     __builtin_amdgcn_wave_barrier();
     n = 0u;
@@ -917,7 +917,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
           unsigned hits = 0u;
           // NaN (nothing is collected) for rows past the range; a bucket past F has a
           // zero row and bias: its 0 is below every floor
-          const float from = tok < t1 ? least : __builtin_nanf("");
+          const float from = tok < collect_to ? least : __builtin_nanf("");
 #pragma unroll
           for (int j = 0; j < kJ; ++j) {
             u32x4 p;
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
               __builtin_amdgcn_raw_buffer_store_b128(
                   p, ar, j < kJ - 1 ? vector_offset(column + at_step) + 64u * j : vector_offset(last_column + at_step), 0, 0);
           }
-          if (kCollect && !full) {
+          if constexpr (kCollect) {
             // a lane's one candidate is its largest value
             const bool one = hits != 0u && (hits & (hits - 1u)) == 0u;
             const unsigned long long m = __ballot(one);
@@ -1256,7 +1256,9 @@ __global__ __launch_bounds__(kUT) void split_kernel(UpdateArgs a) {
   __shared__ unsigned dense[kSampleBins];
   __shared__ Found found;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
-  if (__builtin_expect(!list_ok(a, g), 0)) {  // uniform
+  Found f;
+  if (!find_fine<kUT>(a, g, wsum, &found, f)) {  // uniform
+    if (list_ok(a, g)) return;
     for (int i = tid; i < kSampleBins; i += kUT) dense[i] = 0u;
     unsigned* low = a.ties + (size_t)g * a.list_cap;
     for (int i = (int)blockIdx.x * kUT + tid; i < kLowBins; i += kSplitBlocks * kUT) low[i] = 0u;
@@ -1270,8 +1272,6 @@ __global__ __launch_bounds__(kUT) void split_kernel(UpdateArgs a) {
       if (dense[i]) atomicAdd(&hg[i], dense[i]);
     return;
   }
-  Found f;
-  if (!find_fine<kUT>(a, g, wsum, &found, f)) return;  // uniform
   const unsigned floor = ctl[kFloor];
   uint2* ties = reinterpret_cast<uint2*>(a.ties + (size_t)g * a.list_cap);
   each_value<kUT>(a, g, true, blockIdx.x, gridDim.x, [&](unsigned u, unsigned flat) {
@@ -1473,8 +1473,7 @@ __device__ __forceinline__ void select_dense(const UpdateArgs& a, int g, int x, 
 // Grid (G, kSelectBlocks) x 1024.
 __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
   const int g = blockIdx.x, tid = threadIdx.x;
-  const bool listed = list_ok(a, g);  // uniform
-  if (listed && blockIdx.y) return;
+  if (blockIdx.y && list_ok(a, g)) return;  // uniform
   __shared__ SelectLds L;
   unsigned* ctl = a.ctl + (size_t)g * kCtl;
   const unsigned count = budget_of(a);
@@ -1482,10 +1481,10 @@ __global__ __launch_bounds__(kST) void select_kernel(UpdateArgs a) {
     for (int i = tid; i < kSampleBins; i += kST) a.sample[(size_t)g * kSampleBins + i] = 0u;  // for the next call
   if (tid == 0) L.nbin = 0u;
   Found f;
-  const bool split = listed && find_fine<kST>(a, g, L.wsum, &L.found, f);
+  const bool split = blockIdx.y == 0 && find_fine<kST>(a, g, L.wsum, &L.found, f);  // uniform
   if (blockIdx.y == 0)
     for (int i = tid; i < kBins; i += kST) hist_of(a, g, 0)[i] = 0u;  // for the next call
-  if (!listed) {
+  if (!split && !list_ok(a, g)) {
     select_dense(a, g, blockIdx.y, L);
     return;
   }
