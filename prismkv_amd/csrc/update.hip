@@ -27,8 +27,9 @@
 // `interval` tokens, its cost is amortised):
 //   sample   W as pairs of f16 in the encode's operand order, and a histogram
 //            (13 bits) of the positive activations of a few hundred tokens;
-//   encode   the GEMM on the f16 matrix cores, 512 buckets x 16 tokens per
-//            workgroup and step, a = relu(...): the values at or above a floor
+//   encode   the GEMM on the f16 matrix cores (in fp32 for rows and buckets that
+//            this would not serve), 512 buckets x 16 tokens per workgroup and
+//            step, a = relu(...): the values at or above a floor
 //            read off the sample (about twice the budget of them) go to the
 //            group's candidate list as (flat index, value), and, where the
 //            caller reads them, all of them to [G][N][F];
@@ -38,7 +39,7 @@
 //            a short list;
 //   select   one workgroup per group finds tau in that list and, when ties at
 //            tau overflow the budget, the flat index of the last one taken, and
-//            sets the rest of the bits;
+//            sets the rest of the bits (many, where they read the activations);
 //   moments  per 32-bucket tile: new members from the bitmap, two-pass
 //            moments of their keys, merge, counts += new.
 // The sample decides only how long the list is.  Where it misjudged (fewer
@@ -302,7 +303,8 @@ struct RowsRaw {
   }
 };
 
-// d / s in fp32, rounded to nearest, for many d: r = 1 / s (rounded), one
+// d / s in fp32, rounded to nearest, for many d (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990): r = 1 / s (rounded), one
 // product, its remainder and one correction, which round as the division does
 // while nothing leaves the normal range (8e8 random pairs, none differs); an
 // infinite or NaN d gives NaN, a row that the split does not serve.
@@ -349,7 +351,8 @@ __device__ __forceinline__ bool split_rows(const RowsRaw<KT, kTB>& raw, half8 (&
   return __any(bad);
 }
 
-// acc[tb][j] = the products of the wave's 32 tokens with a split W tile in LDS:
+// The sample's products.  acc[tb][j] = those of the wave's 16 kTB tokens (16 or 32,
+// kTB of them a lane's column) with a split W tile in LDS:
 // v_mfma_f32_16x16x32_f16, lane (i, q) feeding A[i][8 q + t] and B[8 q + t][i],
 // t = 0..7, and holding D[4 q + r][i].  A is W (bucket rows), B is x (token
 // columns), so lane (i, q) ends with buckets 16 j + 4 q + r of token i.
@@ -470,7 +473,7 @@ __device__ __forceinline__ void fp32_products(const UpdateArgs& a, int g, int to
   }
 }
 
-// The values of one bucket tile for the wave's 16 kTB tokens, after the products
+// The sample's values of one bucket tile for the wave's 16 kTB tokens, after the products
 // (made again in fp32 where a row or bucket is not split): four(tb, j, v) gets
 // lane (i, q)'s pre-relu sums of buckets 16 j + 4 q .. + 3.  `tok` is the lane's
 // kTB tokens; sg the tile's biases, then its inverse bucket scales.
@@ -643,8 +646,8 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
 // The other way round (x in registers, W tiles streamed through LDS, a barrier
 // per tile) every wave read 32 KB of LDS per 96 MFMAs; here it is 16 KB, a
 // barrier per 192, and no load of the loop but the next stage's rows.  1024 /
-// 4096 keys with the activations stored: 38 / 121 us then, 35 / 109 now; 65536
-// without: 1.33 ms, now 1.17 (2.07 GHz under this load, 1.03 PFLOP/s; the
+// 4096 keys with the activations stored: 38 / 121 us then, 37 / 113 now; 65536
+// without: 1.33 ms, now 1.18 (2.07 GHz under this load, 1.03 PFLOP/s; the
 // products alone took 0.90 ms, and a large f16 library product runs at 1.2).
 // Neither a higher priority for some of the waves nor the epilogue's values
 // placed one by one between the next step's products changed that.
@@ -2122,7 +2125,7 @@ __global__ __launch_bounds__(NT, 4) void build_moments_kernel(UpdateArgs a) {
 // workgroup lists.  A workgroup each, as any number of them may be (a dense bitmap,
 // a budget of many per key): 64 workgroups for all took 22.9 ms for one group of
 // 32768 keys with half of them in every bucket, 1000 took 2.1, now 1.9 (one launch
-// of 256 threads: 1.7); where there is none, 8 groups' launch takes 10 us.
+// of 256 threads: 1.7); where there is none, 8 groups' launch takes 7.5 us.
 template <typename KT>
 __global__ __launch_bounds__(kUT, 4) void build_moments_rest_kernel(UpdateArgs a) {
   __shared__ BuildMomentsLds<kUT> L;

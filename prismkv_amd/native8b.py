@@ -400,9 +400,10 @@ class Native8B:
     @router.setter
     def router(self, router):
         """"moments" (the native path, one launch per layer) or "q_activation"
-        (src/prismkv/core.py:131-139: route + union of up to 64 buckets, then
-        attention; needs set_query_encoders).  features / valid are [8,16]
-        for moments and [8,64] for q_activation."""
+        (src/prismkv/core.py:131-139; needs set_query_encoders): up to 64
+        buckets, by the queries' activations; two launches per layer, or, with a
+        unique cap or a history past FUSED_MAX_HISTORY, route, then attention.
+        features / valid are [8,16] for moments and [8,64] for q_activation."""
         if router not in ("moments", "q_activation"):
             raise ValueError("unsupported router/bucket count")
         if router == "q_activation" and getattr(self, "W_query", None) is None:
@@ -467,7 +468,9 @@ class Native8B:
         bit-identical, out within rounding of the separate attention kernel.
         With a unique cap the same launch runs the budgeted walk between the
         selection and the union (features / valid / raw then hold the kept
-        buckets, compacted in rank order, as route() leaves them).
+        buckets, compacted in rank order, as route() leaves them).  The
+        q_activation router takes two launches, with a cap or a history past
+        FUSED_MAX_HISTORY route() and attention().
 
         `tail` (no reference counterpart): an int32 CUDA tensor of one element
         holding the tail length T, read by the kernel at launch instead of

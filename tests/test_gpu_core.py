@@ -47,8 +47,8 @@ def test_positive_global_topk(kind):
     count = 8 * N
     if kind == "crowded":
         # 2048 values in [10, 11) (one first-digit bin, tau's) at flat indices
-        # [0, 1024) and [262144, 263168): the positions one refine workgroup
-        # reads, so its 1024-entry candidate buffer overflows into the list
+        # [0, 1024) and [262144, 263168): the positions that one workgroup of a
+        # pass over the matrix reads at once
         a = a.abs() * 0.01
         flat = a.view(-1)
         big = 10.0 + torch.rand(2048, generator=gen, device="cuda")
@@ -56,9 +56,8 @@ def test_positive_global_topk(kind):
         flat[262144:263168] = big[1024:]
         count = 1500
     elif kind == "wide_bin":
-        # 600000 positive values in tau's first-digit bin: more candidates than
-        # the compact list holds (2^19 entries less the chunk tails' 2^18 at
-        # this block size), so the later passes scan every value
+        # 600000 positive values in tau's first-digit bin, all of which the later
+        # levels count again
         a = 1.0 + torch.rand(N, F, generator=gen, device="cuda") * 0.0625
         a.view(-1)[600000:] = -1.0
         count = 5000

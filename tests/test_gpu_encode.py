@@ -1,8 +1,9 @@
 """The encode of the index update and build (relu((k - center) / scale W^T + b),
 src/prismkv/core.py:47-48,98) where its f16 split or its tiles can go wrong:
-blocks around a workgroup's 256 tokens and a wave's 32, rows and buckets of
-extreme magnitudes (scaled per row and per bucket), and rows and buckets that
-are not split (all zero, beyond 2^60, infinite or NaN)."""
+blocks around its 16-token steps, its 64-token stages and a workgroup's range of
+tokens, rows and buckets of extreme magnitudes (scaled per row and per bucket),
+and rows and buckets that are not split (beyond 2^60, infinite or NaN, or of few
+significant dims)."""
 import numpy as np
 import pytest
 import torch
