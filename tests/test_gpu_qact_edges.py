@@ -158,3 +158,24 @@ def test_captured_launches(H):
         for g in range(8):
             assert torch.equal(op.ids[g, :op.count[g]], ids[g]), (i, g)
     assert op.decode_errors() == 0
+
+
+@pytest.mark.parametrize("H,T", [(700, 0), (700, 3), (70000, 0), (70000, 5)])
+def test_no_bucket_of_positive_weight(H, T):
+    # two groups whose activations are all 0, one of NaN queries: the tail alone, or nothing
+    op, q, k, v, W, b = operator(H, T, H + T)
+    W[2:4] = 0
+    b[2:4] = -1.0
+    q[5] = float("nan")
+    op.set_query_encoders(W, b, torch.ones(8))
+    op.router = "q_activation"
+    op.route(q)
+    want_out = op.attention(q, k, v).clone()
+    count, valid, raw = op.count.clone(), op.valid.clone(), op.raw.clone()
+    got = op(q, k, v)
+    assert count[[2, 3, 5]].tolist() == [0, 0, 0] and torch.equal(op.count, count)
+    assert torch.equal(op.valid, valid) and torch.equal(op.raw, raw)
+    assert torch.equal(got.isnan(), want_out.isnan())
+    a, e = got.float().nan_to_num(), want_out.float().nan_to_num()
+    assert float((a - e).norm()) <= 4e-3 * float(e.norm())
+    assert op.decode_errors() == 0
