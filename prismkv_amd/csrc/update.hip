@@ -242,8 +242,32 @@ __device__ __forceinline__ float2 row_scale(float m) {
   return make_float2(__uint_as_float((unsigned)(127 + k) << 23), __uint_as_float((unsigned)(127 - k) << 23));
 }
 
+// The larger, or the sum, of lane l's and lane l ^ M's value, M = 8, 16 or 32, by vector
+// instructions alone: after a swap the two stand in some order in r[0] and r[1].
+template <int M>
+__device__ __forceinline__ float max_xor(float v) {
+  if constexpr (M == 8) {
+    return fmaxf(v, xor8(v));
+  } else {
+    const unsigned u = __float_as_uint(v);
+    const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false)
+                           : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+}
+template <int M>
+__device__ __forceinline__ int add_xor(int v) {
+  if constexpr (M == 8) {
+    return v + __float_as_int(xor8(__int_as_float(v)));
+  } else {
+    const auto r = M == 16 ? __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false)
+                           : __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return (int)(r[0] + r[1]);
+  }
+}
+
 // Whether at least kMinDims of a row's 128 magnitudes are significant.  The
-// calling lane holds N of them, the row's lanes are M apart (M, 2 M, .. < 64); m
+// calling lane holds N of them, the row's lanes are M = 8 or 16 apart; m
 // is the row's largest.  Every row of the wave answers at once: nearly always by
 // the lanes' minima alone (a N(0, 1) row has a smaller value once in 250).
 template <int M, int N>
@@ -256,9 +280,8 @@ __device__ __forceinline__ bool enough_dims(const float (&x)[N], float m) {
   int n = 0;
 #pragma unroll
   for (int i = 0; i < N; ++i) n += fabsf(x[i]) >= least ? 1 : 0;
-#pragma unroll
-  for (int o = M; o < 64; o *= 2) n += __shfl_xor(n, o);
-  return n >= kMinDims;
+  if constexpr (M == 8) n = add_xor<8>(n);
+  return add_xor<32>(add_xor<16>(n)) >= kMinDims;
 }
 
 template <typename Fn>
@@ -340,8 +363,7 @@ __device__ __forceinline__ bool split_rows(const RowsRaw<KT, kTB>& raw, half8 (&
         m = fmaxf(m, fabsf(d));  // NaN is passed over: its sums are NaN either way
         x[kb][t] = divide_by(d, s, rs);
       }
-    m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));
+    m = max_xor<32>(max_xor<16>(m));
     const float2 s2 = row_scale(fabsf(divide_by(m, s, rs)));  // the largest |x|; NaN for an infinite m
     xinv[tb] = s2.y;
     bad |= s2.y == 0.f;
@@ -563,8 +585,7 @@ __global__ __launch_bounds__(kET) void sample_kernel(UpdateArgs a, int S) {
 #pragma unroll
       for (int t = 0; t < 8; ++t) m = fmaxf(m, fabsf(x[kb][t]));
     }
-    m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));
+    m = max_xor<32>(max_xor<16>(m));
     const float2 sc = row_scale(m);
     // (the sample itself, which only places the floor, uses any split there is)
     const bool enough = enough_dims<16>(reinterpret_cast<const float (&)[kKB * 8]>(x), m);
@@ -687,18 +708,19 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   const int ft = part * kEW + w, f0 = ft * kFT + 4 * lq;
   const bool live = ft < kFTiles;  // uniform per wave: the last part's last wave only splits rows
   // rows of a stage: thread (row 8 w + l % 8, dims 16 (l / 8) .. + 15)
-  const int sr = 8 * w + (lane & 7), sp = lane >> 3;
-  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks + 16 * sp;
+  const KT* kg = static_cast<const KT*>(a.k) + (size_t)g * a.ks;
   const float scale = a.scale[g], rscale = 1.0f / scale;
   // (the scale's own range bounds what divide_by may meet)
   const bool scaled = fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p60f;
   typename KeyLoad<KT>::Raw8 raw[2];
   auto load_rows = [&](int t) {
-    const KT* p = kg + (size_t)(a.H + min(t + sr, a.N - 1)) * kD;
+    const int l = lane_again(), sr = 8 * w + (l & 7), sp = l >> 3;
+    const KT* p = kg + (size_t)(a.H + min(t + sr, a.N - 1)) * kD + 16 * sp;
     raw[0] = KeyLoad<KT>::raw8(p);
     raw[1] = KeyLoad<KT>::raw8(p + 8);
   };
   auto split_rows = [&](int buf) {
+    const int l = lane_again(), sr = 8 * w + (l & 7), sp = l >> 3;
     float x[2][8], m = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -710,9 +732,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
         m = fmaxf(m, fabsf(x[h][t]));  // NaN is passed over: its sums are NaN either way
       }
     }
-    m = fmaxf(m, __shfl_xor(m, 8));
-    m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));
+    m = max_xor<32>(max_xor<16>(max_xor<8>(m)));
     const float2 s2 = row_scale(fabsf(divide_by(m, scale, rscale)));  // the largest |x|; NaN for an infinite m
     const bool enough = enough_dims<8>(reinterpret_cast<const float (&)[16]>(x), m);
     // (d / s) times the row's power of two: the quotient and its remainder scale exactly
@@ -726,8 +746,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
       out[64 + 16 * h] = lo;
     }
     // (a quotient's remainder stays in the normal range)
-    const int l = lane_again();
-    if (l < 8) xinv[buf][8 * w + l] = scaled && enough && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
+    if (sp == 0) xinv[buf][sr] = scaled && enough && fabsf(ss) >= 0x1p-100f ? s2.y : 0.f;
   };
   load_rows(t0);
   if (tid < kD) center[tid] = a.center[(size_t)g * kD + tid];
@@ -806,7 +825,7 @@ __global__ __launch_bounds__(kET) void encode_kernel(UpdateArgs a) {
   const unsigned long long odd = __ballot(xinv[0][lane] == 0.f);
   const int odd_steps = (int)((odd & 0xffffull) != 0) + (int)((odd >> 16 & 0xffffull) != 0) +
                         (int)((odd >> 32 & 0xffffull) != 0) + (int)(odd >> 48 != 0);
-  const bool whole = bad_w || odd_steps >= 2;  // uniform
+  const bool whole = __builtin_amdgcn_readfirstlane(bad_w || odd_steps >= 2 ? 1 : 0) != 0;  // uniform, as a scalar
   if (__builtin_expect(whole, 0)) {
     const __amdgpu_buffer_rsrc_t wr = raw_buffer(a.W + (size_t)g * kF * kD, kF * kD * (int)sizeof(float));  // 0 past F
     const unsigned o = ((unsigned)(ft * kFT + li) * kD + 4 * lq) * (unsigned)sizeof(float);
